@@ -28,7 +28,10 @@
 //                               pieces through a register ring into LDS, one
 //                               summing wave keeps a sequential fp32
 //                               accumulator per channel
-//     accum_rows_kernel<T>      the same for rows that are not 16-byte pieces
+//     accum_group_kernel<T>     small inputs, wide or unaligned rows and the
+//                               depth-weighted rows: groups of lanes walk
+//                               their own cells, no LDS staging, no barriers
+//     accum_rows_kernel<T>      rows of fewer than 16 bytes
 //     rows_to_bev_kernel<T>     cell-major rows -> channel-first tile via LDS
 //                               transpose; empty cells written as zero
 //   backward
@@ -44,7 +47,7 @@
 //                               channel-first camera features)
 //     gather_planar_kernel      backward straight into a (BN, C, S) gradient
 //   depth-weighted pooling (fused depth x context)
-//     accum_pipe_kernel<..,true> forward sums of depth[p] * ctx[pix(p)]
+//     accum_group_kernel        forward sums of depth[p] * ctx[pix(p)]
 //     depth_grad_kernel         grad_depth (dot products) and grad_context
 //                               (depth-weighted sums along each ray)
 //
@@ -1542,19 +1545,20 @@ __device__ __forceinline__ int64_t snap_to_cell(int64_t i, int64_t n,
   return cend[r];
 }
 
-// Block b owns the sorted positions [snap(b*P), snap((b+1)*P)): whole cells
-// only, so every cell's sum is one sequential chain.  Rows (feats[point]) of
-// R sorted points at a time are gathered into LDS by all threads; thread c
-// then adds column c of the R rows in order into its fp32 accumulator and
-// stores it to acc[cell*C + c] when the cell ends.
+// Rows of fewer than 16 bytes.  Block b owns the sorted positions
+// [snap(b*P), snap((b+1)*P)): whole cells only, so every cell's sum is one
+// sequential chain.  Rows (feats[point]) of R sorted points at a time are
+// gathered into LDS by all threads; thread c then adds column c of the R rows
+// in order into its fp32 accumulator and stores it to acc[cell*C + c] when
+// the cell ends.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void accum_rows_kernel(
-    const typename T::raw *__restrict__ x, int64_t ld, int C, int CB, int R,
+    const typename T::raw *__restrict__ x, int64_t ld, int C, int R,
     const uint64_t *__restrict__ keys, const int32_t *__restrict__ meta,
     const int32_t *__restrict__ cend, float *__restrict__ acc, int64_t P) {
   extern __shared__ float smem[];
-  float *buf = smem;                         // R * CB floats
-  int *rk = reinterpret_cast<int *>(smem + R * CB);  // R + 1 ints
+  float *buf = smem;                                // R * C floats
+  int *rk = reinterpret_cast<int *>(smem + R * C);  // R + 1 ints
   const int tid = threadIdx.x;
   const int64_t n = meta[BEVPOOL_META_N_KEPT];
   const int64_t r0 = int64_t(blockIdx.x) * P;
@@ -1562,29 +1566,25 @@ __global__ __launch_bounds__(kThreads) void accum_rows_kernel(
   const int64_t s = snap_to_cell(r0, n, keys, cend);
   const int64_t e = snap_to_cell(r0 + P < n ? r0 + P : n, n, keys, cend);
   if (s >= e) return;
-  using raw = typename T::raw;
-  for (int c0 = 0; c0 < C; c0 += CB) {
-    const int cb = C - c0 < CB ? C - c0 : CB;
-    float a = 0.0f;
-    for (int64_t base = s; base < e; base += R) {
-      const int rows = int(e - base < R ? e - base : R);
-      __syncthreads();
-      for (int j = tid; j <= rows; j += kThreads)
-        rk[j] = (base + j < e) ? key_rank(keys[base + j]) : -1;
-      for (int slot = tid; slot < rows * cb; slot += kThreads) {
-        const int j = slot / cb, c = slot - j * cb;
-        const int64_t idx = key_index(keys[base + j]);
-        buf[slot] = T::load(reinterpret_cast<const raw *>(x) + idx * ld + c0 + c);
-      }
-      __syncthreads();
-      if (tid < cb) {
-        for (int j = 0; j < rows; ++j) {
-          a += buf[j * cb + tid];
-          const int r = rk[j];
-          if (rk[j + 1] != r) {
-            acc[int64_t(r) * C + c0 + tid] = a;
-            a = 0.0f;
-          }
+  float a = 0.0f;
+  for (int64_t base = s; base < e; base += R) {
+    const int rows = int(e - base < R ? e - base : R);
+    __syncthreads();
+    for (int j = tid; j <= rows; j += kThreads)
+      rk[j] = (base + j < e) ? key_rank(keys[base + j]) : -1;
+    for (int slot = tid; slot < rows * C; slot += kThreads) {
+      const int j = slot / C, c = slot - j * C;
+      const int64_t idx = key_index(keys[base + j]);
+      buf[slot] = T::load(x + idx * ld + c);
+    }
+    __syncthreads();
+    if (tid < C) {
+      for (int j = 0; j < rows; ++j) {
+        a += buf[j * C + tid];
+        const int r = rk[j];
+        if (rk[j + 1] != r) {
+          acc[int64_t(r) * C + tid] = a;
+          a = 0.0f;
         }
       }
     }
@@ -1640,7 +1640,7 @@ static_assert(kStageRows == 32, "only 32-row accumulation stages are supported")
 
 // native 16-byte vector (register-promotable, unlike the HIP uint4 wrapper)
 
-// Where the accumulation's rows come from and how they are loaded:
+// How the accumulations load their rows:
 //   kRowsPlain   feature rows, ordinary loads;
 //   kRowsStream  feature rows, non-temporal loads: the rows are read once,
 //                and keeping them out of the caches keeps the index (ranks,
@@ -1652,13 +1652,14 @@ static_assert(kStageRows == 32, "only 32-row accumulation stages are supported")
 //                faster, so inputs of more than kStreamRowBytes of rows keep
 //                ordinary loads.
 //   kRowsDepth   depth-weighted context rows (DepthRows), ordinary loads:
-//                a context row is read for every depth bin.
+//                a context row is read for every depth bin
+//                (accum_group_kernel only).
 constexpr int kRowsPlain = 0, kRowsDepth = 1, kRowsStream = 2;
 constexpr int64_t kStreamRowBytes = int64_t(1) << 30;
 
 struct PipeRange {
   int64_t s, e;  // sorted positions [s, e)
-  int rowq;      // 16-byte slots per row of this channel block
+  int rowq;      // 16-byte pieces per row
   __device__ __forceinline__ int rows(int k) const {
     const int64_t b = s + int64_t(k) * kStageRows;
     return b >= e ? 0 : int(e - b < kStageRows ? e - b : kStageRows);
@@ -1671,44 +1672,22 @@ struct LoaderRing {
   u32x4 d[kDepth][kSlots];       // gathered 16-byte pieces of a stage
   uint32_t idx[kDepth][kSlots];  // point indices of a later stage
   int rk[kDepth];                // rank of row (lt % kStageRows) of a stage
-  uint32_t dpi[kDepth];          // depth-weighted rows: point index of that row
-  float dp[kDepth];              //   and its depth weight
   int srow[kSlots];              // row of slot i within a stage (unclamped)
   int sq[kSlots];                // 16-byte column of slot i
 };
 
-// Rows of the depth-weighted forward (fused depth x context pooling): the row
-// of point p = (bn*D + d)*HW + hw is context row pix = bn*HW + hw, weighted by
-// depth[p] (the reference materialises depth[p] * context[pix, c],
-// models/vtransforms/depth_lss.py:91-94).
-struct DepthRows {
-  const float *depth;  // (BN, D, HW) contiguous: depth[p]
-  FastDiv hw, nd;      // HW and D
-  // p = (bn*D + d)*HW + hw -> bn*HW + hw, with e = p / HW = bn*D + d
-  __device__ __forceinline__ uint32_t pix(uint32_t p) const {
-    const uint32_t e = hw.div(p);
-    return nd.div(e) * hw.d + (p - e * hw.d);
-  }
-};
-
 // Point indices of stage k into ring slot j.  Slots past the stage's rows
 // repeat its last row; a stage past the range end reads the range's first row.
-template <int kSlots, int j, int kRows>
-__device__ __forceinline__ void ring_index(LoaderRing<kSlots> &R, int lt,
+template <int kSlots, int j>
+__device__ __forceinline__ void ring_index(LoaderRing<kSlots> &R,
                                            const uint32_t *__restrict__ kw, const PipeRange &pr,
                                            int k) {
-  constexpr bool kMul = kRows == kRowsDepth;
   const int rows = pr.rows(k);
   const int64_t base = pr.s + int64_t(k) * kStageRows;
 #pragma unroll
   for (int i = 0; i < kSlots; ++i) {
     const int r = R.srow[i] < rows - 1 ? R.srow[i] : rows - 1;
     R.idx[j][i] = kw[2 * (rows > 0 ? base + r : pr.s)];  // low word: point index
-  }
-  if constexpr (kMul) {
-    int64_t p = base + (lt & (kStageRows - 1));
-    p = base >= pr.e ? pr.s : (p < pr.e ? p : pr.e - 1);
-    R.dpi[j] = kw[2 * p];
   }
 }
 
@@ -1718,16 +1697,13 @@ template <int kSlots, int j, int kRows>
 __device__ __forceinline__ void ring_rows(LoaderRing<kSlots> &R, int lt,
                                           const uint32_t *__restrict__ kw,
                                           const char *__restrict__ xb, int64_t ld_bytes,
-                                          int col_bytes, const PipeRange &pr, int k,
-                                          const DepthRows &dr) {
-  constexpr bool kMul = kRows == kRowsDepth;
+                                          const PipeRange &pr, int k) {
   const bool live = pr.rows(k) > 0;
 #pragma unroll
   for (int i = 0; i < kSlots; ++i) {
     const int q = live ? R.sq[i] : 0;
-    const uint32_t row = kMul ? dr.pix(R.idx[j][i]) : R.idx[j][i];
     const u32x4 *src =
-        reinterpret_cast<const u32x4 *>(xb + int64_t(row) * ld_bytes + col_bytes + q * 16);
+        reinterpret_cast<const u32x4 *>(xb + int64_t(R.idx[j][i]) * ld_bytes + q * 16);
     if constexpr (kRows == kRowsStream)
       R.d[j][i] = __builtin_nontemporal_load(src);
     else
@@ -1737,47 +1713,18 @@ __device__ __forceinline__ void ring_rows(LoaderRing<kSlots> &R, int lt,
   int64_t p = b + (lt & (kStageRows - 1));
   p = b >= pr.e ? pr.s : (p < pr.e ? p : pr.e - 1);
   R.rk[j] = kw[2 * p + 1];  // high word: rank
-  if constexpr (kMul) R.dp[j] = dr.depth[R.dpi[j]];
 }
 
 // Ring slot j (stage k) into an LDS buffer.
-template <int kSlots, int j, int kRows>
+template <int kSlots, int j>
 __device__ __forceinline__ void ring_store(const LoaderRing<kSlots> &R, int lt,
                                            const PipeRange &pr, int k, u32x4 *__restrict__ lbuf,
                                            int *__restrict__ lrk) {
-  constexpr bool kMul = kRows == kRowsDepth;
-  const int rows = pr.rows(k);
-  const int n = rows * pr.rowq;
-  if constexpr (kMul) {
-    // slot i of this thread holds a piece of row srow[i]; lane r of every
-    // loader wave holds the depth weight of row r (ring_index / ring_rows):
-    // all lanes shuffle it in before any store is masked off, then scale the
-    // piece (one fp32 product per element, as the reference's product)
-    u32x4 v[kSlots];
+  const int n = pr.rows(k) * pr.rowq;
 #pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      const int r = R.srow[i] < kStageRows - 1 ? R.srow[i] : kStageRows - 1;
-      const float w = __shfl(R.dp[j], r, 64);
-      // __uint_as_float takes the element by value: hipcc 7.2's
-      // __builtin_bit_cast of a vector element (v.y) reads element 0
-      const float x0 = __uint_as_float(R.d[j][i].x) * w;
-      const float x1 = __uint_as_float(R.d[j][i].y) * w;
-      const float x2 = __uint_as_float(R.d[j][i].z) * w;
-      const float x3 = __uint_as_float(R.d[j][i].w) * w;
-      v[i] = u32x4{__float_as_uint(x0), __float_as_uint(x1), __float_as_uint(x2),
-                   __float_as_uint(x3)};
-    }
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      const int slot = lt + kLoaders * i;
-      if (slot < n) lbuf[slot] = v[i];
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      const int slot = lt + kLoaders * i;
-      if (slot < n) lbuf[slot] = R.d[j][i];
-    }
+  for (int i = 0; i < kSlots; ++i) {
+    const int slot = lt + kLoaders * i;
+    if (slot < n) lbuf[slot] = R.d[j][i];
   }
   if (lt < kStageRows) lrk[lt] = R.rk[j];
 }
@@ -1787,17 +1734,16 @@ template <int kSlots, int r, int kRows>
 __device__ __forceinline__ void loader_step(LoaderRing<kSlots> &R, int lt,
                                             const uint32_t *__restrict__ kw,
                                             const char *__restrict__ xb, int64_t ld_bytes,
-                                            int col_bytes, const PipeRange &pr, int k, int nst,
+                                            const PipeRange &pr, int k, int nst,
                                             u32x4 *__restrict__ buf0, u32x4 *__restrict__ buf1,
-                                            int *__restrict__ rk0s, int *__restrict__ rk1s,
-                                            const DepthRows &dr) {
-  ring_rows<kSlots, r, kRows>(R, lt, kw, xb, ld_bytes, col_bytes, pr, k + kDepth, dr);
-  ring_index<kSlots, r, kRows>(R, lt, kw, pr, k + 2 * kDepth);
+                                            int *__restrict__ rk0s, int *__restrict__ rk1s) {
+  ring_rows<kSlots, r, kRows>(R, lt, kw, xb, ld_bytes, pr, k + kDepth);
+  ring_index<kSlots, r>(R, kw, pr, k + 2 * kDepth);
   if (k + 1 < nst) {
     if ((k + 1) & 1)
-      ring_store<kSlots, (r + 1) % kDepth, kRows>(R, lt, pr, k + 1, buf1, rk1s);
+      ring_store<kSlots, (r + 1) % kDepth>(R, lt, pr, k + 1, buf1, rk1s);
     else
-      ring_store<kSlots, (r + 1) % kDepth, kRows>(R, lt, pr, k + 1, buf0, rk0s);
+      ring_store<kSlots, (r + 1) % kDepth>(R, lt, pr, k + 1, buf0, rk0s);
   }
   __syncthreads();
 }
@@ -1932,26 +1878,24 @@ struct RowSum {
   }
 };
 
-// kMul: depth-weighted rows (DepthRows): xb holds the context rows and row
-// p's values are depth[p] * ctx[pix(p)].
 template <typename T, int kSlots, int kCPL, int kRows>
 __global__ __launch_bounds__(kPipeThreads) void accum_pipe_kernel(
-    const char *__restrict__ xb, int64_t ld_bytes, int C, int CB,
-    const uint64_t *__restrict__ keys, const int32_t *__restrict__ meta,
-    const int32_t *__restrict__ cend, float *__restrict__ acc, int64_t P, DepthRows dr) {
+    const char *__restrict__ xb, int64_t ld_bytes, int C, const uint64_t *__restrict__ keys,
+    const int32_t *__restrict__ meta, const int32_t *__restrict__ cend, float *__restrict__ acc,
+    int64_t P) {
   using raw = typename T::raw;
   extern __shared__ u32x4 smem4[];
-  const int rowq_max = CB * int(sizeof(raw)) / 16;
+  PipeRange pr;
+  pr.rowq = C * int(sizeof(raw)) / 16;
   u32x4 *buf0 = smem4;
-  u32x4 *buf1 = smem4 + kStageRows * rowq_max;
-  int *rk0s = reinterpret_cast<int *>(smem4 + 2 * kStageRows * rowq_max);
+  u32x4 *buf1 = smem4 + kStageRows * pr.rowq;
+  int *rk0s = reinterpret_cast<int *>(smem4 + 2 * kStageRows * pr.rowq);
   int *rk1s = rk0s + kStageRows;
   const uint32_t *kw = reinterpret_cast<const uint32_t *>(keys);
 
   const int64_t n = meta[BEVPOOL_META_N_KEPT];
   const int64_t r0 = int64_t(blockIdx.x) * P;
   if (r0 >= n) return;
-  PipeRange pr;
   pr.s = snap_to_cell(r0, n, keys, cend);
   pr.e = snap_to_cell(r0 + P < n ? r0 + P : n, n, keys, cend);
   if (pr.s >= pr.e) return;
@@ -1960,81 +1904,434 @@ __global__ __launch_bounds__(kPipeThreads) void accum_pipe_kernel(
   const bool summer = wave < kSummers;
   const int lt = int(threadIdx.x) - 64 * kSummers;  // loader thread index (loader waves only)
 
-  for (int c0 = 0; c0 < C; c0 += CB) {
-    const int cb = C - c0 < CB ? C - c0 : CB;
-    pr.rowq = cb * int(sizeof(raw)) / 16;
-    if (summer) {
-      // summing wave `wave` owns channels [wch, wch + nch) of the block
-      // (an even count with 16-bit input, whose lanes take channel pairs)
-      constexpr bool kPair = RowSum<T, kCPL>::kPair;
-      int cps = (cb + kSummers - 1) / kSummers;
-      if (kPair) cps += cps & 1;
-      const int wch = wave * cps;
-      const int nch = cb - wch < cps ? (cb - wch > 0 ? cb - wch : 0) : cps;
-      int col[kCPL];
+  if (summer) {
+    // summing wave `wave` owns channels [wch, wch + nch)
+    // (an even count with 16-bit input, whose lanes take channel pairs)
+    constexpr bool kPair = RowSum<T, kCPL>::kPair;
+    int cps = (C + kSummers - 1) / kSummers;
+    if (kPair) cps += cps & 1;
+    const int wch = wave * cps;
+    const int nch = C - wch < cps ? (C - wch > 0 ? C - wch : 0) : cps;
+    int col[kCPL];
 #pragma unroll
-      for (int i = 0; i < kCPL; ++i) {
-        const int c = lane_id() + 64 * i;
-        if (kPair) {  // pair index within the stage row
-          const int np = nch >> 1;
-          const int pc = (wch >> 1) + (c < np ? c : (np > 0 ? np - 1 : 0));
-          col[i] = pc < (cb >> 1) ? pc : (cb >> 1) - 1;
-        } else {
-          const int cc = wch + (c < nch ? c : (nch > 0 ? nch - 1 : 0));
-          col[i] = cc < cb ? cc : cb - 1;  // idle lanes read a valid column
-        }
+    for (int i = 0; i < kCPL; ++i) {
+      const int c = lane_id() + 64 * i;
+      if (kPair) {  // pair index within the stage row
+        const int np = nch >> 1;
+        const int pc = (wch >> 1) + (c < np ? c : (np > 0 ? np - 1 : 0));
+        col[i] = pc < (C >> 1) ? pc : (C >> 1) - 1;
+      } else {
+        const int cc = wch + (c < nch ? c : (nch > 0 ? nch - 1 : 0));
+        col[i] = cc < C ? cc : C - 1;  // idle lanes read a valid column
       }
-      using TO = typename RowSum<T, kCPL>::TO;  // 16-bit rows for 16-bit input
-      TO *out = reinterpret_cast<TO *>(acc) + c0 + wch;
-      RowSum<T, kCPL> st;
-      __syncthreads();  // stage 0 is in buffer 0
-      for (int k = 0; k < nst; k += kDepth) {  // barriers match the loaders'
+    }
+    using TO = typename RowSum<T, kCPL>::TO;  // 16-bit rows for 16-bit input
+    TO *out = reinterpret_cast<TO *>(acc) + wch;
+    RowSum<T, kCPL> st;
+    __syncthreads();  // stage 0 is in buffer 0
+    for (int k = 0; k < nst; k += kDepth) {  // barriers match the loaders'
 #pragma unroll
-        for (int r = 0; r < kDepth; ++r) {
-          const int kk = k + r;
-          st.add_stage(reinterpret_cast<const raw *>((kk & 1) ? buf1 : buf0),
-                       (kk & 1) ? rk1s : rk0s, pr.rows(kk), cb, col, nch, out, C);
-          __syncthreads();
-        }
+      for (int r = 0; r < kDepth; ++r) {
+        const int kk = k + r;
+        st.add_stage(reinterpret_cast<const raw *>((kk & 1) ? buf1 : buf0),
+                     (kk & 1) ? rk1s : rk0s, pr.rows(kk), C, col, nch, out, C);
+        __syncthreads();
       }
-      st.flush(nch, out, C);
-    } else {
-      const int col_bytes = c0 * int(sizeof(raw));
-      LoaderRing<kSlots> R;
+    }
+    st.flush(nch, out, C);
+  } else {
+    LoaderRing<kSlots> R;
 #pragma unroll
-      for (int i = 0; i < kSlots; ++i) {
-        const int slot = lt + kLoaders * i;
-        R.srow[i] = slot / pr.rowq;
-        R.sq[i] = slot - R.srow[i] * pr.rowq;
-      }
-      // prologue: indices of stages 0..D-1, rows of 0..D-1 each followed by the
-      // indices of stage j+D; then stage 0 into LDS
+    for (int i = 0; i < kSlots; ++i) {
+      const int slot = lt + kLoaders * i;
+      R.srow[i] = slot / pr.rowq;
+      R.sq[i] = slot - R.srow[i] * pr.rowq;
+    }
+    // prologue: indices of stages 0..D-1, rows of 0..D-1 each followed by the
+    // indices of stage j+D; then stage 0 into LDS
 #define BEVPOOL_RING_PRO(J)                                                                    \
-  if constexpr ((J) < kDepth) ring_index<kSlots, (J), kRows>(R, lt, kw, pr, (J));
-      BEVPOOL_RING_PRO(0) BEVPOOL_RING_PRO(1) BEVPOOL_RING_PRO(2) BEVPOOL_RING_PRO(3)
-      BEVPOOL_RING_PRO(4) BEVPOOL_RING_PRO(5) BEVPOOL_RING_PRO(6) BEVPOOL_RING_PRO(7)
+  if constexpr ((J) < kDepth) ring_index<kSlots, (J)>(R, kw, pr, (J));
+    BEVPOOL_RING_PRO(0) BEVPOOL_RING_PRO(1) BEVPOOL_RING_PRO(2) BEVPOOL_RING_PRO(3)
+    BEVPOOL_RING_PRO(4) BEVPOOL_RING_PRO(5) BEVPOOL_RING_PRO(6) BEVPOOL_RING_PRO(7)
 #undef BEVPOOL_RING_PRO
 #define BEVPOOL_RING_PRO(J)                                                                    \
   if constexpr ((J) < kDepth) {                                                               \
-    ring_rows<kSlots, (J), kRows>(R, lt, kw, xb, ld_bytes, col_bytes, pr, (J), dr);            \
-    ring_index<kSlots, (J), kRows>(R, lt, kw, pr, (J) + kDepth);                               \
+    ring_rows<kSlots, (J), kRows>(R, lt, kw, xb, ld_bytes, pr, (J));                           \
+    ring_index<kSlots, (J)>(R, kw, pr, (J) + kDepth);                                          \
   }
-      BEVPOOL_RING_PRO(0) BEVPOOL_RING_PRO(1) BEVPOOL_RING_PRO(2) BEVPOOL_RING_PRO(3)
-      BEVPOOL_RING_PRO(4) BEVPOOL_RING_PRO(5) BEVPOOL_RING_PRO(6) BEVPOOL_RING_PRO(7)
+    BEVPOOL_RING_PRO(0) BEVPOOL_RING_PRO(1) BEVPOOL_RING_PRO(2) BEVPOOL_RING_PRO(3)
+    BEVPOOL_RING_PRO(4) BEVPOOL_RING_PRO(5) BEVPOOL_RING_PRO(6) BEVPOOL_RING_PRO(7)
 #undef BEVPOOL_RING_PRO
-      ring_store<kSlots, 0, kRows>(R, lt, pr, 0, buf0, rk0s);
-      __syncthreads();
-      for (int k = 0; k < nst; k += kDepth) {
+    ring_store<kSlots, 0>(R, lt, pr, 0, buf0, rk0s);
+    __syncthreads();
+    for (int k = 0; k < nst; k += kDepth) {
 #define BEVPOOL_RING_STEP(J)                                                                   \
   if constexpr ((J) < kDepth)                                                                 \
-    loader_step<kSlots, (J), kRows>(R, lt, kw, xb, ld_bytes, col_bytes, pr, k + (J), nst, buf0, \
-                                   buf1, rk0s, rk1s, dr);
-        BEVPOOL_RING_STEP(0) BEVPOOL_RING_STEP(1) BEVPOOL_RING_STEP(2) BEVPOOL_RING_STEP(3)
-        BEVPOOL_RING_STEP(4) BEVPOOL_RING_STEP(5) BEVPOOL_RING_STEP(6) BEVPOOL_RING_STEP(7)
+    loader_step<kSlots, (J), kRows>(R, lt, kw, xb, ld_bytes, pr, k + (J), nst, buf0, buf1,     \
+                                    rk0s, rk1s);
+      BEVPOOL_RING_STEP(0) BEVPOOL_RING_STEP(1) BEVPOOL_RING_STEP(2) BEVPOOL_RING_STEP(3)
+      BEVPOOL_RING_STEP(4) BEVPOOL_RING_STEP(5) BEVPOOL_RING_STEP(6) BEVPOOL_RING_STEP(7)
 #undef BEVPOOL_RING_STEP
+    }
+  }
+}
+
+// ---- grouped forward accumulation ------------------------------------------
+//
+// Used for depth-weighted context rows, for rows that are no run of aligned
+// 16-byte pieces, for rows of more than kPipeRowBytes and for small inputs
+// (group_plan).  A row is cut into q 16-byte pieces (the last one ends at the
+// row's end and overlaps the piece before it where the row is no multiple of
+// 16 bytes: both lanes then hold and store the same sums), a wave into ng =
+// 64 / q groups of q lanes.  Each group owns the cells that start in its P
+// nominal sorted positions and walks their points in order, lane j keeping
+// the sums of piece j in registers and storing them when the rank changes: no
+// barrier, and one load, 4 (8) products and sums per lane for ng rows at a
+// time, where accum_pipe_kernel spends loader and summer instructions on
+// every row.
+//   * Row addresses, ranks and depth weights of kK points per group are
+//     worked out once, by one lane per point, and read back from the wave's
+//     64 LDS entries; the keys of the batch after next and the weights of the
+//     next one are in flight meanwhile.
+//   * Rows are in flight kK at a time in two register halves: one is added
+//     while the other loads.
+// What bounds it: L2 -> CU traffic of the gathered rows when those are
+// context rows (1 x 360 x 360, C = 80: 568 MB in 55 us, 10.3 TB/s; the
+// pipelined kernel, bound by its instructions per row, took 88; 4 x 360 x 360
+// 204 against 339 us), HBM for feature rows.  There 16-byte aligned rows of
+// one channel block stay with accum_pipe_kernel, whose blocks keep more rows
+// of few cells in flight (131 against 147 us at 1 x 360 x 360).  Rows of 128
+// fp32 channels, two channel blocks to that kernel, take 189 against 215 us;
+// 180-byte fp16 rows at 1.06 M points 81 against 457 us for
+// accum_rows_kernel's element-wise loads.  Walking the ranges in
+// XCD-contiguous eighths cost 5-10%, rings of 4 + 4 rows 3-10%, and a
+// register limit for 4 waves per SIMD spilled.
+//
+// Long cells.  One group would walk a cell of L points as a chain of L / kK
+// round trips, so cells of at least lcell points go to the launch's first
+// blocks instead: a cell of lcell or more sorted points covers a multiple of
+// lcell, so lane l of such a block tests the cell at one multiple and takes
+// it if that is the cell's first.  A long cell is summed by one wave per 64
+// bytes of the row: 16 rows per load, 64 in flight and 64 more being added,
+// transposed through LDS so that lane c adds element c of the rows in order.
+// Every element is still one sequential chain from +0.0 in point order.
+
+// 16 bytes at element alignment (rows need no vector alignment).
+struct __attribute__((packed, aligned(2))) Bytes16 {
+  u32x4 v;
+};
+
+// Rows of the depth-weighted forward (fused depth x context pooling): the row
+// of point p = (bn*D + d)*HW + hw is context row pix = bn*HW + hw, weighted by
+// depth[p] (the reference materialises depth[p] * context[pix, c],
+// models/vtransforms/depth_lss.py:91-94).
+struct DepthRows {
+  const float *depth;  // (BN, D, HW) contiguous: depth[p]
+  FastDiv hw, nd;      // HW and D
+  // p = (bn*D + d)*HW + hw -> bn*HW + hw, with e = p / HW = bn*D + d
+  __device__ __forceinline__ uint32_t pix(uint32_t p) const {
+    const uint32_t e = hw.div(p);
+    return nd.div(e) * hw.d + (p - e * hw.d);
+  }
+};
+
+// The running sums of one lane's 16-byte piece of a row.
+template <typename T>
+struct PieceSum {
+  static constexpr int kE = 16 / int(sizeof(typename T::raw));  // elements per piece
+  float a[kE];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (int i = 0; i < kE; ++i) a[i] = 0.0f;
+  }
+  template <bool kMul>
+  __device__ __forceinline__ void add(u32x4 v, float w) {
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (kE == 4) {
+        // one fp32 product, then the sum (the reference's product and sum)
+        const float x = __uint_as_float(d[i]);
+        a[i] += kMul ? x * w : x;
+      } else {
+        a[2 * i] += T::from_raw(d[i] & 0xffffu);
+        a[2 * i + 1] += T::from_raw(d[i] >> 16);
       }
     }
   }
+  // the sums in the output's element type (16-bit: rounded once)
+  __device__ __forceinline__ u32x4 bits() const {
+    uint32_t d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (kE == 4)
+        d[i] = __float_as_uint(a[i]);
+      else
+        d[i] = uint32_t(T::to_raw(a[2 * i])) | (uint32_t(T::to_raw(a[2 * i + 1])) << 16);
+    }
+    return u32x4{d[0], d[1], d[2], d[3]};
+  }
+};
+
+template <int kRows>
+__device__ __forceinline__ u32x4 load_piece(const char *p) {
+  if constexpr (kRows == kRowsStream) {
+    typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+    return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(p));
+  } else {
+    return reinterpret_cast<const Bytes16 *>(p)->v;
+  }
+}
+
+// Orders this wave's LDS accesses (its lanes exchange data through LDS; one
+// wave's LDS operations complete in order, so no wait is needed).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// kH rows of a group: this lane's pieces, and each row's rank and weight.
+template <int kH>
+struct GroupRing {
+  u32x4 v[kH];
+  int rk[kH];
+  float w[kH];
+};
+
+// Loads the rows of kH entries (ent: row offset, rank, weight).
+template <int kH, int kRows>
+__device__ __forceinline__ void group_load(GroupRing<kH> &R, const u32x4 *ent, const char *xp) {
+#pragma unroll
+  for (int u = 0; u < kH; ++u) {
+    const u32x4 e = ent[u];
+    R.rk[u] = int(e.z);
+    if constexpr (kRows == kRowsDepth) R.w[u] = __uint_as_float(e.w);
+    R.v[u] = load_piece<kRows>(xp + (uint64_t(e.x) | (uint64_t(e.y) << 32)));
+  }
+}
+
+// Adds kH rows; where the rank changes, the finished cell's piece is stored.
+template <typename T, int kH, int kRows>
+__device__ __forceinline__ void group_add(const GroupRing<kH> &R, PieceSum<T> &sum, int &cur,
+                                          bool own, char *op, int64_t out_row_bytes) {
+#pragma unroll
+  for (int u = 0; u < kH; ++u) {
+    if (R.rk[u] != cur) {
+      if (cur >= 0 && own)
+        reinterpret_cast<Bytes16 *>(op + int64_t(cur) * out_row_bytes)->v = sum.bits();
+      sum.clear();
+      cur = R.rk[u];
+    }
+    sum.template add<kRows == kRowsDepth>(R.v[u], kRows == kRowsDepth ? R.w[u] : 0.0f);
+  }
+}
+
+// One wave's share of a long cell: elements of pieces [j0, j0 + 4) of the row
+// (pieces from jend on repeat the last one and are not stored) summed over
+// sorted positions [b0, b1).  tile: the wave's 64 16-byte LDS entries.
+template <typename T, int kRows>
+__device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64_t ld_bytes,
+                                              int row_bytes, int j0, int jend,
+                                              const uint32_t *__restrict__ kw, int b0, int b1,
+                                              char *__restrict__ out_row, u32x4 *tile,
+                                              const DepthRows &dr) {
+  using raw = typename T::raw;
+  constexpr bool kMul = kRows == kRowsDepth;
+  constexpr int kPe = 16 / int(sizeof(raw));  // elements per piece
+  constexpr int kEl = 4 * kPe;                // elements of the four pieces
+  constexpr int kT = 4;                       // 16-row loads in flight
+  const int lane = lane_id(), slot = lane >> 2;
+  const int j = j0 + (lane & 3) < jend ? j0 + (lane & 3) : jend - 1;
+  const char *xp = xb + (16 * j < row_bytes - 16 ? 16 * j : row_bytes - 16);
+  float a = 0.0f, w[kT];
+  u32x4 v[kT];
+  uint32_t idx[kT];
+  auto indices = [&](int base) {  // past the cell: its last point
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      const int p = base + 16 * t + slot;
+      idx[t] = kw[2 * int64_t(p < b1 ? p : b1 - 1)];
+    }
+  };
+  auto rows = [&]() {
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      const uint32_t row = kMul ? dr.pix(idx[t]) : idx[t];
+      if constexpr (kMul) w[t] = dr.depth[idx[t]];
+      v[t] = load_piece<kRows>(xp + int64_t(row) * ld_bytes);
+    }
+  };
+  indices(b0);
+  rows();
+  indices(b0 + 16 * kT);
+  for (int base = b0; base < b1; base += 16 * kT) {
+    u32x4 c[kT];
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      c[t] = v[t];
+      if constexpr (kMul) {
+        const float x0 = __uint_as_float(v[t].x) * w[t];
+        const float x1 = __uint_as_float(v[t].y) * w[t];
+        const float x2 = __uint_as_float(v[t].z) * w[t];
+        const float x3 = __uint_as_float(v[t].w) * w[t];
+        c[t] = u32x4{__float_as_uint(x0), __float_as_uint(x1), __float_as_uint(x2),
+                     __float_as_uint(x3)};
+      }
+    }
+    rows();  // of the next 64 positions, whose indices have arrived
+    indices(base + 32 * kT);
+#pragma unroll
+    for (int t = 0; t < kT; ++t) {
+      const int left = b1 - (base + 16 * t);
+      if (left <= 0) break;
+      wave_lds_order();
+      tile[lane] = c[t];
+      wave_lds_order();
+      const raw *col = reinterpret_cast<const raw *>(tile) + (lane < kEl ? lane : kEl - 1);
+      float x[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) x[u] = T::load(col + u * kEl);
+      if (left >= 16) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) a += x[u];
+      } else {
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+          if (u < left) a += x[u];
+      }
+    }
+  }
+  const int jo = j0 + lane / kPe;
+  if (lane < kEl && jo < jend) {
+    const int pb = 16 * jo < row_bytes - 16 ? 16 * jo : row_bytes - 16;
+    reinterpret_cast<raw *>(out_row + pb)[lane % kPe] = T::to_raw(a);
+  }
+}
+
+constexpr int kLongLanes = 16;  // long-cell candidates per block
+
+// blockIdx.y: block of at most qmax (<= 64) row pieces.  The first
+// long_blocks blocks of x take the long cells, the others the ranges.
+template <typename T, int kK, int kRows>
+__global__ __launch_bounds__(kThreads) void accum_group_kernel(
+    const char *__restrict__ xb, int64_t ld_bytes, int C, int qmax,
+    const uint64_t *__restrict__ keys, const int32_t *__restrict__ meta,
+    const int32_t *__restrict__ cstart, const int32_t *__restrict__ cend, char *__restrict__ acc,
+    int P, int lcell, int long_blocks, DepthRows dr) {
+  constexpr bool kMul = kRows == kRowsDepth;
+  constexpr int kH = kK / 2;
+  __shared__ u32x4 s_ent[kWaves][64];
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  u32x4 *ent = s_ent[wave];
+  const uint32_t *kw = reinterpret_cast<const uint32_t *>(keys);  // low word: point index
+  const int n = meta[BEVPOOL_META_N_KEPT];
+  if (n <= 0) return;
+  const int row_bytes = C * int(sizeof(typename T::raw));
+  const int q0 = int(blockIdx.y) * qmax;
+  const int qt = (row_bytes + 15) >> 4;
+  const int q = qt - q0 < qmax ? qt - q0 : qmax;
+
+  if (int(blockIdx.x) < long_blocks) {
+    const int64_t pos = (int64_t(lane) * long_blocks + blockIdx.x) * lcell;
+    int cs = 0, ce = 0, r = 0;
+    bool found = false;
+    if (lane < kLongLanes && pos < n) {
+      r = key_rank(keys[pos]);
+      cs = cstart[r];
+      ce = cend[r];
+      found = ce - cs >= lcell && int64_t(cs) > pos - lcell;
+    }
+    int task = 0;  // the block's waves take its (cell, four pieces) tasks in turn
+    for (uint64_t m = __ballot(found); m; m &= m - 1) {
+      const int src = __builtin_ctzll(m);
+      const int b0 = __builtin_amdgcn_readlane(cs, src), b1 = __builtin_amdgcn_readlane(ce, src);
+      const int cell = __builtin_amdgcn_readlane(r, src);
+      for (int j0 = q0; j0 < q0 + q; j0 += 4)
+        if ((task++ & (kWaves - 1)) == wave)
+          sum_long_cell<T, kRows>(xb, ld_bytes, row_bytes, j0, q0 + q, kw, b0, b1,
+                                  acc + int64_t(cell) * row_bytes, ent, dr);
+    }
+    return;
+  }
+
+  const int ng = 64 / q < 64 / kK ? 64 / q : 64 / kK;
+  const int64_t gw = (int64_t(blockIdx.x) - long_blocks) * kWaves + wave;
+  if (gw * ng * P >= n) return;  // no barriers below
+  // lanes past the last group repeat its last piece and store nothing
+  const bool own = lane / q < ng;
+  const int g = own ? lane / q : ng - 1;
+  const int li = lane - g * q < q ? lane - g * q : q - 1;
+  const int pb = 16 * (q0 + li) < row_bytes - 16 ? 16 * (q0 + li) : row_bytes - 16;
+  const char *xp = xb + pb;
+  char *op = acc + pb;
+
+  // this group's whole cells: sorted positions [s, e).  A long cell that
+  // starts in the range is its last cell (P < lcell) and ends it.
+  int s, e;
+  {
+    const int64_t p0 = (gw * ng + g) * P, p1 = p0 + P;
+    const int64_t a0 = p0 < n ? p0 : n - 1, a1 = p1 < n ? p1 : n - 1;
+    const int r0 = key_rank(keys[a0]), r0b = key_rank(keys[a0 > 0 ? a0 - 1 : 0]);
+    const int r1 = key_rank(keys[a1]), r1b = key_rank(keys[a1 > 0 ? a1 - 1 : 0]);
+    const int e0 = cend[r0], s1 = cstart[r1], e1 = cend[r1];
+    s = p0 >= n ? n : (p0 == 0 || r0b != r0 ? int(p0) : e0);
+    e = p1 >= n ? n : (r1b != r1 ? int(p1) : (e1 - s1 >= lcell ? s1 : e1));
+  }
+  const int len = e > s ? e - s : 0;
+  int most = len;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_xor(most, o, 64);
+    most = most > y ? most : y;
+  }
+  const int nb = __builtin_amdgcn_readfirstlane((most + kK - 1) / kK);
+  if (nb == 0) return;
+  // this lane's LDS entry: point lane % kK of each batch of group lane / kK
+  const int eg = lane / kK < ng ? lane / kK : ng - 1;
+  const int es = __shfl(s, eg * q, 64), el = __shfl(len, eg * q, 64);
+  const int er = lane % kK;
+
+  auto fetch = [&](int b) -> uint64_t {  // past the group's points: its first key
+    const int i = b * kK + er;
+    return keys[i < el ? es + i : (el > 0 ? es : 0)];
+  };
+  // Entries of batch b.  Past the group's points: rank -2, which ends the
+  // last cell; what is added then is never stored.
+  auto put = [&](int b, uint64_t key, float w) {
+    const uint32_t row = kMul ? dr.pix(key_index(key)) : key_index(key);
+    const uint64_t off = uint64_t(row) * uint64_t(ld_bytes);
+    const int rk = b * kK + er < el ? key_rank(key) : -2;
+    wave_lds_order();
+    ent[lane] = u32x4{uint32_t(off), uint32_t(off >> 32), uint32_t(rk), __float_as_uint(w)};
+    wave_lds_order();
+  };
+
+  PieceSum<T> sum;
+  sum.clear();
+  int cur = -1;
+  GroupRing<kH> A, B;
+  const u32x4 *ge = ent + g * kK;
+  uint64_t k0 = fetch(0), k1 = fetch(1);
+  float w = 0.0f;
+  if constexpr (kMul) w = dr.depth[key_index(k0)];
+  put(0, k0, w);
+  k0 = k1;
+  if constexpr (kMul) w = dr.depth[key_index(k0)];
+  k1 = fetch(2);
+  group_load<kH, kRows>(A, ge, xp);
+  for (int b = 0; b < nb; ++b) {
+    // k0, w: keys and weights of batch b + 1; k1: keys of batch b + 2
+    group_load<kH, kRows>(B, ge + kH, xp);
+    put(b + 1, k0, w);
+    k0 = k1;
+    if constexpr (kMul) w = dr.depth[key_index(k0)];
+    k1 = fetch(b + 3);
+    group_add<T, kH, kRows>(A, sum, cur, own, op, row_bytes);
+    group_load<kH, kRows>(A, ge, xp);
+    group_add<T, kH, kRows>(B, sum, cur, own, op, row_bytes);
+  }
+  if (cur >= 0 && own)
+    reinterpret_cast<Bytes16 *>(op + int64_t(cur) * row_bytes)->v = sum.bits();
 }
 
 // ---------------------------------------------------------------------------
@@ -3230,27 +3527,18 @@ bool bev_vec_ok(const void *base, size_t es, int64_t n_xy, int64_t sb, int64_t s
 
 template <typename T, int kCPL>
 int launch_accum_pipe_t(int slots, unsigned grid, size_t smem, hipStream_t s, const char *x,
-                        int64_t ld_bytes, int C, int CB, const uint64_t *keys,
-                        const int32_t *meta, const int32_t *cend, float *acc,
-                        const DepthRows &dr, bool stream_rows) {
+                        int64_t ld_bytes, int C, const uint64_t *keys, const int32_t *meta,
+                        const int32_t *cend, float *acc, bool stream_rows) {
 #define BEVPOOL_PIPE_CASE(K)                                                                   \
   case K:                                                                                      \
-    if constexpr (std::is_same<T, F32>::value) { /* depth-weighted rows are fp32 only */       \
-      if (dr.depth) {                                                                          \
-        hipLaunchKernelGGL((accum_pipe_kernel<T, K, kCPL, kRowsDepth>), dim3(grid),            \
-                           dim3(kPipeThreads), smem, s, x, ld_bytes, C, CB, keys, meta, cend,  \
-                           acc, kRangePoints, dr);                                            \
-        break;                                                                                 \
-      }                                                                                        \
-    }                                                                                          \
     if (stream_rows)                                                                           \
       hipLaunchKernelGGL((accum_pipe_kernel<T, K, kCPL, kRowsStream>), dim3(grid),             \
-                         dim3(kPipeThreads), smem, s, x, ld_bytes, C, CB, keys, meta, cend,    \
-                         acc, kRangePoints, dr);                                              \
+                         dim3(kPipeThreads), smem, s, x, ld_bytes, C, keys, meta, cend, acc,   \
+                         kRangePoints);                                                        \
     else                                                                                       \
       hipLaunchKernelGGL((accum_pipe_kernel<T, K, kCPL, kRowsPlain>), dim3(grid),              \
-                         dim3(kPipeThreads), smem, s, x, ld_bytes, C, CB, keys, meta, cend,    \
-                         acc, kRangePoints, dr);                                              \
+                         dim3(kPipeThreads), smem, s, x, ld_bytes, C, keys, meta, cend, acc,   \
+                         kRangePoints);                                                        \
     break;
   switch (slots) {
     BEVPOOL_PIPE_CASE(1)
@@ -3259,8 +3547,6 @@ int launch_accum_pipe_t(int slots, unsigned grid, size_t smem, hipStream_t s, co
     BEVPOOL_PIPE_CASE(4)
     BEVPOOL_PIPE_CASE(5)
     BEVPOOL_PIPE_CASE(6)
-    BEVPOOL_PIPE_CASE(7)
-    BEVPOOL_PIPE_CASE(8)
     default:
       return fail(BEVPOOL_EINVAL, "internal: %d slots per thread", slots);
   }
@@ -3268,25 +3554,32 @@ int launch_accum_pipe_t(int slots, unsigned grid, size_t smem, hipStream_t s, co
   return check_launch("accum_pipe");
 }
 
-// Channels per summing lane for a block of CB channels split over kSummers
-// waves: 1 (<= 64 per wave), 2 (<= 128) or 4 (<= 256).
-int pipe_cpl(int CB) {
-  const int cps = (CB + kSummers - 1) / kSummers;
-  return cps <= 64 ? 1 : (cps <= 128 ? 2 : 4);
-}
+// Widest row of the pipelined accumulation: 6 16-byte slots per loader thread
+// and stage, two stages and their ranks in 24.3 KB of LDS.  Wider rows took
+// it several passes; the grouped kernel takes them in one (128 fp32 channels
+// at 1 x 360 x 360: 215 -> 189 us).
+constexpr int kPipeRowBytes = 384;
 
-int launch_accum_pipe(int32_t dtype, int slots, unsigned grid, size_t smem, hipStream_t s,
-                      const char *x, int64_t ld_bytes, int C, int CB, const uint64_t *keys,
-                      const int32_t *meta, const int32_t *cend, float *acc,
-                      const DepthRows &dr, bool stream_rows) {
-  // summing-lane slots: channels for fp32, channel pairs for 16-bit rows
-  const int cpl = dtype == BEVPOOL_F32 ? pipe_cpl(CB) : pipe_cpl((CB + 1) / 2);
-#define BEVPOOL_PIPE_ARGS                                                                      \
-  slots, grid, smem, s, x, ld_bytes, C, CB, keys, meta, cend, acc, dr, stream_rows
+// Pipelined forward accumulation into cell-major rows, for rows of at most
+// kPipeRowBytes that are runs of aligned 16-byte pieces.
+int launch_accum_pipe(int32_t dtype, const char *x, int64_t ld_bytes, int C, int64_t n_points,
+                      const uint64_t *keys, const int32_t *meta, const int32_t *cend, float *acc,
+                      bool stream_rows, hipStream_t s) {
+  const size_t es = dtype_size(dtype);
+  // plain block order: ranges that run at the same time then read rows from
+  // one window of the feature tensor (an XCD-contiguous order measured slower)
+  const unsigned grid = unsigned(ceil_div(n_points, kRangePoints));
+  const int rowq = int(size_t(C) * es / 16);
+  const int slots = (kStageRows * rowq + kLoaders - 1) / kLoaders;
+  const size_t smem = size_t(2) * kStageRows * rowq * 16 + size_t(2) * kStageRows * sizeof(int);
+  // channels (pairs with 16-bit rows) per lane of a summing wave
+  const int lanes = es == 4 ? C : (C + 1) / 2;
+  const bool wide = (lanes + kSummers - 1) / kSummers > 64;
 #define BEVPOOL_PIPE_DTYPE(T)                                                                  \
-  return cpl == 1   ? launch_accum_pipe_t<T, 1>(BEVPOOL_PIPE_ARGS)                            \
-         : cpl == 2 ? launch_accum_pipe_t<T, 2>(BEVPOOL_PIPE_ARGS)                            \
-                    : launch_accum_pipe_t<T, 4>(BEVPOOL_PIPE_ARGS);
+  return wide ? launch_accum_pipe_t<T, 2>(slots, grid, smem, s, x, ld_bytes, C, keys, meta,    \
+                                          cend, acc, stream_rows)                              \
+              : launch_accum_pipe_t<T, 1>(slots, grid, smem, s, x, ld_bytes, C, keys, meta,    \
+                                          cend, acc, stream_rows);
   switch (dtype) {
     case BEVPOOL_F32:
       BEVPOOL_PIPE_DTYPE(F32)
@@ -3296,30 +3589,71 @@ int launch_accum_pipe(int32_t dtype, int slots, unsigned grid, size_t smem, hipS
       BEVPOOL_PIPE_DTYPE(BF16)
   }
 #undef BEVPOOL_PIPE_DTYPE
-#undef BEVPOOL_PIPE_ARGS
 }
 
-// Pipelined forward accumulation (16-byte rows) into cell-major fp32 rows.
-int launch_forward_pipe(int32_t dtype, const char *x, int64_t ld_bytes, int C, int64_t n_points,
-                        const uint64_t *keys, const int32_t *meta, const int32_t *cend,
-                        float *acc, const DepthRows &dr, hipStream_t s) {
-  const size_t es = dtype_size(dtype);
-  // plain block order: ranges that run at the same time then read rows from
-  // one window of the feature tensor (an XCD-contiguous order measured slower)
-  const unsigned grid = unsigned(ceil_div(n_points, kRangePoints));
-  // channel block of at most 384 bytes per row: <= 6 16-byte slots per thread per
-  // stage and two stages + ranks in <= 24.3 KB of LDS
-  const int CBmax = int(384 / es);
-  const int CB = C < CBmax ? C : CBmax;
-  const int rowq = int(size_t(CB) * es / 16);
-  const int slots = (kStageRows * rowq + kLoaders - 1) / kLoaders;
-  const size_t smem = size_t(2) * kStageRows * rowq * 16 + size_t(2) * kStageRows * sizeof(int);
-  if (smem > 65536) return fail(BEVPOOL_EINVAL, "internal: %zu bytes of LDS", smem);
-  // rows of every point (an upper bound of the kept rows read)
-  const bool stream_rows = !dr.depth && n_points * int64_t(C) * int64_t(es) <= kStreamRowBytes;
-  LaunchTimer t("accum_rows", s);
-  return launch_accum_pipe(dtype, slots, grid, smem, s, x, ld_bytes, C, CB, keys, meta, cend, acc,
-                           dr, stream_rows);
+// Shape of a grouped accumulation (accum_group_kernel) of n_points rows.
+struct GroupPlan {
+  int qmax, nblk;   // 16-byte pieces per channel block, channel blocks
+  int kk, ng;       // points per batch and groups per wave
+  int P, lcell;     // nominal points per group, points of a long cell (P < lcell)
+  int64_t waves64;  // waves at 64 points per group
+};
+
+// Points per group: fewer where 64 would leave the chip without waves, since a
+// group's chain of loads is the whole kernel there.  Measured (MI355X, rows
+// of 64-512 bytes, 31 K to 4 M points; us at (P, lcell) = (16, 64), (64, 128),
+// (64, 256)): below 4 waves per CU at 64 points (31 K points, C = 80) 14.1,
+// 14.2, 20.1 and (140 K, C = 16) 14.9, 26, 34; below 16 per CU (498 K points,
+// C = 80, depth-weighted) 26.5, 21.2, 24.6; above (1.99 M) 106, 59, 54.
+constexpr int64_t kGroupFewWaves = 4 * 256, kGroupManyWaves = 16 * 256;
+
+GroupPlan group_plan(int32_t dtype, int C, int64_t n_points) {
+  GroupPlan g;
+  const int qt = int((size_t(C) * dtype_size(dtype) + 15) / 16);
+  g.nblk = (qt + 63) / 64;
+  g.qmax = (qt + g.nblk - 1) / g.nblk;
+  const int per = 64 / g.qmax;  // groups a wave's lanes allow
+  g.kk = per <= 4 ? 16 : (per <= 8 ? 8 : 4);
+  g.ng = per < 64 / g.kk ? per : 64 / g.kk;
+  g.waves64 = ceil_div(ceil_div(n_points, int64_t(64)), int64_t(g.ng));
+  g.P = g.waves64 < kGroupFewWaves ? 16 : 64;
+  g.lcell = g.waves64 < kGroupFewWaves ? 64 : (g.waves64 < kGroupManyWaves ? 128 : 256);
+  return g;
+}
+
+// Grouped forward accumulation into cell-major rows (rows of 16 bytes or
+// more, any element alignment).  dr.depth: context rows, else feature rows.
+int launch_accum_group(int32_t dtype, const GroupPlan &g, const char *x, int64_t ld_bytes, int C,
+                       int64_t n_points, const uint64_t *keys, const int32_t *meta,
+                       const int32_t *cstart, const int32_t *cend, void *acc, const DepthRows &dr,
+                       bool stream_rows, hipStream_t s) {
+  const int long_blocks = int(ceil_div(ceil_div(n_points, int64_t(g.lcell)), kLongLanes));
+  const int64_t waves = ceil_div(ceil_div(n_points, int64_t(g.P)), int64_t(g.ng));
+  const int64_t blocks = long_blocks + ceil_div(waves, kWaves);
+  if (int st = check_grid(blocks, kThreads, "accum_group")) return st;
+  const dim3 grid{unsigned(blocks), unsigned(g.nblk), 1};
+#define BEVPOOL_AG(T, K, M)                                                                    \
+  hipLaunchKernelGGL((accum_group_kernel<T, K, M>), grid, dim3(kThreads), 0, s, x, ld_bytes, C, \
+                     g.qmax, keys, meta, cstart, cend, static_cast<char *>(acc), g.P, g.lcell, \
+                     long_blocks, dr)
+#define BEVPOOL_AG_K(T, M)                                                                     \
+  {                                                                                            \
+    if (g.kk == 16) BEVPOOL_AG(T, 16, M);                                                     \
+    else if (g.kk == 8) BEVPOOL_AG(T, 8, M);                                                  \
+    else BEVPOOL_AG(T, 4, M);                                                                 \
+  }
+#define BEVPOOL_AG_T(T)                                                                        \
+  {                                                                                            \
+    if (stream_rows) BEVPOOL_AG_K(T, kRowsStream) else BEVPOOL_AG_K(T, kRowsPlain)            \
+  }
+  if (dr.depth) BEVPOOL_AG_K(F32, kRowsDepth)
+  else if (dtype == BEVPOOL_F32) BEVPOOL_AG_T(F32)
+  else if (dtype == BEVPOOL_F16) BEVPOOL_AG_T(F16)
+  else BEVPOOL_AG_T(BF16)
+#undef BEVPOOL_AG_T
+#undef BEVPOOL_AG_K
+#undef BEVPOOL_AG
+  return check_launch("accum_group");
 }
 
 // cell-major fp32 rows -> channel-first output (zeros for empty cells).
@@ -3911,46 +4245,45 @@ static int forward_impl(const void *feats, int32_t dtype, int64_t feats_row_stri
   hipStream_t s = static_cast<hipStream_t>(stream);
   float *acc = static_cast<float *>(scratch);
   int st;
-  bool raw16 = false;  // cell rows hold 16-bit output values (pipelined accumulation)
+  bool raw16 = false;  // cell rows hold 16-bit output values (rows of 16 bytes or more)
   if (n_points > 0) {
     const size_t es = dtype_size(dtype);
-    const bool vec16 = (size_t(C) * es) % 16 == 0 && (size_t(feats_row_stride) * es) % 16 == 0 &&
+    const size_t row_bytes = size_t(C) * es;
+    const int64_t ld_bytes = int64_t(size_t(feats_row_stride) * es);
+    const char *x = static_cast<const char *>(feats);
+    const bool vec16 = row_bytes % 16 == 0 && ld_bytes % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(feats) % 16 == 0;
-    // plain block order: ranges that run at the same time then read rows from
-    // one window of the feature tensor (an XCD-contiguous order measured slower)
-    const unsigned grid = unsigned(ceil_div(n_points, kRangePoints));
-    if (vec16) {
-      st = launch_forward_pipe(dtype, static_cast<const char *>(feats),
-                               int64_t(size_t(feats_row_stride) * es), C, n_points, keys, meta,
-                               cell_end, acc, DepthRows{nullptr, {}, {}}, s);
-      if (st) return st;
-      raw16 = es == 2;
+    // rows of every point (an upper bound of the kept rows read)
+    const bool stream_rows = n_points * int64_t(row_bytes) <= kStreamRowBytes;
+    const GroupPlan plan = group_plan(dtype, C, n_points);
+    LaunchTimer t("accum_rows", s);
+    if (vec16 && row_bytes <= size_t(kPipeRowBytes) && plan.waves64 >= kGroupFewWaves) {
+      // From 4 waves per CU on (C = 80: 197 K points) the pipelined blocks are
+      // as fast or faster: 43.9 against 42.4-46 us at 498 K points, 131 against
+      // 147 at 2 M.  Below, the groups' shorter chain is: 20.6 -> 12.5 us at
+      // 31 K points, C = 80, and 18.4 -> 13.4 at C = 16.
+      st = launch_accum_pipe(dtype, x, ld_bytes, C, n_points, keys, meta, cell_end, acc,
+                             stream_rows, s);
+    } else if (row_bytes >= 16) {
+      st = launch_accum_group(dtype, plan, x, ld_bytes, C, n_points, keys, meta, cell_start,
+                              cell_end, acc, DepthRows{nullptr, {}, {}}, stream_rows, s);
     } else {
-      const int CB = C < kThreads ? C : kThreads;
-      int R = 8192 / CB;
-      if (R > 64) R = 64;
-      if (R < 1) R = 1;
-      const size_t smem = size_t(R) * CB * sizeof(float) + size_t(R + 1) * sizeof(int);
-      LaunchTimer t("accum_rows", s);
-      switch (dtype) {
-        case BEVPOOL_F32:
-          hipLaunchKernelGGL(accum_rows_kernel<F32>, dim3(grid), dim3(kThreads), smem, s,
-                             static_cast<const uint32_t *>(feats), feats_row_stride, C, CB, R,
-                             keys, meta, cell_end, acc, kRangePoints);
-          break;
-        case BEVPOOL_F16:
-          hipLaunchKernelGGL(accum_rows_kernel<F16>, dim3(grid), dim3(kThreads), smem, s,
-                             static_cast<const uint16_t *>(feats), feats_row_stride, C, CB, R,
-                             keys, meta, cell_end, acc, kRangePoints);
-          break;
-        default:
-          hipLaunchKernelGGL(accum_rows_kernel<BF16>, dim3(grid), dim3(kThreads), smem, s,
-                             static_cast<const uint16_t *>(feats), feats_row_stride, C, CB, R,
-                             keys, meta, cell_end, acc, kRangePoints);
-          break;
-      }
-      if ((st = check_launch("accum_rows"))) return st;
+      // rows of fewer than 16 bytes: element by element
+      const unsigned grid = unsigned(ceil_div(n_points, kRangePoints));
+      const int R = 64;
+      const size_t smem = size_t(R) * C * sizeof(float) + size_t(R + 1) * sizeof(int);
+#define BEVPOOL_ROWS(T)                                                                        \
+  hipLaunchKernelGGL(accum_rows_kernel<T>, dim3(grid), dim3(kThreads), smem, s,                \
+                     static_cast<const T::raw *>(feats), feats_row_stride, C, R, keys, meta,   \
+                     cell_end, acc, kRangePoints)
+      if (dtype == BEVPOOL_F32) BEVPOOL_ROWS(F32);
+      else if (dtype == BEVPOOL_F16) BEVPOOL_ROWS(F16);
+      else BEVPOOL_ROWS(BF16);
+#undef BEVPOOL_ROWS
+      st = check_launch("accum_rows");
     }
+    if (st) return st;
+    raw16 = es == 2 && row_bytes >= 16;
   }
   return launch_rows_to_bev(acc, dtype, C, cell_start, cell_end, n_cells, n_z, n_xy,
                             out_stride_b, out_stride_c, out_stride_z, out, s, report, raw16);
@@ -4100,8 +4433,10 @@ int bevpool_forward_depth(const float *depth, const float *context_rows, int32_t
   int st;
   if (n_points > 0) {
     const DepthRows dr{depth, make_fast_div(uint32_t(HW)), make_fast_div(uint32_t(D))};
-    st = launch_forward_pipe(BEVPOOL_F32, reinterpret_cast<const char *>(context_rows),
-                             int64_t(C) * 4, C, n_points, keys, meta, cell_end, acc, dr, s);
+    LaunchTimer t("accum_rows", s);
+    st = launch_accum_group(BEVPOOL_F32, group_plan(BEVPOOL_F32, C, n_points),
+                            reinterpret_cast<const char *>(context_rows), int64_t(C) * 4, C,
+                            n_points, keys, meta, cell_start, cell_end, acc, dr, false, s);
     if (st) return st;
   }
   return launch_rows_to_bev(acc, BEVPOOL_F32, C, cell_start, cell_end, n_cells, n_z, n_xy,

@@ -1,0 +1,71 @@
+"""The grouped forward accumulation at the sizes where it can go wrong: rows
+of one 16-byte piece up to two blocks of 64, pieces that overlap, cells
+around the points per batch, per group and per long cell in each of its three
+regimes, against the CPU oracle.  Forward bit-exact (16-bit: the fp32 sum
+rounded once), backward a copy."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import torch_fallback as ref
+from test_gpu_op import assert_bit_equal, run_op
+
+pytestmark = pytest.mark.gpu
+
+# points per cell, in rank order (0: an empty cell), around 4/8/16 points a
+# batch, 16/64 a group and 64/128/256 a long cell
+LENGTHS = [1, 2, 3, 4, 5, 7, 8, 9, 0, 15, 16, 17, 31, 32, 33, 0, 63, 64, 65, 1, 127, 128, 129, 255,
+           256, 257, 0, 0, 300, 511, 512, 513, 1, 1500, 64, 64, 128, 256]
+
+F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
+
+
+@pytest.mark.parametrize('C,dtype,N', [
+    (3, F32, 9000), (4, F32, 9000), (5, F32, 9000), (12, F32, 9000), (16, F32, 9000),
+    (80, F32, 20000), (97, F32, 9000), (100, F32, 9000), (255, F32, 9000), (257, F32, 9000),
+    (7, BF16, 9000), (8, F16, 9000), (9, BF16, 9000), (90, F16, 9000), (513, BF16, 9000),
+    (256, F32, 70000), (256, F32, 270000),  # 64 points a group, long cells from 128 and 256
+])
+def test_cell_lengths(pkg, cuda, C, dtype, N):
+    g = torch.Generator().manual_seed(C + N)
+    H, W = 40, 50
+    lengths = torch.tensor(LENGTHS)
+    spare = N - int(lengths.sum())
+    rank = torch.cat((torch.arange(len(LENGTHS)).repeat_interleave(lengths),
+                      torch.randint(len(LENGTHS), H * W, (spare,), generator=g)))
+    rank = rank[torch.randperm(N, generator=g)]
+    coords = torch.stack((rank // W, rank % W, rank * 0, rank * 0), 1).to(torch.int32)
+    feats = torch.randn((N, C), generator=g).to(dtype)
+    out, grad, up = run_op(pkg, feats, coords, (1, 1, H, W), cuda)
+    assert_bit_equal(out, ref.bev_pool(feats.float(), coords, 1, 1, H, W).to(dtype), 'forward')
+    want = up.to(dtype).permute(0, 2, 3, 4, 1).reshape(H * W, C)[rank]
+    assert_bit_equal(grad, want, 'backward')
+
+
+@pytest.mark.parametrize('offset', [1, 2, 3])
+@pytest.mark.parametrize('C,dtype', [(80, F32), (64, F16), (33, BF16)])
+def test_unaligned_rows(pkg, cuda, C, dtype, offset):
+    """Feature rows that start at any element of a wider storage."""
+    g = torch.Generator().manual_seed(offset)
+    N, H, W = 3001, 13, 11
+    store = torch.randn((N, C + 7), generator=g).to(dtype)
+    feats = store[:, offset:offset + C]
+    coords = torch.stack([torch.randint(0, n, (N,), generator=g) for n in (H, W, 1, 1)], 1)
+    out = pkg.bev_pool(store.to(cuda)[:, offset:offset + C], coords.to(cuda), 1, 1, H, W)
+    assert_bit_equal(out, ref.bev_pool(feats.float(), coords, 1, 1, H, W).to(dtype), 'forward')
+
+
+@pytest.mark.parametrize('C', [4, 60, 100, 252, 256])
+def test_depth_rows(pkg, cuda, C):
+    from bevfusion_triton_amd import synthetic
+
+    case = synthetic.make_case('tiny', features=False)
+    B, N, D, fH, fW = case.geom.shape[:5]
+    g = torch.Generator().manual_seed(C)
+    depth = torch.randn(B * N, D, fH, fW, generator=g).softmax(1)
+    context = torch.randn(B * N, C, fH, fW, generator=g)
+    dx, bx, nx = ref.gen_dx_bx(case.xbound, case.ybound, case.zbound)
+    module = pkg.BevPoolTransform(case.xbound, case.ybound, case.zbound).to(cuda)
+    out = module.bev_pool_depth(case.geom.to(cuda), depth.to(cuda), context.to(cuda))
+    assert_bit_equal(out, ref.lss_bev_pool_depth(case.geom, depth, context, dx, bx, nx), 'forward')
