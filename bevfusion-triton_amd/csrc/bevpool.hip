@@ -339,6 +339,17 @@ __device__ int block_exclusive_scan(int v, int *scratch, int *total) {
   return before + x - v;
 }
 
+// 16 and 8 bytes at element alignment: gfx950 loads and stores them in one
+// instruction at any address, so rows need no vector alignment.
+struct __attribute__((packed, aligned(2))) Bytes16 {
+  u32x4 v;
+};
+struct __attribute__((packed, aligned(2))) Bytes8 {
+  u32x2 v;
+};
+typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+typedef u32x2 __attribute__((aligned(2))) u32x2_any;
+
 // fp32 / fp16 / bf16 element conversion.
 struct F32 {
   using raw = uint32_t;
@@ -2016,11 +2027,6 @@ __global__ __launch_bounds__(kPipeThreads) void accum_pipe_kernel(
 // transposed through LDS so that lane c adds element c of the rows in order.
 // Every element is still one sequential chain from +0.0 in point order.
 
-// 16 bytes at element alignment (rows need no vector alignment).
-struct __attribute__((packed, aligned(2))) Bytes16 {
-  u32x4 v;
-};
-
 // Rows of the depth-weighted forward (fused depth x context pooling): the row
 // of point p = (bn*D + d)*HW + hw is context row pix = bn*HW + hw, weighted by
 // depth[p] (the reference materialises depth[p] * context[pix, c],
@@ -2076,7 +2082,6 @@ struct PieceSum {
 template <int kRows>
 __device__ __forceinline__ u32x4 load_piece(const char *p) {
   if constexpr (kRows == kRowsStream) {
-    typedef u32x4 __attribute__((aligned(2))) u32x4_any;
     return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any *>(p));
   } else {
     return reinterpret_cast<const Bytes16 *>(p)->v;
@@ -2340,11 +2345,16 @@ __global__ __launch_bounds__(kThreads) void accum_group_kernel(
 // A tile is 64 consecutive cells (ranks); rows are staged in LDS as
 // [cell][channel] with a pitch of CT + 1 elements, CT = channels per pass.
 // On the channel-first side each thread moves 4 consecutive cells of one
-// channel: one 16-byte (fp32) or 8-byte (16-bit) access when kVecBev (n_xy,
-// the b/z/c strides and the base are multiples of 4 elements, so 4 cells
-// starting at a multiple of 4 share a (b, z) plane and are contiguous), else
-// one access per cell.  On the row side kVecRow moves 16-byte pieces of a row
-// (C * element size a multiple of 16).
+// channel with one 16-byte (fp32) or 8-byte (16-bit) access.  With kVecBev
+// (n_xy, the b/z/c strides and the base are multiples of 4 elements) 4 cells
+// starting at a multiple of 4 always share a (b, z) plane and the access is
+// aligned; otherwise it is an access at element alignment, and the few groups
+// of 4 cells that a plane's end cuts go cell by cell.  On the row side
+// kVecRow (rows of 16 bytes or more) moves 16-byte pieces of a row; where the
+// row is no multiple of 16 bytes the last piece ends at the row's end and
+// overlaps the one before it.  Measured (MI355X, 3 x 201 x 199 cells of 90
+// fp16 channels, which no vector width divides): rows_to_bev 32.6 -> 18.9,
+// bev_to_rows 21.8 -> 15.8 us against element-wise loads and stores.
 
 // Offset of cell `cell` (< 2^31) in a channel-first (b, c, z, xy) tensor
 // without the channel term.
@@ -2354,28 +2364,6 @@ __device__ __forceinline__ int64_t cell_offset(uint32_t cell, uint32_t n_z, uint
   const uint32_t b = cell / per_b, rem = cell - b * per_b;
   const uint32_t z = rem / n_xy, xy = rem - z * n_xy;
   return int64_t(b) * sb + int64_t(z) * sz + int64_t(xy);
-}
-
-// Per-tile cell table in LDS: occupied flag and channel-first offset (-1 past
-// the last cell).  Returns whether any cell of the tile is occupied.
-__device__ __forceinline__ bool load_tile_cells(int64_t cell0, int64_t n_cells,
-                                                const int32_t *__restrict__ cstart,
-                                                const int32_t *__restrict__ cend, int n_z,
-                                                int64_t n_xy, int64_t sb, int64_t sz, int *occ,
-                                                int64_t *off) {
-  const int tid = threadIdx.x;
-  int mine = 0;
-  if (tid < kCellTile) {
-    const int64_t cell = cell0 + tid;
-    if (cell < n_cells) {
-      mine = cend[cell] > cstart[cell] ? 1 : 0;
-      off[tid] = cell_offset(uint32_t(cell), uint32_t(n_z), uint32_t(n_xy), sb, sz);
-    } else {
-      off[tid] = -1;
-    }
-    occ[tid] = mine;
-  }
-  return __syncthreads_or(mine) != 0;
 }
 
 // acc rows (cell-major fp32, written for occupied cells only) -> out
@@ -2437,16 +2425,15 @@ __global__ void meta_report_kernel(const int32_t *__restrict__ meta, int32_t *__
 // otherwise they are fp32 sums converted on the way out.
 template <typename T, bool kVecRow, bool kVecBev, bool kRaw16 = false>
 __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
-    const float *__restrict__ acc, int C, int CT, const int32_t *__restrict__ cstart,
-    const int32_t *__restrict__ cend, int64_t n_cells, int n_z, int64_t n_xy, int64_t sb,
-    int64_t sc, int64_t sz, typename T::raw *__restrict__ out, MetaReport report) {
+    const float *__restrict__ acc, int C, int CT, const int32_t *__restrict__ cend,
+    int64_t n_cells, int n_z, int64_t n_xy, int64_t sb, int64_t sc, int64_t sz,
+    typename T::raw *__restrict__ out, MetaReport report) {
   using raw = typename T::raw;
   static_assert(!kRaw16 || sizeof(raw) == 2, "16-bit rows for 16-bit output only");
   write_meta_report(report);
   extern __shared__ uint32_t tile_bits[];  // kCellTile * (CT + 1)
   __shared__ int occ[kCellTile];
   __shared__ int64_t off[kCellTile];
-  (void)cstart;
   const int tid = threadIdx.x;
   const int64_t cell0 = int64_t(blockIdx.x) * kCellTile;
   const uint32_t *accb = reinterpret_cast<const uint32_t *>(acc);
@@ -2479,7 +2466,8 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
     const int cb = C - c0 < CT ? C - c0 : CT;
     if (kVecRow) {
       constexpr uint32_t kPer = kRaw16 ? 8 : 4;  // channels per 16-byte piece
-      const uint32_t q = uint32_t(cb) / kPer;    // 16-byte pieces per row
+      const uint32_t q = (uint32_t(cb) + kPer - 1) / kPer;  // 16-byte pieces per row
+      const uint32_t last = uint32_t(cb) - kPer;            // first channel of the last one
       const uint32_t n_items = kCellTile * q;
       u32x4 v[kTileSlots];
 #pragma unroll
@@ -2487,10 +2475,10 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
         const uint32_t i = tid + it * kThreads;
         uint32_t t = i / q, k = i - t * q;
         if (i >= n_items || cell0 + t >= n_cells) t = k = 0;
-        const void *src = kRaw16
-                              ? static_cast<const void *>(acch + (cell0 + t) * C + c0 + kPer * k)
-                              : static_cast<const void *>(accb + (cell0 + t) * C + c0 + kPer * k);
-        v[it] = ((occm >> t) & 1) ? *reinterpret_cast<const u32x4 *>(src)
+        const uint32_t c = kPer * k < last ? kPer * k : last;
+        const void *src = kRaw16 ? static_cast<const void *>(acch + (cell0 + t) * C + c0 + c)
+                                 : static_cast<const void *>(accb + (cell0 + t) * C + c0 + c);
+        v[it] = ((occm >> t) & 1) ? reinterpret_cast<const Bytes16 *>(src)->v
                                   : u32x4{0u, 0u, 0u, 0u};
       }
       if (c0 == 0 && tid < kCellTile) {
@@ -2502,7 +2490,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
         const uint32_t i = tid + it * kThreads;
         if (i < n_items) {
           const uint32_t t = i / q, k = i - t * q;
-          uint32_t *d = tile_bits + t * pitch + kPer * k;
+          uint32_t *d = tile_bits + t * pitch + (kPer * k < last ? kPer * k : last);
           if constexpr (kRaw16) {  // 8 values, low half first
             d[0] = v[it].x & 0xffffu;
             d[1] = v[it].x >> 16;
@@ -2540,8 +2528,8 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
         else
           r[u] = T::to_raw(__builtin_bit_cast(float, b));
       }
-      if (kVecBev) {
-        if (off[j] < 0) continue;
+      if (kVecBev && off[j] < 0) continue;
+      if (kVecBev || (off[j] >= 0 && off[j + 3] == off[j] + 3)) {
         raw *dst = out + off[j] + int64_t(c0 + c) * sc;
         if constexpr (sizeof(raw) == 4) {
           u32x4 w;
@@ -2549,12 +2537,18 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
           w.y = r[1];
           w.z = r[2];
           w.w = r[3];
-          __builtin_nontemporal_store(w, reinterpret_cast<u32x4 *>(dst));
+          if constexpr (kVecBev)
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x4 *>(dst));
+          else
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any *>(dst));
         } else {
           u32x2 w;
           w.x = uint32_t(r[0]) | (uint32_t(r[1]) << 16);
           w.y = uint32_t(r[2]) | (uint32_t(r[3]) << 16);
-          __builtin_nontemporal_store(w, reinterpret_cast<u32x2 *>(dst));
+          if constexpr (kVecBev)
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x2 *>(dst));
+          else
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x2_any *>(dst));
         }
       } else {
 #pragma unroll
@@ -2571,121 +2565,112 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
 // ---------------------------------------------------------------------------
 
 // grad (channel-first, any b/c/z strides, xy contiguous) -> cell-major rows of
-// the occupied cells (raw bits copied).  With kVecBev each thread always
-// handles the same 4 cells (j = 4 * (tid % 16)) of channels tid / 16 + 16 it;
-// all its tile loads are issued up front (clamped in-bounds addresses,
-// empty cells included) together with the occupancy loads, or, with
-// occ_first, after reading its 4 cells' occupancy (none when all 4 are
-// empty).
+// the occupied cells (raw bits copied).  Each thread always handles the same
+// 4 cells (j = 4 * (tid % 16)) of channels tid / 16 + 16 it; all its tile
+// loads are issued up front (clamped in-bounds addresses, empty cells
+// included) together with the occupancy loads, or, with occ_first, after
+// reading its 4 cells' occupancy (none when all 4 are empty).
 template <typename TR, bool kVecRow, bool kVecBev>
 __global__ __launch_bounds__(kThreads) void bev_to_rows_kernel(
-    const TR *__restrict__ grad, int C, int CT, const int32_t *__restrict__ cstart,
-    const int32_t *__restrict__ cend, int64_t n_cells, int n_z, int64_t n_xy, int64_t sb,
-    int64_t sc, int64_t sz, bool occ_first, TR *__restrict__ rows) {
+    const TR *__restrict__ grad, int C, int CT, const int32_t *__restrict__ cend,
+    int64_t n_cells, int n_z, int64_t n_xy, int64_t sb, int64_t sc, int64_t sz, bool occ_first,
+    TR *__restrict__ rows) {
   extern __shared__ u32x4 smem_b2r[];
   TR *tile = reinterpret_cast<TR *>(smem_b2r);  // kCellTile * (CT + 1)
   __shared__ int occ[kCellTile];
-  __shared__ int64_t off[kCellTile];
   const int tid = threadIdx.x;
   const int64_t cell0 = int64_t(blockIdx.x) * kCellTile;
   const int pitch = CT + 1;
   constexpr int kPer = 16 / int(sizeof(TR));  // elements per 16-byte row piece
-  if (kVecBev) {
-    (void)cstart;
-    const int j = (tid & 15) * 4;
-    const bool live = cell0 + j < n_cells;  // then all 4 cells are (n_cells % 4 == 0)
-    const int64_t offj =
-        cell_offset(uint32_t(live ? cell0 + j : cell0), uint32_t(n_z), uint32_t(n_xy), sb, sz);
-    // sparse grids: the 4 cells' occupancy first, no gradient loads when all are empty
-    bool need = true;
-    if (occ_first) {
-      need = false;
-      if (live)
+  const int j = (tid & 15) * 4;
+  // with kVecBev a live thread's 4 cells all exist (n_cells % 4 == 0)
+  const bool live = cell0 + j < n_cells;
+  const int64_t offj =
+      cell_offset(uint32_t(live ? cell0 + j : cell0), uint32_t(n_z), uint32_t(n_xy), sb, sz);
+  // are they 4 consecutive elements of a channel?
+  const bool run =
+      kVecBev || (cell0 + j + 3 < n_cells &&
+                  cell_offset(uint32_t(cell0 + j + 3), uint32_t(n_z), uint32_t(n_xy), sb, sz) ==
+                      offj + 3);
+  // sparse grids: the 4 cells' occupancy first, no gradient loads when all are empty
+  bool need = kVecBev || live;
+  if (occ_first) {
+    need = false;
+    if (live)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) need |= cend[cell0 + j + u] != 0;
-    }
-    for (int c0 = 0; c0 < C; c0 += CT) {
-      const int cb = C - c0 < CT ? C - c0 : CT;
-      using V = typename std::conditional<sizeof(TR) == 4, u32x4, u32x2>::type;
-      V v[kTileSlots];
+      for (int u = 0; u < 4; ++u)
+        need |= (kVecBev || cell0 + j + u < n_cells) && cend[cell0 + j + u] != 0;
+  }
+  for (int c0 = 0; c0 < C; c0 += CT) {
+    const int cb = C - c0 < CT ? C - c0 : CT;
+    using V = typename std::conditional<sizeof(TR) == 4, u32x4, u32x2>::type;
+    using VA = typename std::conditional<sizeof(TR) == 4, Bytes16, Bytes8>::type;
+    V v[kTileSlots];
+    if (run) {
 #pragma unroll
       for (int it = 0; it < kTileSlots; ++it) {
         int c = (tid >> 4) + 16 * it;
         c = c < cb ? c : 0;
-        v[it] = need ? *reinterpret_cast<const V *>(grad + offj + int64_t(c0 + c) * sc) : V{};
+        const TR *src = grad + offj + int64_t(c0 + c) * sc;
+        if constexpr (kVecBev)
+          v[it] = need ? *reinterpret_cast<const V *>(src) : V{};
+        else
+          v[it] = need ? reinterpret_cast<const VA *>(src)->v : V{};
       }
-      // the cells' occupancy, loaded after the gradient loads so that one
-      // round trip brings both
-      if (c0 == 0 && tid < kCellTile)
-        occ[tid] = cell0 + tid < n_cells && cend[cell0 + tid] != 0 ? 1 : 0;
-#pragma unroll
-      for (int it = 0; it < kTileSlots; ++it) {
-        const int c = (tid >> 4) + 16 * it;
-        if (c < cb) {
-          TR e[4];
-          if constexpr (sizeof(TR) == 4) {
-            e[0] = v[it].x;
-            e[1] = v[it].y;
-            e[2] = v[it].z;
-            e[3] = v[it].w;
-          } else {
-            e[0] = TR(v[it].x);
-            e[1] = TR(v[it].x >> 16);
-            e[2] = TR(v[it].y);
-            e[3] = TR(v[it].y >> 16);
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) tile[(j + u) * pitch + c] = e[u];
-        }
-      }
-      __syncthreads();
-      if (kVecRow) {
-        const uint32_t q = uint32_t(cb) / kPer;  // 16-byte pieces per row
-        for (uint32_t i = tid; i < kCellTile * q; i += kThreads) {
-          const uint32_t t = i / q, k = i - t * q;
-          if (!occ[t]) continue;
-          const TR *srow = tile + t * pitch + kPer * k;
-          u32x4 w;
-          if constexpr (sizeof(TR) == 4) {
-            w.x = srow[0];
-            w.y = srow[1];
-            w.z = srow[2];
-            w.w = srow[3];
-          } else {
-            w.x = uint32_t(srow[0]) | (uint32_t(srow[1]) << 16);
-            w.y = uint32_t(srow[2]) | (uint32_t(srow[3]) << 16);
-            w.z = uint32_t(srow[4]) | (uint32_t(srow[5]) << 16);
-            w.w = uint32_t(srow[6]) | (uint32_t(srow[7]) << 16);
-          }
-          *reinterpret_cast<u32x4 *>(rows + (cell0 + t) * C + c0 + kPer * k) = w;
-        }
-      } else {
-        for (uint32_t i = tid; i < uint32_t(kCellTile * cb); i += kThreads) {
-          const uint32_t t = i / uint32_t(cb), c = i - t * uint32_t(cb);
-          if (occ[t]) rows[(cell0 + t) * C + c0 + c] = tile[t * pitch + c];
-        }
-      }
-      __syncthreads();
-    }
-    return;
-  }
-  // general strides: per-cell loads after the occupancy test
-  if (!load_tile_cells(cell0, n_cells, cstart, cend, n_z, n_xy, sb, sz, occ, off)) return;
-  for (int c0 = 0; c0 < C; c0 += CT) {
-    const int cb = C - c0 < CT ? C - c0 : CT;
-    for (int i = tid; i < cb * (kCellTile / 4); i += kThreads) {
-      const int c = i >> 4, j = (i & 15) * 4;
+    } else {
+      // a plane or the grid ends among the 4 cells
+      int64_t ou[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        tile[(j + u) * pitch + c] = occ[j + u] ? grad[off[j + u] + int64_t(c0 + c) * sc] : TR(0);
+        ou[u] = cell0 + j + u < n_cells ? cell_offset(uint32_t(cell0 + j + u), uint32_t(n_z),
+                                                      uint32_t(n_xy), sb, sz)
+                                        : offj;
+#pragma unroll
+      for (int it = 0; it < kTileSlots; ++it) {
+        int c = (tid >> 4) + 16 * it;
+        c = c < cb ? c : 0;
+        uint32_t e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) e[u] = need ? grad[ou[u] + int64_t(c0 + c) * sc] : 0u;
+        if constexpr (sizeof(TR) == 4)
+          v[it] = u32x4{e[0], e[1], e[2], e[3]};
+        else
+          v[it] = u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
+      }
+    }
+    // the cells' occupancy, loaded after the gradient loads so that one
+    // round trip brings both
+    if (c0 == 0 && tid < kCellTile)
+      occ[tid] = cell0 + tid < n_cells && cend[cell0 + tid] != 0 ? 1 : 0;
+#pragma unroll
+    for (int it = 0; it < kTileSlots; ++it) {
+      const int c = (tid >> 4) + 16 * it;
+      if (c < cb) {
+        TR e[4];
+        if constexpr (sizeof(TR) == 4) {
+          e[0] = v[it].x;
+          e[1] = v[it].y;
+          e[2] = v[it].z;
+          e[3] = v[it].w;
+        } else {
+          e[0] = TR(v[it].x);
+          e[1] = TR(v[it].x >> 16);
+          e[2] = TR(v[it].y);
+          e[3] = TR(v[it].y >> 16);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) tile[(j + u) * pitch + c] = e[u];
+      }
     }
     __syncthreads();
     if (kVecRow) {
-      const uint32_t q = uint32_t(cb) / kPer;
+      const uint32_t q = (uint32_t(cb) + kPer - 1) / kPer;  // 16-byte pieces per row
+      const uint32_t last = uint32_t(cb) - kPer;
       for (uint32_t i = tid; i < kCellTile * q; i += kThreads) {
         const uint32_t t = i / q, k = i - t * q;
         if (!occ[t]) continue;
-        const TR *srow = tile + t * pitch + kPer * k;
+        const uint32_t c = kPer * k < last ? kPer * k : last;
+        const TR *srow = tile + t * pitch + c;
         u32x4 w;
         if constexpr (sizeof(TR) == 4) {
           w.x = srow[0];
@@ -2698,7 +2683,7 @@ __global__ __launch_bounds__(kThreads) void bev_to_rows_kernel(
           w.z = uint32_t(srow[4]) | (uint32_t(srow[5]) << 16);
           w.w = uint32_t(srow[6]) | (uint32_t(srow[7]) << 16);
         }
-        *reinterpret_cast<u32x4 *>(rows + (cell0 + t) * C + c0 + kPer * k) = w;
+        reinterpret_cast<Bytes16 *>(rows + (cell0 + t) * C + c0 + c)->v = w;
       }
     } else {
       for (uint32_t i = tid; i < uint32_t(kCellTile * cb); i += kThreads) {
@@ -2736,8 +2721,9 @@ struct GatherWarm {
   int64_t xcd_span;      // gather pieces (vectors of xg) per XCD
   int vpr;               // gather pieces per point
   int per_xcd;           // rank blocks per XCD
-  const u32x4 *rows16;   // gradient rows as 16-byte pieces (null: skip)
-  int rowq;              // 16-byte pieces per row
+  const char *rows;      // gradient rows, 16 bytes or more each (null: skip)
+  int rowq;              // 16-byte pieces per row (as gather_rows_kernel's)
+  int row_bytes;
 };
 
 // Warm-up work of block wb (< warm_blocks(w, tiles)); returns nothing, reads only.
@@ -2766,7 +2752,7 @@ __device__ __forceinline__ void gather_warm_block(const GatherWarm &w, int wb, i
       const u32x4 v = w.rank16[i];
       m ^= v.x ^ v.y ^ v.z ^ v.w;
     }
-  } else if (w.rows16) {
+  } else if (w.rows) {
     // kWarmCells consecutive cells per block: occupancy, then the occupied
     // rows' pieces, kWarmBatch loads in flight per thread
     const int64_t cell0 = int64_t(wb - rank_blocks) * kWarmCells;
@@ -2783,7 +2769,9 @@ __device__ __forceinline__ void gather_warm_block(const GatherWarm &w, int wb, i
       for (int b = 0; b < kWarmBatch; ++b) {
         const uint32_t i = i0 + uint32_t(b) * kThreads < n ? i0 + uint32_t(b) * kThreads : n - 1;
         const uint32_t t = i / q, k = i - t * q;
-        v[b] = occ[t] ? w.rows16[(cell0 + t) * q + k] : u32x4{0u, 0u, 0u, 0u};
+        const int o = int(16 * k) < w.row_bytes - 16 ? int(16 * k) : w.row_bytes - 16;
+        v[b] = occ[t] ? reinterpret_cast<const Bytes16 *>(w.rows + (cell0 + t) * w.row_bytes + o)->v
+                      : u32x4{0u, 0u, 0u, 0u};
       }
 #pragma unroll
       for (int b = 0; b < kWarmBatch; ++b) m ^= v[b].x ^ v[b].y ^ v[b].z ^ v[b].w;
@@ -2793,27 +2781,23 @@ __device__ __forceinline__ void gather_warm_block(const GatherWarm &w, int wb, i
 }
 
 // x_grad[p, :] = rows[rank[p], :] (kept) or 0 (dropped); point order, so the
-// writes stream.  V is a 16-byte vector when rows allow it, else one element.
-// Each thread copies kGatherPer vectors spaced kThreads apart (coalesced),
-// blocks walk XCD-contiguous chunks (an XCD's points map to a compact set of
-// cells, whose rows then stay in its L2), and the destination is written
-// with non-temporal stores (it is not read again here, and keeping it out of
-// L2 leaves room for the gradient rows).  Each piece is a dependent chain
-// rank -> row -> store, so the leading warm_blocks blocks first pull the ranks
-// and the rows into the caches (gather_warm_block).  kNarrow: indices fit in 32
-// bits.
-#ifndef BEVPOOL_GATHER_PER
-#define BEVPOOL_GATHER_PER 1
-#endif
-#ifndef BEVPOOL_GATHER_NT
-#define BEVPOOL_GATHER_NT 1
-#endif
-constexpr int kGatherPer = BEVPOOL_GATHER_PER;
-
-template <typename V, bool kNarrow>
+// writes stream.  A row is moved as vpr vectors V: 16-byte ones for rows of
+// 16 bytes or more (kAny: at element alignment, the last one ending at the
+// row's end and overlapping the one before it with the same bytes), else
+// elements.  Each thread copies one vector, blocks walk XCD-contiguous chunks
+// (an XCD's points map to a compact set of cells, whose rows then stay in its
+// L2), and the destination is written with non-temporal stores (it is not
+// read again here, and keeping it out of L2 leaves room for the gradient
+// rows).  Each piece is a dependent chain rank -> row -> store, so the leading
+// warm_blocks blocks first pull the ranks and the rows into the caches
+// (gather_warm_block).  kNarrow: indices fit in 32 bits.  What bounds it is
+// the write stream (6.6 TB/s at 1 x 360 x 360, C = 80; a fill reaches 6.9).
+// Rows of 90 fp16 values (1.06 M points, 191 MB written) take 38 us with
+// unaligned 16-byte vectors, 147 element by element.
+template <typename V, bool kNarrow, bool kAny>
 __global__ __launch_bounds__(kThreads) void gather_rows_kernel(
-    const V *__restrict__ rows, int vpr, const int32_t *__restrict__ rank, int64_t n_points,
-    V *__restrict__ xg, int64_t xg_ld, int warm_blocks, GatherWarm w,
+    const char *__restrict__ rows, int vpr, int row_bytes, const int32_t *__restrict__ rank,
+    int64_t n_points, char *__restrict__ xg, int64_t xg_ld, int warm_blocks, GatherWarm w,
     const int32_t *__restrict__ cstart, const int32_t *__restrict__ cend, int64_t n_cells,
     int never, int zero_dropped) {
   // the first warm_blocks blocks (a multiple of 8, so XCD parity is kept)
@@ -2825,32 +2809,31 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(
   }
   const int64_t total = n_points * vpr;
   const int64_t gb = int64_t(blockIdx.x) - warm_blocks;
-  const int64_t base =
-      xcd_chunk(gb, int64_t(gridDim.x) - warm_blocks) * (kThreads * kGatherPer) + threadIdx.x;
-#pragma unroll
-  for (int j = 0; j < kGatherPer; ++j) {
-    const int64_t i = base + j * kThreads;
-    if (i < total) {
-      int64_t p;
-      int q;
-      if (kNarrow) {
-        const uint32_t ui = uint32_t(i), up = ui / uint32_t(vpr);
-        p = up;
-        q = int(ui - up * uint32_t(vpr));
-      } else {
-        p = i / vpr;
-        q = int(i - p * vpr);
-      }
-      const int r = rank[p];
-      V v = V{};
-      if (r >= 0) v = rows[int64_t(r) * vpr + q];
-      else if (!zero_dropped) continue;  // the caller keeps dropped rows as they are
-#if BEVPOOL_GATHER_NT
-      __builtin_nontemporal_store(v, xg + p * xg_ld + q);
-#else
-      xg[p * xg_ld + q] = v;
-#endif
-    }
+  const int64_t i = xcd_chunk(gb, int64_t(gridDim.x) - warm_blocks) * kThreads + threadIdx.x;
+  if (i >= total) return;
+  int64_t p;
+  int q;
+  if (kNarrow) {
+    const uint32_t ui = uint32_t(i), up = ui / uint32_t(vpr);
+    p = up;
+    q = int(ui - up * uint32_t(vpr));
+  } else {
+    p = i / vpr;
+    q = int(i - p * vpr);
+  }
+  int o = q * int(sizeof(V));
+  if (kAny) o = o < row_bytes - 16 ? o : row_bytes - 16;
+  const int r = rank[p];
+  if (r < 0 && !zero_dropped) return;  // the caller keeps dropped rows as they are
+  char *dst = xg + p * xg_ld + o;
+  if constexpr (kAny) {
+    u32x4 v = u32x4{0u, 0u, 0u, 0u};
+    if (r >= 0) v = reinterpret_cast<const Bytes16 *>(rows + int64_t(r) * row_bytes + o)->v;
+    __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any *>(dst));
+  } else {
+    V v = V{};
+    if (r >= 0) v = *reinterpret_cast<const V *>(rows + int64_t(r) * row_bytes + o);
+    __builtin_nontemporal_store(v, reinterpret_cast<V *>(dst));
   }
 }
 
@@ -3656,27 +3639,33 @@ int launch_accum_group(int32_t dtype, const GroupPlan &g, const char *x, int64_t
   return check_launch("accum_group");
 }
 
+// Channels per transpose pass: at most kTileChannels, the passes about equal
+// (so that the last one too holds a whole 16-byte piece) and multiples of 8.
+int tile_channels(int C) {
+  const int passes = (C + kTileChannels - 1) / kTileChannels;
+  const int per = ((C + passes - 1) / passes + 7) / 8 * 8;
+  return C < per ? C : per;
+}
+
 // cell-major fp32 rows -> channel-first output (zeros for empty cells).
-int launch_rows_to_bev(const float *acc, int32_t dtype, int C, const int32_t *cell_start,
-                       const int32_t *cell_end, int64_t n_cells, int n_z, int64_t n_xy,
-                       int64_t out_stride_b, int64_t out_stride_c, int64_t out_stride_z, void *out,
+int launch_rows_to_bev(const float *acc, int32_t dtype, int C, const int32_t *cell_end,
+                       int64_t n_cells, int n_z, int64_t n_xy, int64_t out_stride_b,
+                       int64_t out_stride_c, int64_t out_stride_z, void *out,
                        hipStream_t s, MetaReport report = {}, bool raw16 = false) {
   if (int st = check_grid(ceil_div(n_cells, kCellTile), kThreads, "cell tiles")) return st;
   const unsigned tiles = unsigned(ceil_div(n_cells, kCellTile));
-  const int CT = C < kTileChannels ? C : kTileChannels;
+  const int CT = tile_channels(C);
   const size_t es = dtype_size(dtype);
   const size_t smem = size_t(kCellTile) * size_t(CT + 1) * sizeof(uint32_t);
   if (raw16 && es != 2) return fail(BEVPOOL_EINVAL, "internal: 16-bit rows for a 32-bit output");
   // 16-byte row pieces: 4 fp32 or 8 16-bit channels
-  const int per = raw16 ? 8 : 4;
-  const bool vrow = (C % per == 0) && (CT % per == 0) &&
-                    (reinterpret_cast<uintptr_t>(acc) % 16 == 0);
+  const bool vrow = C >= (raw16 ? 8 : 4);
   const bool vbev = bev_vec_ok(out, es, n_xy, out_stride_b, out_stride_c, out_stride_z);
   LaunchTimer t("rows_to_bev", s);
 #define BEVPOOL_R2B(T, VR, VB, R16)                                                            \
   hipLaunchKernelGGL((rows_to_bev_kernel<T, VR, VB, R16>), dim3(tiles), dim3(kThreads), smem,  \
-                     s, acc, C, CT, cell_start, cell_end, n_cells, n_z, n_xy, out_stride_b,    \
-                     out_stride_c, out_stride_z, static_cast<T::raw *>(out), report)
+                     s, acc, C, CT, cell_end, n_cells, n_z, n_xy, out_stride_b, out_stride_c,   \
+                     out_stride_z, static_cast<T::raw *>(out), report)
 #define BEVPOOL_R2B_T(T, R16)                                                                  \
   if (vrow && vbev) BEVPOOL_R2B(T, true, true, R16);                                          \
   else if (vrow) BEVPOOL_R2B(T, true, false, R16);                                            \
@@ -3708,21 +3697,20 @@ int launch_rows_to_bev(const float *acc, int32_t dtype, int C, const int32_t *ce
 
 // channel-first gradient -> cell-major rows of the occupied cells (raw bits).
 int launch_bev_to_rows(const void *grad, size_t es, int64_t gsb, int64_t gsc, int64_t gsz, int C,
-                       const int32_t *cell_start, const int32_t *cell_end, int64_t n_cells,
-                       int n_z, int64_t n_xy, void *rows, hipStream_t s) {
+                       const int32_t *cell_end, int64_t n_cells, int n_z, int64_t n_xy,
+                       void *rows, hipStream_t s) {
   if (int st = check_grid(ceil_div(n_cells, kCellTile), kThreads, "cell tiles")) return st;
   const unsigned tiles = unsigned(ceil_div(n_cells, kCellTile));
-  const int CT = C < kTileChannels ? C : kTileChannels;
+  const int CT = tile_channels(C);
   const size_t smem = size_t(kCellTile) * size_t(CT + 1) * es;
-  const bool vrow = (size_t(C) * es % 16 == 0) && (size_t(CT) * es % 16 == 0) &&
-                    (reinterpret_cast<uintptr_t>(rows) % 16 == 0);
+  const bool vrow = size_t(C) * es >= 16;
   const bool vbev = bev_vec_ok(grad, es, n_xy, gsb, gsc, gsz);
   const bool occ_first = n_cells >= kOccFirstCells;
   LaunchTimer t("bev_to_rows", s);
 #define BEVPOOL_B2R(TR, VR, VB)                                                                \
   hipLaunchKernelGGL((bev_to_rows_kernel<TR, VR, VB>), dim3(tiles), dim3(kThreads), smem, s,   \
-                     static_cast<const TR *>(grad), C, CT, cell_start, cell_end, n_cells, n_z, \
-                     n_xy, gsb, gsc, gsz, occ_first, static_cast<TR *>(rows))
+                     static_cast<const TR *>(grad), C, CT, cell_end, n_cells, n_z, n_xy, gsb,   \
+                     gsc, gsz, occ_first, static_cast<TR *>(rows))
 #define BEVPOOL_B2R_T(TR)                                                                      \
   if (vrow && vbev) BEVPOOL_B2R(TR, true, true);                                              \
   else if (vrow) BEVPOOL_B2R(TR, true, false);                                                \
@@ -4285,7 +4273,7 @@ static int forward_impl(const void *feats, int32_t dtype, int64_t feats_row_stri
     if (st) return st;
     raw16 = es == 2 && row_bytes >= 16;
   }
-  return launch_rows_to_bev(acc, dtype, C, cell_start, cell_end, n_cells, n_z, n_xy,
+  return launch_rows_to_bev(acc, dtype, C, cell_end, n_cells, n_z, n_xy,
                             out_stride_b, out_stride_c, out_stride_z, out, s, report, raw16);
 }
 
@@ -4387,7 +4375,7 @@ int bevpool_backward_planar(const float *grad, int64_t grad_stride_b, int64_t gr
                        kThreads, "gather_planar")))
     return st;
   if ((st = launch_bev_to_rows(grad, 4, grad_stride_b, grad_stride_c, grad_stride_z, C,
-                               cell_start, cell_end, n_cells, n_z, n_xy, scratch, s)))
+                               cell_end, n_cells, n_z, n_xy, scratch, s)))
     return st;
   const float *g = static_cast<const float *>(scratch);
   LaunchTimer t("gather_planar", s);
@@ -4439,7 +4427,7 @@ int bevpool_forward_depth(const float *depth, const float *context_rows, int32_t
                             n_points, keys, meta, cell_start, cell_end, acc, dr, false, s);
     if (st) return st;
   }
-  return launch_rows_to_bev(acc, BEVPOOL_F32, C, cell_start, cell_end, n_cells, n_z, n_xy,
+  return launch_rows_to_bev(acc, BEVPOOL_F32, C, cell_end, n_cells, n_z, n_xy,
                             out_stride_b, out_stride_c, out_stride_z, out, s);
 }
 
@@ -4474,7 +4462,7 @@ int bevpool_backward_depth(const float *grad, int64_t grad_stride_b, int64_t gra
   int st;
   if ((st = check_grid(ceil_div(n_pix, kDgPix) + kXcds, kThreads, "depth_grad"))) return st;
   if ((st = launch_bev_to_rows(grad, 4, grad_stride_b, grad_stride_c, grad_stride_z, C,
-                               cell_start, cell_end, n_cells, n_z, n_xy, scratch, s)))
+                               cell_end, n_cells, n_z, n_xy, scratch, s)))
     return st;
   const unsigned grid = xcd_grid(ceil_div(n_pix, kDgPix));
   LaunchTimer t("depth_grad", s);
@@ -4528,12 +4516,14 @@ int bevpool_backward(const void *grad, int32_t dtype, int64_t grad_stride_b,
   const size_t es = dtype_size(dtype);
   // gather layout (decided first: the warm-up blocks mirror it)
   const size_t row_bytes = size_t(C) * es;
-  const bool vec16 = (row_bytes % 16 == 0) && ((size_t(x_grad_row_stride) * es) % 16 == 0) &&
-                     (reinterpret_cast<uintptr_t>(x_grad) % 16 == 0) &&
-                     (reinterpret_cast<uintptr_t>(scratch) % 16 == 0);
-  const int vpr = vec16 ? int(row_bytes / 16) : int(C);
+  const int64_t ld_bytes = int64_t(size_t(x_grad_row_stride) * es);
+  const bool wide = row_bytes >= 16;  // 16-byte pieces, else elements
+  const bool aligned = row_bytes % 16 == 0 && ld_bytes % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(x_grad) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(scratch) % 16 == 0;
+  const int vpr = wide ? int((row_bytes + 15) / 16) : int(C);
   const int64_t total = n_points * vpr;
-  const int64_t gather_blocks = ceil_div(total, int64_t(kThreads) * kGatherPer);
+  const int64_t gather_blocks = ceil_div(total, int64_t(kThreads));
   int st;
   if ((st = check_grid(gather_blocks + kXcds, kThreads, "gather_rows"))) return st;
   const unsigned grid = xcd_grid(gather_blocks);
@@ -4544,40 +4534,40 @@ int bevpool_backward(const void *grad, int32_t dtype, int64_t grad_stride_b,
   if (BEVPOOL_XCD_MAP && reinterpret_cast<uintptr_t>(rank) % 16 == 0 && n_points >= 4) {
     w.rank16 = reinterpret_cast<const u32x4 *>(rank);
     w.n16 = n_points / 4;
-    w.xcd_span = int64_t(grid / kXcds) * kThreads * kGatherPer;
+    w.xcd_span = int64_t(grid / kXcds) * kThreads;
     w.vpr = vpr;
     const int64_t pts = ceil_div(w.xcd_span, int64_t(vpr)) + 1;
     w.per_xcd = int(ceil_div(ceil_div(pts, 4), int64_t(kThreads) * 16));  // <= 16 pieces/thread
     rank_blocks = kXcds * w.per_xcd;
   }
   int row_blocks = 0;
-  if (BEVPOOL_XCD_MAP && vec16) {
-    w.rows16 = static_cast<const u32x4 *>(scratch);
+  if (BEVPOOL_XCD_MAP && wide) {
+    w.rows = static_cast<const char *>(scratch);
     w.rowq = vpr;
+    w.row_bytes = int(row_bytes);
     row_blocks = int(ceil_div(n_cells, kWarmCells));
   }
   int warm_blocks = rank_blocks + row_blocks;
   warm_blocks = int(ceil_div(warm_blocks, kXcds) * kXcds);  // keep XCD parity
   if ((st = check_grid(int64_t(grid) + warm_blocks, kThreads, "gather_rows"))) return st;
   if ((st = launch_bev_to_rows(grad, es, grad_stride_b, grad_stride_c, grad_stride_z, C,
-                               cell_start, cell_end, n_cells, n_z, n_xy, scratch, s)))
+                               cell_end, n_cells, n_z, n_xy, scratch, s)))
     return st;
   LaunchTimer t("gather_rows", s);
-#define BEVPOOL_GATHER(V, NARROW, LD)                                                          \
-  hipLaunchKernelGGL((gather_rows_kernel<V, NARROW>), dim3(grid + unsigned(warm_blocks)),      \
-                     dim3(kThreads), 0, s, static_cast<const V *>(scratch), vpr, rank,        \
-                     n_points, static_cast<V *>(x_grad), LD, warm_blocks, w, cell_start,     \
-                     cell_end, n_cells, 0, zero_dropped ? 1 : 0)
-  if (vec16) {
-    const int64_t ld = int64_t(size_t(x_grad_row_stride) * es / 16);
-    if (narrow) BEVPOOL_GATHER(u32x4, true, ld); else BEVPOOL_GATHER(u32x4, false, ld);
-  } else if (es == 4) {
-    if (narrow) BEVPOOL_GATHER(uint32_t, true, x_grad_row_stride);
-    else BEVPOOL_GATHER(uint32_t, false, x_grad_row_stride);
-  } else {
-    if (narrow) BEVPOOL_GATHER(uint16_t, true, x_grad_row_stride);
-    else BEVPOOL_GATHER(uint16_t, false, x_grad_row_stride);
+#define BEVPOOL_GATHER(V, NARROW, ANY)                                                         \
+  hipLaunchKernelGGL((gather_rows_kernel<V, NARROW, ANY>), dim3(grid + unsigned(warm_blocks)), \
+                     dim3(kThreads), 0, s, static_cast<const char *>(scratch), vpr,            \
+                     int(row_bytes), rank, n_points, static_cast<char *>(x_grad), ld_bytes,    \
+                     warm_blocks, w, cell_start, cell_end, n_cells, 0, zero_dropped ? 1 : 0)
+#define BEVPOOL_GATHER_V(V, ANY)                                                               \
+  {                                                                                            \
+    if (narrow) BEVPOOL_GATHER(V, true, ANY); else BEVPOOL_GATHER(V, false, ANY);             \
   }
+  if (wide && aligned) BEVPOOL_GATHER_V(u32x4, false)
+  else if (wide) BEVPOOL_GATHER_V(u32x4, true)
+  else if (es == 4) BEVPOOL_GATHER_V(uint32_t, false)
+  else BEVPOOL_GATHER_V(uint16_t, false)
+#undef BEVPOOL_GATHER_V
 #undef BEVPOOL_GATHER
   return check_launch("gather_rows");
 }

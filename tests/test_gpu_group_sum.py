@@ -69,3 +69,32 @@ def test_depth_rows(pkg, cuda, C):
     module = pkg.BevPoolTransform(case.xbound, case.ybound, case.zbound).to(cuda)
     out = module.bev_pool_depth(case.geom.to(cuda), depth.to(cuda), context.to(cuda))
     assert_bit_equal(out, ref.lss_bev_pool_depth(case.geom, depth, context, dx, bx, nx), 'forward')
+
+
+ROWS = [(3, F32), (4, F32), (5, F32), (7, F16), (8, F16), (9, BF16), (90, F16), (129, F32),
+        (130, F32), (257, BF16)]
+
+
+@pytest.mark.parametrize('grid,C,dtype', [
+    (grid, C, dtype) for grid in [(2, 3, 5, 7), (1, 1, 1, 1), (1, 2, 9, 15), (2, 1, 331, 333)]
+    for C, dtype in ROWS if grid[2] < 100 or C <= 90])
+def test_odd_planes(pkg, cuda, grid, C, dtype):
+    """Planes that no vector width divides (4 cells that straddle two planes or
+    the grid's end; from 200,000 cells the occupancy is read first), rows that
+    none divides, and a gradient whose planes start at any element."""
+    B, D, H, W = grid
+    g = torch.Generator().manual_seed(C)
+    N = 4001
+    coords = torch.stack([torch.randint(0, n, (N,), generator=g) for n in (H, W, D, B)], 1)
+    feats = torch.randn((N, C), generator=g).to(dtype)
+    up = torch.randn((B, C + 1, D, H * W + 3), generator=g).to(dtype)[:, 1:, :, 2:2 + H * W]
+    up = up.unflatten(3, (H, W))
+    f = feats.to(cuda).requires_grad_(True)
+    out = pkg.bev_pool(f, coords.to(cuda), B, D, H, W)
+    store = torch.empty((B, C + 1, D, H * W + 3), dtype=dtype, device=cuda)
+    view = store[:, 1:, :, 2:2 + H * W].unflatten(3, (H, W))
+    view.copy_(up)
+    grad, = torch.autograd.grad(out, f, view)
+    assert_bit_equal(out, ref.bev_pool(feats.float(), coords, B, D, H, W).to(dtype), 'forward')
+    x, y, z, b = coords.unbind(1)
+    assert_bit_equal(grad, up[b, :, z, x, y], 'backward')
