@@ -1665,7 +1665,9 @@ static_assert(kStageRows == 32, "only 32-row accumulation stages are supported")
 //   kRowsDepth   depth-weighted context rows (DepthRows), ordinary loads:
 //                a context row is read for every depth bin
 //                (accum_group_kernel only).
-constexpr int kRowsPlain = 0, kRowsDepth = 1, kRowsStream = 2;
+//   kRowsRun     consecutive rows: position p of a cell is row p
+//                (legacy_sum_kernel only).
+constexpr int kRowsPlain = 0, kRowsDepth = 1, kRowsStream = 2, kRowsRun = 3;
 constexpr int64_t kStreamRowBytes = int64_t(1) << 30;
 
 struct PipeRange {
@@ -2155,7 +2157,8 @@ __device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
       const int p = base + 16 * t + slot;
-      idx[t] = kw[2 * int64_t(p < b1 ? p : b1 - 1)];
+      const int pc = p < b1 ? p : b1 - 1;
+      idx[t] = kRows == kRowsRun ? uint32_t(pc) : kw[2 * int64_t(pc)];
     }
   };
   auto rows = [&]() {
@@ -2842,11 +2845,13 @@ __global__ __launch_bounds__(kThreads) void gather_rows_kernel(
 // ---------------------------------------------------------------------------
 
 // Zero bytes [0, n16 * 16) as 16-byte vectors plus a 4-byte tail (n4 words
-// from `tail`), grid-stride.  A kernel rather than a memset so that a graph
-// capture records no memset node.
+// from `tail`), grid-stride; with `when`, only if *when != 0.  A kernel
+// rather than a memset so that a graph capture records no memset node.
 __global__ __launch_bounds__(kThreads) void zero_fill_kernel(u32x4 *__restrict__ p, int64_t n16,
                                                              uint32_t *__restrict__ tail,
-                                                             int64_t n4) {
+                                                             int64_t n4,
+                                                             const int32_t *__restrict__ when) {
+  if (when && *when == 0) return;
   const int64_t stride = int64_t(gridDim.x) * kThreads;
   for (int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x; i < n16; i += stride)
     p[i] = u32x4{0u, 0u, 0u, 0u};
@@ -2877,18 +2882,124 @@ __device__ __forceinline__ int64_t legacy_count(int64_t cap, const int32_t *__re
 
 // ops/bev_pool/csrc/bev_pool_cuda.cu:20-42: interval j sums rows [s, s + len)
 // of x (n, C) -- fp32 from +0.0, rows in order -- and stores the sum to
-// out[cell, :] (channels last).  One wave per interval; lane l owns channels
-// c0 + l + 64 i, so each row is read as one coalesced run; rows are loaded
-// kLegacyBatch at a time before they are added.  Invalid intervals are
-// skipped and counted in meta[BEVPOOL_META_N_BAD] (meta may be null).
-constexpr int kLegacyBatch = 8;
+// out[cell, :] (channels last).  Invalid intervals are skipped and counted in
+// meta[BEVPOOL_META_N_BAD] (meta may be null).
+//
+// Rows of 4 channels or more are cut into 16-byte pieces (the last one ends
+// at the row's end), a wave into 64 / q groups of q lanes, one interval per
+// group, 8 rows in flight while 8 are added.  Intervals of kLegacyLong rows or
+// more are left to the block's waves together afterwards, one per 64 bytes of
+// the row (sum_long_cell), so that no chain of loads outlasts the rest.
+// Neighbouring intervals go to different blocks: the long ones, the cells
+// near the cameras, are neighbours.  The rows are read once, so HBM bounds it:
+// 1.54 M rows of 80 channels (494 MB) in 39 K intervals 118 us, against 230 with
+// one wave per interval and 4 bytes per lane.
+constexpr int kLegacyLong = 256;
+// Blocks of a legacy launch; more intervals loop (2048 and 16384 blocks: forward
+// 129 and 133 us, backward 110 and 108).
+constexpr int kLegacyBlocks = 4096;
 
-template <int kCPL>
-__global__ __launch_bounds__(kThreads) void legacy_forward_kernel(
+__global__ __launch_bounds__(kThreads) void legacy_sum_kernel(
+    const char *__restrict__ x, int64_t n, int C, int qmax, const int32_t *__restrict__ geom,
+    const int32_t *__restrict__ starts, const int32_t *__restrict__ lengths, int64_t cap,
+    const int32_t *__restrict__ count_dev, int nb, int nd, int nh, int nw,
+    char *__restrict__ out, int32_t *__restrict__ meta) {
+  constexpr int kU = 8;
+  __shared__ u32x4 s_tile[kWaves][64];
+  __shared__ int s_long[kThreads], s_n;  // this pass's long intervals
+  const int64_t n_int = legacy_count(cap, count_dev);
+  const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int row_bytes = C * 4;
+  const int q0 = int(blockIdx.y) * qmax, qt = (row_bytes + 15) >> 4;
+  const int q = qt - q0 < qmax ? qt - q0 : qmax;
+  const int ng = 64 / q;
+  const bool own = lane / q < ng;  // lanes past the last group repeat its last piece
+  const int g = own ? lane / q : ng - 1;
+  const int li = lane - g * q < q ? lane - g * q : q - 1;
+  const int pb = 16 * (q0 + li) < row_bytes - 16 ? 16 * (q0 + li) : row_bytes - 16;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  const int64_t per_pass = int64_t(kWaves) * ng * gridDim.x;
+  for (int64_t j0 = 0; j0 < n_int; j0 += per_pass) {
+    const int64_t j = j0 + int64_t(wave * ng + g) * gridDim.x + blockIdx.x;
+    int64_t s = 0, cell = -1;
+    int len = 0;
+    if (j < n_int) {
+      s = starts[j];
+      len = lengths[j];
+      cell = legacy_cell(geom, n, s, len, nb, nd, nh, nw);
+    }
+    const bool lead = own && li == 0 && j < n_int;
+    if (cell < 0) {
+      if (meta && lead && blockIdx.y == 0) atomicAdd(meta + BEVPOOL_META_N_BAD, 1);
+      s = len = 0;
+    } else if (len >= kLegacyLong) {
+      if (lead) s_long[atomicAdd(&s_n, 1)] = int(j);
+      s = len = 0;
+      cell = -1;
+    }
+    int most = len;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_xor(most, o, 64);
+      most = most > y ? most : y;
+    }
+    most = __builtin_amdgcn_readfirstlane(most);
+    PieceSum<F32> sum;
+    sum.clear();
+    if (most > 0) {
+      const char *xp = x + s * row_bytes + pb;
+      u32x4 a[kU], b[kU];
+      auto load = [&](u32x4(&v)[kU], int i0) {  // past the interval: its last row
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          const int r = i0 + u < len ? i0 + u : (len > 0 ? len - 1 : 0);
+          v[u] = reinterpret_cast<const Bytes16 *>(xp + int64_t(r) * row_bytes)->v;
+        }
+      };
+      // rows past the interval add +0.0, which changes no sum that started
+      // at +0.0 (it is never -0.0)
+      auto add = [&](const u32x4(&v)[kU], int i0) {
+#pragma unroll
+        for (int u = 0; u < kU; ++u)
+          sum.add<false>(i0 + u < len ? v[u] : u32x4{0u, 0u, 0u, 0u}, 0.0f);
+      };
+      load(a, 0);
+      for (int i = 0; i < most; i += 2 * kU) {
+        load(b, i + kU);
+        add(a, i);
+        load(a, i + 2 * kU);
+        add(b, i + kU);
+      }
+    }
+    if (cell >= 0 && own)
+      reinterpret_cast<Bytes16 *>(out + cell * row_bytes + pb)->v = sum.bits();
+    __syncthreads();
+    const int slices = (q + 3) >> 2, tasks = s_n * slices;
+    for (int t = wave; t < tasks; t += kWaves) {
+      const int64_t jl = s_long[t / slices];
+      const int64_t sl = starts[jl];
+      const int ll = lengths[jl];
+      const int64_t cl = legacy_cell(geom, n, sl, ll, nb, nd, nh, nw);
+      const int b0 = __builtin_amdgcn_readfirstlane(int(sl));
+      const int b1 = b0 + __builtin_amdgcn_readfirstlane(ll);
+      sum_long_cell<F32, kRowsRun>(x, row_bytes, row_bytes, q0 + 4 * (t % slices), q0 + q, nullptr,
+                                   b0, b1, out + cl * row_bytes, s_tile[wave], DepthRows{});
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) s_n = 0;
+    __syncthreads();
+  }
+}
+
+// The same for rows of fewer than 4 channels: one wave per interval, lane l
+// owns channel l, 8 rows at a time.
+__global__ __launch_bounds__(kThreads) void legacy_sum_narrow_kernel(
     const float *__restrict__ x, int64_t n, int C, const int32_t *__restrict__ geom,
     const int32_t *__restrict__ starts, const int32_t *__restrict__ lengths, int64_t cap,
     const int32_t *__restrict__ count_dev, int nb, int nd, int nh, int nw,
     float *__restrict__ out, int32_t *__restrict__ meta) {
+  constexpr int kU = 8;
   const int64_t n_int = legacy_count(cap, count_dev);
   const int lane = lane_id();
   const int64_t nwaves = (int64_t(gridDim.x) * kThreads) >> 6;
@@ -2899,82 +3010,138 @@ __global__ __launch_bounds__(kThreads) void legacy_forward_kernel(
       if (meta && lane == 0) atomicAdd(meta + BEVPOOL_META_N_BAD, 1);
       continue;
     }
-    for (int c0 = 0; c0 < C; c0 += 64 * kCPL) {
-      int col[kCPL];
-      float acc[kCPL];
+    const int col = lane < C ? lane : C - 1;  // lanes past C store nothing
+    float acc = 0.0f;
+    for (int64_t r0 = 0; r0 < len; r0 += kU) {
+      float v[kU];
 #pragma unroll
-      for (int i = 0; i < kCPL; ++i) {
-        const int c = c0 + lane + 64 * i;
-        col[i] = c < C ? c : C - 1;  // lanes past C read a valid column, store nothing
-        acc[i] = 0.0f;
-      }
-      for (int64_t r0 = 0; r0 < len; r0 += kLegacyBatch) {
-        float v[kLegacyBatch][kCPL];
+      for (int u = 0; u < kU; ++u) v[u] = x[(s + (r0 + u < len ? r0 + u : 0)) * C + col];
 #pragma unroll
-        for (int u = 0; u < kLegacyBatch; ++u) {
-          const int64_t r = s + (r0 + u < len ? r0 + u : 0);
-#pragma unroll
-          for (int i = 0; i < kCPL; ++i) v[u][i] = x[r * C + col[i]];
-        }
-#pragma unroll
-        for (int u = 0; u < kLegacyBatch; ++u)
-          if (r0 + u < len)
-#pragma unroll
-            for (int i = 0; i < kCPL; ++i) acc[i] += v[u][i];
-      }
-#pragma unroll
-      for (int i = 0; i < kCPL; ++i)
-        if (c0 + lane + 64 * i < C) out[cell * C + c0 + lane + 64 * i] = acc[i];
+      for (int u = 0; u < kU; ++u)
+        if (r0 + u < len) acc += v[u];
     }
+    if (lane < C) out[cell * C + lane] = acc;
   }
+}
+
+// Sets *unordered unless the intervals lie within the n rows, in order and
+// without overlap, and there is at least one.  Then legacy_spread_kernel
+// writes every row itself (rows between the intervals as zeros) and the
+// gradient needs no zero fill before it.
+__global__ __launch_bounds__(kThreads) void legacy_order_kernel(
+    const int32_t *__restrict__ starts, const int32_t *__restrict__ lengths, int64_t cap,
+    const int32_t *__restrict__ count_dev, int64_t n, int32_t *__restrict__ unordered) {
+  const int64_t n_int = legacy_count(cap, count_dev);
+  if (n_int == 0 && blockIdx.x == 0 && threadIdx.x == 0) *unordered = 1;
+  bool bad = false;
+  for (int64_t j = int64_t(blockIdx.x) * kThreads + threadIdx.x; j < n_int;
+       j += int64_t(gridDim.x) * kThreads) {
+    const int64_t s = starts[j], len = lengths[j];
+    const int64_t next = j + 1 < n_int ? int64_t(starts[j + 1]) : n;
+    bad |= s < 0 || len < 0 || s + len > next;
+  }
+  if (bad) *unordered = 1;  // every writer writes the same
 }
 
 // ops/bev_pool/csrc/bev_pool_cuda.cu:61-84: every row of interval j gets the
 // gradient row of its cell, x_grad[r, :] = g[cell, :] (g channels last).  One
-// wave per interval, lanes over channels as in the forward.
-template <int kCPL>
-__global__ __launch_bounds__(kThreads) void legacy_backward_kernel(
-    const float *__restrict__ g, int64_t n, int C, const int32_t *__restrict__ geom,
+// wave per interval; V (16-byte pieces at element alignment, or elements for
+// rows of fewer than 4 channels) of ng rows per store, non-temporal.
+// unordered: null or *unordered != 0: x_grad is zero already and invalid
+// intervals are skipped; else the wave also writes its interval's gap up to
+// the next one (and up to the first one) as zeros, and an invalid cell's rows.
+// The write stream bounds it: 1.54 M rows of 80 channels (494 MB) in 104 us
+// (and 6 + 3 for the order check and the skipped fill), against 78 us of zero
+// fill and 154 us with 4 bytes per lane.  Temporal stores took 94 us and the
+// forward that follows 36 us more.
+template <bool kWide>
+__global__ __launch_bounds__(kThreads) void legacy_spread_kernel(
+    const char *__restrict__ g, int64_t n, int C, int qmax, const int32_t *__restrict__ geom,
     const int32_t *__restrict__ starts, const int32_t *__restrict__ lengths, int64_t cap,
     const int32_t *__restrict__ count_dev, int nb, int nd, int nh, int nw,
-    float *__restrict__ xg, int32_t *__restrict__ meta) {
+    char *__restrict__ xg, int32_t *__restrict__ meta, const int32_t *__restrict__ unordered) {
+  constexpr int kV = kWide ? 16 : 4;
   const int64_t n_int = legacy_count(cap, count_dev);
-  const int lane = lane_id();
-  const int64_t nwaves = (int64_t(gridDim.x) * kThreads) >> 6;
-  for (int64_t j = (int64_t(blockIdx.x) * kThreads + threadIdx.x) >> 6; j < n_int; j += nwaves) {
+  const bool ordered = unordered && *unordered == 0;
+  const int lane = lane_id(), wave = int(threadIdx.x) >> 6;
+  const int row_bytes = C * 4;
+  const int q0 = int(blockIdx.y) * qmax, qt = (row_bytes + kV - 1) / kV;
+  const int q = qt - q0 < qmax ? qt - q0 : qmax;
+  const int ng = 64 / q, gi = lane / q, li = lane - gi * q;
+  const int pb = kV * (q0 + li) < row_bytes - kV ? kV * (q0 + li) : row_bytes - kV;
+  const int64_t stride = int64_t(gridDim.x) * kWaves;
+  for (int64_t j = int64_t(blockIdx.x) * kWaves + wave; j < n_int; j += stride) {
     const int64_t s = starts[j], len = lengths[j];
     const int64_t cell = legacy_cell(geom, n, s, len, nb, nd, nh, nw);
     if (cell < 0) {
-      if (meta && lane == 0) atomicAdd(meta + BEVPOOL_META_N_BAD, 1);
-      continue;
+      if (meta && lane == 0 && blockIdx.y == 0) atomicAdd(meta + BEVPOOL_META_N_BAD, 1);
+      if (!ordered) continue;
     }
-    for (int c0 = 0; c0 < C; c0 += 64 * kCPL) {
-      float v[kCPL];
-#pragma unroll
-      for (int i = 0; i < kCPL; ++i) {
-        const int c = c0 + lane + 64 * i;
-        v[i] = g[cell * C + (c < C ? c : C - 1)];
+    u32x4 v = u32x4{0u, 0u, 0u, 0u};
+    if (cell >= 0) {
+      if constexpr (kWide)
+        v = reinterpret_cast<const Bytes16 *>(g + cell * row_bytes + pb)->v;
+      else
+        v.x = *reinterpret_cast<const uint32_t *>(g + cell * row_bytes + pb);
+    }
+    auto fill = [&](int64_t a, int64_t b, u32x4 w) {
+      for (int64_t r = a + gi; r < b; r += ng) {
+        char *dst = xg + r * row_bytes + pb;
+        if constexpr (kWide)
+          __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any *>(dst));
+        else
+          __builtin_nontemporal_store(uint32_t(w.x), reinterpret_cast<uint32_t *>(dst));
       }
-      for (int64_t r = s; r < s + len; ++r)
-#pragma unroll
-        for (int i = 0; i < kCPL; ++i)
-          if (c0 + lane + 64 * i < C) xg[r * C + c0 + lane + 64 * i] = v[i];
+    };
+    if (gi < ng) {
+      if (ordered && j == 0) fill(0, s, u32x4{0u, 0u, 0u, 0u});
+      fill(s, s + len, v);
+      if (ordered)
+        fill(s + len, j + 1 < n_int ? int64_t(starts[j + 1]) : n, u32x4{0u, 0u, 0u, 0u});
     }
   }
 }
 
 // Run boundaries of a rank array (ops/bev_pool/bev_pool_legacy.py:56-61:
-// flag[0] = 1, flag[i] = rank[i] != rank[i-1]).  Per block of 256 positions:
-// the number of run starts.
+// flag[0] = 1, flag[i] = rank[i] != rank[i-1]).  A block takes kRunTile
+// consecutive positions, a wave kRunIt batches of 64 of them in order.
+constexpr int kRunIt = 4;
+constexpr int kRunTile = kThreads * kRunIt;
+
+// The start flags of this wave's batches, as one mask per batch.
+template <typename TR>
+__device__ __forceinline__ void run_flags(const TR *__restrict__ ranks, int64_t n, int64_t base,
+                                          uint64_t (&flags)[kRunIt]) {
+  TR r[kRunIt], before[kRunIt];
+#pragma unroll
+  for (int k = 0; k < kRunIt; ++k) {  // all loads first
+    const int64_t i = base + 64 * k + lane_id(), c = i < n ? i : n - 1;
+    r[k] = ranks[c];
+    before[k] = ranks[c > 0 ? c - 1 : 0];
+  }
+#pragma unroll
+  for (int k = 0; k < kRunIt; ++k) {
+    const int64_t i = base + 64 * k + lane_id();
+    flags[k] = __ballot(i < n && (i == 0 || r[k] != before[k]));
+  }
+}
+
+// Per block: the number of run starts.  Block 0 also resets meta.
 template <typename TR>
 __global__ __launch_bounds__(kThreads) void run_count_kernel(const TR *__restrict__ ranks,
                                                              int64_t n,
-                                                             int32_t *__restrict__ bcount) {
+                                                             int32_t *__restrict__ bcount,
+                                                             int32_t *__restrict__ meta) {
   __shared__ int s_w[kWaves];
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-  const bool is_start = i < n && (i == 0 || ranks[i] != ranks[i - 1]);
-  const uint64_t b = __ballot(is_start);
-  if (lane_id() == 0) s_w[threadIdx.x >> 6] = __popcll(b);
+  if (blockIdx.x == 0 && threadIdx.x < BEVPOOL_META_LEN)
+    meta[threadIdx.x] = threadIdx.x == BEVPOOL_META_FIRST_BAD ? 0x7fffffff : 0;
+  const int w = threadIdx.x >> 6;
+  uint64_t flags[kRunIt];
+  run_flags(ranks, n, int64_t(blockIdx.x) * kRunTile + int64_t(w) * 64 * kRunIt, flags);
+  int c = 0;
+#pragma unroll
+  for (int k = 0; k < kRunIt; ++k) c += __popcll(flags[k]);
+  if (lane_id() == 0) s_w[w] = c;
   __syncthreads();
   if (threadIdx.x == 0) {
     int s = 0;
@@ -2990,16 +3157,22 @@ __global__ __launch_bounds__(kThreads) void run_write_kernel(const TR *__restric
                                                              const int32_t *__restrict__ boff,
                                                              int32_t *__restrict__ starts) {
   __shared__ int s_w[kWaves];
-  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
   const int w = threadIdx.x >> 6;
-  const bool is_start = i < n && (i == 0 || ranks[i] != ranks[i - 1]);
-  const uint64_t b = __ballot(is_start);
-  if (lane_id() == 0) s_w[w] = __popcll(b);
+  const int64_t base = int64_t(blockIdx.x) * kRunTile + int64_t(w) * 64 * kRunIt;
+  uint64_t flags[kRunIt];
+  run_flags(ranks, n, base, flags);
+  int c = 0;
+#pragma unroll
+  for (int k = 0; k < kRunIt; ++k) c += __popcll(flags[k]);
+  if (lane_id() == 0) s_w[w] = c;
   __syncthreads();
-  if (is_start) {
-    int off = boff[blockIdx.x] + __popcll(b & lanes_below());
-    for (int j = 0; j < w; ++j) off += s_w[j];
-    starts[off] = int(i);
+  int off = boff[blockIdx.x];
+  for (int j = 0; j < w; ++j) off += s_w[j];
+#pragma unroll
+  for (int k = 0; k < kRunIt; ++k) {
+    if ((flags[k] >> lane_id()) & 1)
+      starts[off + __popcll(flags[k] & lanes_below())] = int(base + 64 * k + lane_id());
+    off += __popcll(flags[k]);
   }
 }
 
@@ -3727,8 +3900,8 @@ int launch_bev_to_rows(const void *grad, size_t es, int64_t gsb, int64_t gsc, in
 }
 
 // Zero `bytes` bytes at p (4-byte aligned, a multiple of 4 bytes) with
-// zero_fill_kernel.
-int launch_zero_fill(void *p, size_t bytes, hipStream_t s) {
+// zero_fill_kernel; with `when` (device memory), only if *when != 0.
+int launch_zero_fill(void *p, size_t bytes, hipStream_t s, const int32_t *when = nullptr) {
   if (bytes == 0) return BEVPOOL_OK;
   const bool vec = reinterpret_cast<uintptr_t>(p) % 16 == 0;
   const int64_t n16 = vec ? int64_t(bytes / 16) : 0;
@@ -3738,17 +3911,23 @@ int launch_zero_fill(void *p, size_t bytes, hipStream_t s) {
   LaunchTimer t("zero_fill", s);
   hipLaunchKernelGGL(zero_fill_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, s,
                      static_cast<u32x4 *>(p), n16,
-                     reinterpret_cast<uint32_t *>(static_cast<char *>(p) + n16 * 16), n4);
+                     reinterpret_cast<uint32_t *>(static_cast<char *>(p) + n16 * 16), n4, when);
   return check_launch("zero_fill");
 }
 
-// Channels per lane of the legacy kernels: 1 (C <= 64), 2 (<= 128), else 4
-// (with a loop over 256-channel blocks).
-int legacy_cpl(int C) { return C <= 64 ? 1 : (C <= 128 ? 2 : 4); }
-
-unsigned legacy_grid(int64_t cap) {
-  const int64_t b = ceil_div(cap, kWaves);
-  return unsigned(b < 1 ? 1 : (b > 65536 ? 65536 : b));
+// Launch shape of the legacy kernels for rows cut into pieces of `piece`
+// bytes: at most 64 pieces per channel block (grid.y), `per_wave` intervals
+// per wave of at most kLegacyBlocks blocks (grid.x; more intervals loop).
+struct LegacyShape {
+  int qmax;
+  dim3 grid;
+};
+LegacyShape legacy_shape(int C, int piece, int64_t cap, bool groups) {
+  const int qt = (C * 4 + piece - 1) / piece, nblk = (qt + 63) / 64;
+  const int qmax = (qt + nblk - 1) / nblk;
+  const int64_t blocks = ceil_div(cap, int64_t(kWaves) * (groups ? 64 / qmax : 1));
+  return {qmax, dim3(unsigned(blocks < 1 ? 1 : (blocks < kLegacyBlocks ? blocks : kLegacyBlocks)),
+                     unsigned(nblk))};
 }
 
 int check_legacy_args(int64_t n, int32_t C, const void *geom, const void *starts,
@@ -3817,6 +3996,9 @@ OpScratchLayout op_scratch_layout(int64_t n, int64_t cells, int32_t C) {
 // current device, cached per device by noalloc_scratch().
 constexpr size_t kNoAllocScratchBytes = BEVPOOL_NOALLOC_MAX_BYTES;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+
+// legacy backward: the counter slot that holds its order check
+constexpr int kMetaUnordered = 4;
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -4587,16 +4769,17 @@ int bevpool_legacy_forward(const float *x, int64_t n, int32_t C, const int32_t *
   if ((st = launch_zero_fill(out, size_t(cells) * size_t(C) * sizeof(float), s))) return st;
   if (n_intervals == 0) return BEVPOOL_OK;
   LaunchTimer t("legacy_forward", s);
-#define BEVPOOL_LF(K)                                                                          \
-  hipLaunchKernelGGL((legacy_forward_kernel<K>), dim3(legacy_grid(n_intervals)), dim3(kThreads), \
-                     0, s, x, n, C, geom_feats, interval_starts, interval_lengths, n_intervals,  \
-                     n_intervals_dev, b, d, h, w, out, meta)
-  switch (legacy_cpl(C)) {
-    case 1: BEVPOOL_LF(1); break;
-    case 2: BEVPOOL_LF(2); break;
-    default: BEVPOOL_LF(4); break;
+  if (C >= 4) {
+    const LegacyShape L = legacy_shape(C, 16, n_intervals, true);
+    hipLaunchKernelGGL(legacy_sum_kernel, L.grid, dim3(kThreads), 0, s,
+                       reinterpret_cast<const char *>(x), n, C, L.qmax, geom_feats,
+                       interval_starts, interval_lengths, n_intervals, n_intervals_dev, b, d, h,
+                       w, reinterpret_cast<char *>(out), meta);
+  } else {
+    hipLaunchKernelGGL(legacy_sum_narrow_kernel, legacy_shape(C, 4, n_intervals, false).grid,
+                       dim3(kThreads), 0, s, x, n, C, geom_feats, interval_starts,
+                       interval_lengths, n_intervals, n_intervals_dev, b, d, h, w, out, meta);
   }
-#undef BEVPOOL_LF
   return check_launch("legacy_forward");
 }
 
@@ -4611,19 +4794,31 @@ int bevpool_legacy_backward(const float *out_grad, int64_t n, int32_t C,
   if (st) return st;
   if (n_intervals > 0 && !out_grad) return fail(BEVPOOL_EINVAL, "null out_grad");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if ((st = launch_zero_fill(x_grad, size_t(n) * size_t(C) * sizeof(float), s))) return st;
+  // Intervals in order and without overlap, the usual case, write every row
+  // themselves: the device decides (meta[4] holds the answer during the call;
+  // a caller's leftover there only costs the fill).
+  int32_t *unordered = nullptr;
+  if (meta && n_intervals > 0 && n > 0) {
+    unordered = meta + kMetaUnordered;
+    LaunchTimer t("legacy_order", s);
+    const int64_t blocks = ceil_div(n_intervals, int64_t(kThreads));
+    hipLaunchKernelGGL(legacy_order_kernel, dim3(unsigned(blocks < 512 ? blocks : 512)),
+                       dim3(kThreads), 0, s, interval_starts, interval_lengths, n_intervals,
+                       n_intervals_dev, n, unordered);
+    if ((st = check_launch("legacy_order"))) return st;
+  }
+  if ((st = launch_zero_fill(x_grad, size_t(n) * size_t(C) * sizeof(float), s, unordered)))
+    return st;
   if (n_intervals == 0 || n == 0) return BEVPOOL_OK;
   LaunchTimer t("legacy_backward", s);
-#define BEVPOOL_LB(K)                                                                          \
-  hipLaunchKernelGGL((legacy_backward_kernel<K>), dim3(legacy_grid(n_intervals)),              \
-                     dim3(kThreads), 0, s, out_grad, n, C, geom_feats, interval_starts,        \
-                     interval_lengths, n_intervals, n_intervals_dev, b, d, h, w, x_grad, meta)
-  switch (legacy_cpl(C)) {
-    case 1: BEVPOOL_LB(1); break;
-    case 2: BEVPOOL_LB(2); break;
-    default: BEVPOOL_LB(4); break;
-  }
-#undef BEVPOOL_LB
+  const LegacyShape L = legacy_shape(C, C >= 4 ? 16 : 4, n_intervals, false);
+#define BEVPOOL_LS(WIDE)                                                                       \
+  hipLaunchKernelGGL(legacy_spread_kernel<WIDE>, L.grid, dim3(kThreads), 0, s,                 \
+                     reinterpret_cast<const char *>(out_grad), n, C, L.qmax, geom_feats,        \
+                     interval_starts, interval_lengths, n_intervals, n_intervals_dev, b, d, h, \
+                     w, reinterpret_cast<char *>(x_grad), meta, unordered)
+  if (C >= 4) BEVPOOL_LS(true); else BEVPOOL_LS(false);
+#undef BEVPOOL_LS
   return check_launch("legacy_backward");
 }
 
@@ -4647,23 +4842,22 @@ int bevpool_runs(const void *ranks, int32_t rank_bytes, int64_t n, int32_t *star
     return fail(BEVPOOL_EINVAL, "null ranks / starts / lengths");
   hipStream_t s = static_cast<hipStream_t>(stream);
   int st;
-  {
+  if (n == 0) {
     LaunchTimer t("init_meta", s);
     hipLaunchKernelGGL(init_meta_kernel, dim3(1), dim3(64), 0, s, meta);
-    if ((st = check_launch("init_meta"))) return st;
+    return check_launch("init_meta");
   }
-  if (n == 0) return BEVPOOL_OK;
-  const int64_t blocks = ceil_div(n, kThreads);
-  if ((st = check_grid(blocks, kThreads, "runs"))) return st;
+  const int64_t blocks = ceil_div(n, int64_t(kRunTile));
+  if ((st = check_grid(ceil_div(n, kThreads), kThreads, "runs"))) return st;
   int32_t *bcount = static_cast<int32_t *>(workspace);
   {
     LaunchTimer t("run_count", s);
     if (rank_bytes == 4)
       hipLaunchKernelGGL(run_count_kernel<int32_t>, dim3(unsigned(blocks)), dim3(kThreads), 0, s,
-                         static_cast<const int32_t *>(ranks), n, bcount);
+                         static_cast<const int32_t *>(ranks), n, bcount, meta);
     else
       hipLaunchKernelGGL(run_count_kernel<int64_t>, dim3(unsigned(blocks)), dim3(kThreads), 0, s,
-                         static_cast<const int64_t *>(ranks), n, bcount);
+                         static_cast<const int64_t *>(ranks), n, bcount, meta);
     if ((st = check_launch("run_count"))) return st;
   }
   {
@@ -4683,8 +4877,8 @@ int bevpool_runs(const void *ranks, int32_t rank_bytes, int64_t n, int32_t *star
     if ((st = check_launch("run_write"))) return st;
   }
   LaunchTimer t("run_length", s);
-  hipLaunchKernelGGL(run_length_kernel, dim3(unsigned(blocks)), dim3(kThreads), 0, s, starts, n,
-                     meta + BEVPOOL_META_N_INTERVALS, lengths);
+  hipLaunchKernelGGL(run_length_kernel, dim3(unsigned(ceil_div(n, kThreads))), dim3(kThreads), 0,
+                     s, starts, n, meta + BEVPOOL_META_N_INTERVALS, lengths);
   return check_launch("run_length");
 }
 

@@ -186,3 +186,45 @@ def test_runs_entry(pkg, cuda):
             es, el = ref.runs(r)
             assert m == es.numel()
             assert torch.equal(starts[:m].cpu(), es) and torch.equal(lengths[:m].cpu(), el)
+
+
+@pytest.mark.parametrize('order', ['rows', 'reversed', 'gaps', 'invalid'])
+@pytest.mark.parametrize('C', [1, 3, 4, 7, 64, 256, 260])
+def test_ext_module_interval_lengths(pkg, cuda, C, order):
+    """Intervals around the rows in flight and the long intervals' limit, more
+    of them than one pass of the grid takes at C = 256, in row order (the
+    backward writes every row itself, gaps and skipped intervals as zeros) and
+    in reversed order (it fills with zeros first)."""
+    g = torch.Generator().manual_seed(C)
+    lengths = torch.tensor([1, 7, 8, 9, 15, 16, 17, 255, 256, 257, 0, 1000, 300, 1]
+                           + [1] * (17000 if C == 256 else 500), dtype=torch.int32)
+    gaps = torch.randint(0, 3, lengths.shape, generator=g).int() * (order == 'gaps')
+    ends = (lengths + gaps).cumsum(0).int()
+    starts, n = ends - lengths, int(ends[-1]) + 5
+    H, W = 160, 128
+    cell = torch.randperm(H * W, generator=g)[:n + lengths.numel()]
+    coords = torch.zeros((n, 4), dtype=torch.int32)
+    coords[starts.long(), 0] = (cell[:starts.numel()] // W).int()
+    coords[starts.long(), 1] = (cell[:starts.numel()] % W).int()
+    if order == 'reversed':
+        starts, lengths = starts.flip(0).contiguous(), lengths.flip(0).contiguous()
+    if order == 'invalid':
+        coords[int(starts[7]), 0] = H  # a cell outside the grid
+    keep = lengths > 0  # an empty interval shares its first row, and cell, with the next one
+    starts, lengths = starts[keep].contiguous(), lengths[keep].contiguous()
+    x = torch.randn((n, C), generator=g)
+    ext, sizes = pkg.legacy.ext_module, (1, 1, H, W)
+    args = (coords.to(cuda), lengths.to(cuda), starts.to(cuda))
+    out = ext.bev_pool_forward(x.to(cuda), *args, *sizes)
+    exp, bad = ref.legacy_forward(x, coords, lengths, starts, *sizes)
+    assert bad == (order == 'invalid')
+    assert_bit_equal(out, exp, 'forward')
+    if bad:  # reported by the next call
+        with pytest.raises(RuntimeError, match='bev_pool_forward: 1 intervals'):
+            pkg.check_errors()
+    up = torch.randn(exp.shape, generator=g)
+    xg = ext.bev_pool_backward(up.to(cuda), *args, *sizes)
+    assert_bit_equal(xg, ref.legacy_backward(up, coords, lengths, starts, *sizes)[0], 'backward')
+    if bad:
+        with pytest.raises(RuntimeError, match='bev_pool_backward: 1 intervals'):
+            pkg.check_errors()
