@@ -118,6 +118,11 @@ _SIGNATURES = {
          _i64, _vp, _vp, _i64, _i64, _vp, _sz, _vp],
         ctypes.c_int,
     ),
+    'bevpool_backward_depth_image': (
+        [_vp, _i64, _i64, _i64, _i32, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32,
+         _i32, _i64, _vp, _vp, _i64, _i64, _vp, _sz, _vp],
+        ctypes.c_int,
+    ),
     'bevpool_timing_enable': ([ctypes.c_int], ctypes.c_int),
     'bevpool_timing_reset': ([], ctypes.c_int),
     'bevpool_timing_read': (

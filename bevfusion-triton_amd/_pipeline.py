@@ -350,21 +350,21 @@ def forward_depth(idx: PoolIndex, depth_flat, rows, D: int, HW: int, out, stride
 
 
 def backward_depth(idx: PoolIndex, grad, C: int, stride_b: int, stride_c: int, stride_z: int,
-                   depth_flat, rows, D: int, HW: int, grad_depth, grad_context3d) -> None:
-    """grad_depth (n_points,) and grad_context (BN, C, HW) <- grad."""
+                   depth_flat, rows, D: int, fH: int, fW: int, grad_depth, grad_context3d) -> None:
+    """grad_depth (n_points,) and grad_context (BN, C, fH*fW) <- grad."""
     lib = L.library()
     scratch_bytes = lib.bevpool_backward_scratch_bytes(idx.n_cells, C, L.F32)
     scratch = torch.empty(max(int(scratch_bytes), 256), dtype=torch.uint8, device=idx.device)
     with torch.cuda.device(idx.device):
         L.check(
-            lib.bevpool_backward_depth(
+            lib.bevpool_backward_depth_image(
                 L.ptr(grad), stride_b, stride_c, stride_z, C, L.ptr(idx.rank), idx.n_points, D,
-                HW, L.ptr(depth_flat), L.ptr(rows), L.ptr(idx.cell_start), L.ptr(idx.cell_end),
-                idx.B, idx.D, idx.H * idx.W, L.ptr(grad_depth), L.ptr(grad_context3d),
-                grad_context3d.stride(0), grad_context3d.stride(1), L.ptr(scratch),
-                scratch.numel(), L.stream_handle(idx.device),
+                fH, fW, L.ptr(depth_flat), L.ptr(rows), L.ptr(idx.cell_start),
+                L.ptr(idx.cell_end), idx.B, idx.D, idx.H * idx.W, L.ptr(grad_depth),
+                L.ptr(grad_context3d), grad_context3d.stride(0), grad_context3d.stride(1),
+                L.ptr(scratch), scratch.numel(), L.stream_handle(idx.device),
             ),
-            'bevpool_backward_depth',
+            'bevpool_backward_depth_image',
         )
 
 

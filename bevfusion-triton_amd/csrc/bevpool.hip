@@ -3456,134 +3456,146 @@ constexpr int kDgPix = 16;  // pixels per depth_grad block (4 per wave)
 //   grad_depth[p]        = sum_c g[rank[p], c] * ctx[pix(p), c]  (0 if dropped)
 //   grad_ctx[bn, c, hw]  = sum_d g[rank[p_d], c] * depth[p_d]
 // with p_d = (bn*D + d)*HW + hw.
-// A block takes kDgPix consecutive pixels.  Their ranks and depths are staged
-// in LDS ([d][pixel], read coalesced over the pixels); each wave then takes
-// kDgPix/4 pixels one after another, its four 16-lane rows taking the depth
-// bins d = 4 i + row, lane j of a row the channels j + 16 k (k < kK).  Per bin
-// a row gathers its cell's gradient row, reduces the dot product with
-// row_sum16 and adds depth * row to its context sums; the four rows' context
-// sums are combined in row order at the end of the pixel.  The dot products
-// replace the ranks in LDS and, like the context sums, are written out
-// coalesced.  g: cell-major fp32 rows of the occupied cells; ctx:
-// channel-last rows (planar_rows_kernel).  Blocks map XCD-contiguously, so
-// the cells of neighbouring pixels' rays meet in one L2.
-template <int kK, int kU>
+// A block takes a patch of kDgPix pixels: 4 rows of 4 columns of the image
+// (pw = 4), or 16 in a row (pw = 16, fH = 1) where the image's width is not
+// known.  Their ranks and depths are staged in LDS ([d][pixel]); each wave
+// then takes 4 pixels, one per 16-lane row of the wave: of a 4 x 4 patch a
+// column of 4, which lie above each other and so, bin by bin, mostly hit one
+// cell: the wave's four row loads are then one row's lines.  Lane j of a row
+// holds channels 64 q + 4 j + 0..3 (q < kX = C / 64, one 16-byte load each) and
+// 64 kX + 16 k + j (k < kR, the rest).  Per bin a row gathers its cell's
+// gradient row, reduces the dot product with row_sum16 and adds depth * row to
+// its context sums, bins d = 4 i + u in chain u; the chains are added in order
+// at the end.  The dot products replace the ranks in LDS and, like the context
+// sums, are written out from there.  g: cell-major fp32 rows of the occupied
+// cells; ctx: channel-last rows (planar_rows_kernel).  Blocks map
+// XCD-contiguously, so the cells of neighbouring pixels' rays meet in one L2.
+// Gathered rows from L2 bound it: 4 x 360 x 360, C = 80 (2.26 GB): 216 us with
+// one bin per row of the wave and 4-byte loads, 184 with 16-byte loads, 162
+// with the columns.
+template <int kX, int kR>
 __global__ __launch_bounds__(kThreads) void depth_grad_kernel(
     const float *__restrict__ g, int C, const int32_t *__restrict__ rank,
-    const float *__restrict__ depth, const float *__restrict__ ctx, int D, int64_t HW,
-    int64_t n_pix, uint32_t *__restrict__ grad_depth, float *__restrict__ grad_ctx,
-    int64_t gsbn, int64_t gsc) {
+    const float *__restrict__ depth, const float *__restrict__ ctx, int D, int fH, int fW, int pw,
+    int h_tiles, int w_tiles, int64_t n_tiles, uint32_t *__restrict__ grad_depth,
+    float *__restrict__ grad_ctx, int64_t gsbn, int64_t gsc) {
+  constexpr int kK = 4 * kX + kR;
+  constexpr int kU = 4;  // bins in flight (2, 3, 6, 8: 210, 194, 183, 198 against 184 us)
   extern __shared__ int dg_smem[];
   int *lr = dg_smem;                                             // [D][kDgPix]
   float *ldp = reinterpret_cast<float *>(dg_smem + D * kDgPix);  // [D][kDgPix]
   float *lgc = ldp + D * kDgPix;                                 // [C][kDgPix]
   const int tid = threadIdx.x;
-  const int64_t pix0 = xcd_chunk(blockIdx.x, gridDim.x) * kDgPix;
-  if (pix0 >= n_pix) return;  // XCD padding blocks
-  const int npx = n_pix - pix0 < kDgPix ? int(n_pix - pix0) : kDgPix;
-  for (int i = tid; i < D * kDgPix; i += kThreads) {
-    const int d = i / kDgPix, t = i - d * kDgPix;
-    int r = -1;
-    float dv = 0.0f;
-    if (t < npx) {
-      const int64_t pix = pix0 + t;
-      const int64_t bn = pix / HW, hw = pix - bn * HW;
-      const int64_t p = (bn * D + d) * HW + hw;
-      r = rank[p];
-      dv = depth[p];
+  const int64_t tile = xcd_chunk(blockIdx.x, gridDim.x);
+  if (tile >= n_tiles) return;  // XCD padding blocks
+  const int64_t bn = tile / (h_tiles * w_tiles);
+  const int tr = int(tile - bn * (h_tiles * w_tiles));
+  const int h0 = tr / w_tiles * (kDgPix / pw), w0 = tr % w_tiles * pw;
+  const int64_t plane = int64_t(fH) * fW;
+  // pixel t of the patch
+  auto pixel = [&](int t, int &h, int &w) {
+    h = h0 + t / pw;
+    w = w0 + t % pw;
+    return h < fH && w < fW;
+  };
+  {
+    int h, w;  // kThreads is a multiple of kDgPix: a thread stays with one pixel
+    const bool ok = pixel(tid % kDgPix, h, w);
+    const int64_t p0 = bn * D * plane + int64_t(h) * fW + w;
+    for (int i = tid; i < D * kDgPix; i += kThreads) {
+      const int64_t p = p0 + (i / kDgPix) * plane;
+      lr[i] = ok ? rank[p] : -1;
+      ldp[i] = ok ? depth[p] : 0.0f;
     }
-    lr[i] = r;
-    ldp[i] = dv;
   }
   __syncthreads();
-  const int lane = lane_id();
-  const int row = lane >> 4, j = lane & 15;
-  const int wave = tid >> 6;
-  int col[kK];
-  bool cv[kK];
+  const int lane = lane_id(), j = lane & 15;
+  const int t = (lane >> 4) * 4 + (tid >> 6);  // this row's pixel
+  // channels past C (possible in the last of the single ones only) are read
+  // clamped and masked
+  const int c1 = 64 * kX + 16 * (kR - 1) + j;
+  const bool last_ok = kR == 0 || c1 < C;
+  const int c1c = last_ok ? c1 : C - 1;
+  // a row's values for this lane, as raw bits
+  auto load_row = [&](const uint32_t *row, uint32_t(&v)[kK]) {
+#pragma unroll
+    for (int q = 0; q < kX; ++q) {
+      const u32x4 p = reinterpret_cast<const Bytes16 *>(row + 64 * q + 4 * j)->v;
+      v[4 * q] = p.x;
+      v[4 * q + 1] = p.y;
+      v[4 * q + 2] = p.z;
+      v[4 * q + 3] = p.w;
+    }
+#pragma unroll
+    for (int k = 0; k < kR; ++k)
+      v[4 * kX + k] = row[k + 1 < kR ? 64 * kX + 16 * k + j : c1c];
+  };
+  float xc[kK], gc[kU][kK];
+  {
+    int h, w;
+    const bool ok = pixel(t, h, w);
+    const int64_t pix = ok ? bn * plane + int64_t(h) * fW + w : 0;
+    uint32_t v[kK];
+    load_row(reinterpret_cast<const uint32_t *>(ctx + pix * C), v);
+#pragma unroll
+    for (int k = 0; k < kK; ++k) {
+      xc[k] = kR > 0 && k == kK - 1 && !last_ok ? 0.0f : __uint_as_float(v[k]);
+#pragma unroll
+      for (int u = 0; u < kU; ++u) gc[u][k] = 0.0f;
+    }
+  }
+  const uint32_t *gb = reinterpret_cast<const uint32_t *>(g);
+  for (int d0 = 0; d0 < D; d0 += kU) {
+    int rr[kU];
+    float dp[kU];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      const int d = d0 + u, dc = d < D ? d : D - 1;
+      const int r = lr[dc * kDgPix + t];
+      const float w = ldp[dc * kDgPix + t];
+      rr[u] = d < D ? r : -1;
+      dp[u] = d < D ? w : 0.0f;
+    }
+    // every load is issued (clamped rows/columns) and masked by a bitwise
+    // AND afterwards: a select would let the compiler sink each load into
+    // a branch of its own and wait for it there
+    float gv[kU][kK];
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      uint32_t v[kK];
+      load_row(gb + int64_t(rr[u] >= 0 ? rr[u] : 0) * C, v);
+      const uint32_t m = rr[u] >= 0 ? 0xFFFFFFFFu : 0u, ml = last_ok ? m : 0u;
+#pragma unroll
+      for (int k = 0; k < kK; ++k)
+        gv[u][k] = __uint_as_float(v[k] & (kR > 0 && k == kK - 1 ? ml : m));
+    }
+#pragma unroll
+    for (int u = 0; u < kU; ++u) {
+      float part = 0.0f;
+#pragma unroll
+      for (int k = 0; k < kK; ++k) part += gv[u][k] * xc[k];
+      const float dot = row_sum16(part);
+      if (j == 0 && d0 + u < D)
+        lr[(d0 + u) * kDgPix + t] = __builtin_bit_cast(int, rr[u] >= 0 ? dot : 0.0f);
+#pragma unroll
+      for (int k = 0; k < kK; ++k) gc[u][k] += gv[u][k] * dp[u];
+    }
+  }
 #pragma unroll
   for (int k = 0; k < kK; ++k) {
-    const int c = j + 16 * k;
-    cv[k] = c < C;
-    col[k] = cv[k] ? c : C - 1;
-  }
-  const int nrow = (D + 3) >> 2;  // bins per row
-  constexpr int kPerWave = kDgPix / kWaves;
-  for (int q = 0; q < kPerWave; ++q) {
-    const int t = wave * kPerWave + q;
-    if (t >= npx) break;  // wave-uniform
-    const int64_t pix = pix0 + t;
-    float xc[kK], gc[kK];
-#pragma unroll
-    for (int k = 0; k < kK; ++k) {
-      const float v = ctx[pix * C + col[k]];
-      xc[k] = cv[k] ? v : 0.0f;
-      gc[k] = 0.0f;
-    }
-    for (int i0 = 0; i0 < nrow; i0 += kU) {
-      int rr[kU];
-      float dp[kU];
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int d = 4 * (i0 + u) + row;
-        const int dc = d < D ? d : D - 1;
-        const int r = lr[dc * kDgPix + t];
-        const float w = ldp[dc * kDgPix + t];
-        rr[u] = d < D ? r : -1;
-        dp[u] = d < D ? w : 0.0f;
-      }
-      // every load is issued (clamped rows/columns) and masked by a bitwise
-      // AND afterwards: a select would let the compiler sink each load into
-      // a branch of its own and wait for it there
-      const uint32_t *gb = reinterpret_cast<const uint32_t *>(g);
-      float gv[kU][kK];
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        const int64_t base = int64_t(rr[u] >= 0 ? rr[u] : 0) * C;
-#pragma unroll
-        for (int k = 0; k < kK; ++k) {
-          const uint32_t m = (rr[u] >= 0 && cv[k]) ? 0xFFFFFFFFu : 0u;
-          gv[u][k] = __builtin_bit_cast(float, gb[base + col[k]] & m);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kU; ++u) {
-        float part = 0.0f;
-#pragma unroll
-        for (int k = 0; k < kK; ++k) part += gv[u][k] * xc[k];
-        const float dot = row_sum16(part);
-        const int d = 4 * (i0 + u) + row;
-        if (j == 0 && d < D) lr[d * kDgPix + t] = __builtin_bit_cast(int, rr[u] >= 0 ? dot : 0.0f);
-#pragma unroll
-        for (int k = 0; k < kK; ++k) gc[k] += gv[u][k] * dp[u];
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < kK; ++k) {
-      const float s0 = __shfl(gc[k], j, 64);
-      const float s1 = __shfl(gc[k], j + 16, 64);
-      const float s2 = __shfl(gc[k], j + 32, 64);
-      const float s3 = __shfl(gc[k], j + 48, 64);
-      const float tot = ((s0 + s1) + s2) + s3;
-      if (row == 0 && cv[k]) lgc[(j + 16 * k) * kDgPix + t] = tot;
-    }
+    const float tot = ((gc[0][k] + gc[1][k]) + gc[2][k]) + gc[3][k];
+    const int c = k < 4 * kX ? 64 * (k >> 2) + 4 * j + (k & 3) : 64 * kX + 16 * (k - 4 * kX) + j;
+    if (c < C) lgc[c * kDgPix + t] = tot;
   }
   __syncthreads();
-  for (int i = tid; i < D * kDgPix; i += kThreads) {
-    const int d = i / kDgPix, t = i - d * kDgPix;
-    if (t < npx) {
-      const int64_t pix = pix0 + t;
-      const int64_t bn = pix / HW, hw = pix - bn * HW;
-      grad_depth[(bn * D + d) * HW + hw] = uint32_t(lr[i]);
-    }
-  }
-  for (int i = tid; i < C * kDgPix; i += kThreads) {
-    const int c = i / kDgPix, t = i - c * kDgPix;
-    if (t < npx) {
-      const int64_t pix = pix0 + t;
-      const int64_t bn = pix / HW, hw = pix - bn * HW;
-      grad_ctx[bn * gsbn + int64_t(c) * gsc + hw] = lgc[i];
-    }
+  {
+    int h, w;
+    if (!pixel(tid % kDgPix, h, w)) return;
+    const int64_t hw = int64_t(h) * fW + w;
+    for (int i = tid; i < D * kDgPix; i += kThreads)
+      grad_depth[(bn * D + i / kDgPix) * plane + hw] = uint32_t(lr[i]);
+    for (int i = tid; i < C * kDgPix; i += kThreads)
+      grad_ctx[bn * gsbn + int64_t(i / kDgPix) * gsc + hw] = lgc[i];
   }
 }
 
@@ -4657,15 +4669,16 @@ int bevpool_forward_depth(const float *depth, const float *context_rows, int32_t
                             out_stride_b, out_stride_c, out_stride_z, out, s);
 }
 
-int bevpool_backward_depth(const float *grad, int64_t grad_stride_b, int64_t grad_stride_c,
-                           int64_t grad_stride_z, int32_t C, const int32_t *rank,
-                           int64_t n_points, int32_t D, int64_t HW, const float *depth,
-                           const float *context_rows, const int32_t *cell_start,
-                           const int32_t *cell_end, int32_t n_batch, int32_t n_z, int64_t n_xy,
-                           float *grad_depth, float *grad_context, int64_t gctx_stride_bn,
-                           int64_t gctx_stride_c, void *scratch, size_t scratch_bytes,
-                           void *stream) {
-  g_last_error.clear();
+// fH, fW: the image plane (HW = fH * fW); fH = 1 if its width is not known.
+static int backward_depth_impl(const float *grad, int64_t grad_stride_b, int64_t grad_stride_c,
+                               int64_t grad_stride_z, int32_t C, const int32_t *rank,
+                               int64_t n_points, int32_t D, int64_t HW, int32_t fH,
+                               const float *depth,
+                               const float *context_rows, const int32_t *cell_start,
+                               const int32_t *cell_end, int32_t n_batch, int32_t n_z, int64_t n_xy,
+                               float *grad_depth, float *grad_context, int64_t gctx_stride_bn,
+                               int64_t gctx_stride_c, void *scratch, size_t scratch_bytes,
+                               void *stream) {
   if (C < 1 || C > 256) return fail(BEVPOOL_EINVAL, "C must be in [1, 256]");
   if (D < 1 || HW < 1) return fail(BEVPOOL_EINVAL, "bad depth layout");
   if (n_batch < 1 || n_z < 1 || n_xy < 1) return fail(BEVPOOL_EINVAL, "bad grid");
@@ -4684,32 +4697,71 @@ int bevpool_backward_depth(const float *grad, int64_t grad_stride_b, int64_t gra
   if (smem > 65536)
     return fail(BEVPOOL_EINVAL, "depth bins and channels too many (2*D + C = %lld > 1024)",
                 (long long)(2 * int64_t(D) + C));
+  if (HW > INT32_MAX) return fail(BEVPOOL_EINVAL, "bad depth layout");
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const int fW = int(HW / fH);
+  // 4 x 4 pixels per block, or 16 in a row without an image plane (or with one
+  // of fewer than 4 rows or columns, which would leave most of a patch empty)
+  const int pw = fH >= 4 && fW >= 4 ? 4 : kDgPix;
+  const int h_tiles = int(ceil_div(fH, kDgPix / pw)), w_tiles = int(ceil_div(fW, pw));
+  const int64_t n_tiles = n_pix / HW * h_tiles * w_tiles;
   int st;
-  if ((st = check_grid(ceil_div(n_pix, kDgPix) + kXcds, kThreads, "depth_grad"))) return st;
+  if ((st = check_grid(n_tiles + kXcds, kThreads, "depth_grad"))) return st;
   if ((st = launch_bev_to_rows(grad, 4, grad_stride_b, grad_stride_c, grad_stride_z, C,
                                cell_end, n_cells, n_z, n_xy, scratch, s)))
     return st;
-  const unsigned grid = xcd_grid(ceil_div(n_pix, kDgPix));
+  const unsigned grid = xcd_grid(n_tiles);
   LaunchTimer t("depth_grad", s);
   const float *g = static_cast<const float *>(scratch);
   uint32_t *gd = reinterpret_cast<uint32_t *>(grad_depth);
-#define BEVPOOL_DG(K, U)                                                                       \
-  hipLaunchKernelGGL((depth_grad_kernel<K, U>), dim3(grid), dim3(kThreads), smem, s, g, C,     \
-                     rank, depth, context_rows, D, HW, n_pix, gd, grad_context, gctx_stride_bn, \
-                     gctx_stride_c)
-  const int kk = (C + 15) / 16;
-  if (kk <= 1) BEVPOOL_DG(1, 8);
-  else if (kk <= 2) BEVPOOL_DG(2, 8);
-  else if (kk <= 3) BEVPOOL_DG(3, 8);
-  else if (kk <= 4) BEVPOOL_DG(4, 8);
-  else if (kk <= 5) BEVPOOL_DG(5, 8);
-  else if (kk <= 6) BEVPOOL_DG(6, 8);
-  else if (kk <= 8) BEVPOOL_DG(8, 4);
-  else if (kk <= 12) BEVPOOL_DG(12, 4);
-  else BEVPOOL_DG(16, 4);
+#define BEVPOOL_DG(X, R)                                                                       \
+  case 5 * X + R:                                                                              \
+    hipLaunchKernelGGL((depth_grad_kernel<X, R>), dim3(grid), dim3(kThreads), smem, s, g, C,    \
+                       rank, depth, context_rows, D, fH, fW, pw, h_tiles, w_tiles, n_tiles,    \
+                       gd, grad_context, gctx_stride_bn, gctx_stride_c);                       \
+    break;
+  // a lane's channels: 4 for each 64, then one for each 16 of the rest
+  switch (5 * (C / 64) + (C % 64 + 15) / 16) {
+    BEVPOOL_DG(0, 1) BEVPOOL_DG(0, 2) BEVPOOL_DG(0, 3) BEVPOOL_DG(0, 4)
+    BEVPOOL_DG(1, 0) BEVPOOL_DG(1, 1) BEVPOOL_DG(1, 2) BEVPOOL_DG(1, 3) BEVPOOL_DG(1, 4)
+    BEVPOOL_DG(2, 0) BEVPOOL_DG(2, 1) BEVPOOL_DG(2, 2) BEVPOOL_DG(2, 3) BEVPOOL_DG(2, 4)
+    BEVPOOL_DG(3, 0) BEVPOOL_DG(3, 1) BEVPOOL_DG(3, 2) BEVPOOL_DG(3, 3) BEVPOOL_DG(3, 4)
+    BEVPOOL_DG(4, 0)
+  }
 #undef BEVPOOL_DG
   return check_launch("depth_grad");
+}
+
+int bevpool_backward_depth(const float *grad, int64_t grad_stride_b, int64_t grad_stride_c,
+                           int64_t grad_stride_z, int32_t C, const int32_t *rank,
+                           int64_t n_points, int32_t D, int64_t HW, const float *depth,
+                           const float *context_rows, const int32_t *cell_start,
+                           const int32_t *cell_end, int32_t n_batch, int32_t n_z, int64_t n_xy,
+                           float *grad_depth, float *grad_context, int64_t gctx_stride_bn,
+                           int64_t gctx_stride_c, void *scratch, size_t scratch_bytes,
+                           void *stream) {
+  g_last_error.clear();
+  return backward_depth_impl(grad, grad_stride_b, grad_stride_c, grad_stride_z, C, rank, n_points,
+                             D, HW, 1, depth, context_rows, cell_start, cell_end, n_batch, n_z,
+                             n_xy, grad_depth, grad_context, gctx_stride_bn, gctx_stride_c,
+                             scratch, scratch_bytes, stream);
+}
+
+int bevpool_backward_depth_image(const float *grad, int64_t grad_stride_b, int64_t grad_stride_c,
+                                 int64_t grad_stride_z, int32_t C, const int32_t *rank,
+                                 int64_t n_points, int32_t D, int32_t fH, int32_t fW,
+                                 const float *depth, const float *context_rows,
+                                 const int32_t *cell_start, const int32_t *cell_end,
+                                 int32_t n_batch, int32_t n_z, int64_t n_xy, float *grad_depth,
+                                 float *grad_context, int64_t gctx_stride_bn,
+                                 int64_t gctx_stride_c, void *scratch, size_t scratch_bytes,
+                                 void *stream) {
+  g_last_error.clear();
+  if (fH < 1 || fW < 1) return fail(BEVPOOL_EINVAL, "bad feature map (%d x %d)", fH, fW);
+  return backward_depth_impl(grad, grad_stride_b, grad_stride_c, grad_stride_z, C, rank, n_points,
+                             D, int64_t(fH) * fW, fH, depth, context_rows, cell_start, cell_end,
+                             n_batch, n_z, n_xy, grad_depth, grad_context, gctx_stride_bn,
+                             gctx_stride_c, scratch, scratch_bytes, stream);
 }
 
 size_t bevpool_backward_scratch_bytes(int64_t n_cells, int32_t C, int32_t dtype) {

@@ -184,7 +184,7 @@ class _LSSBevPoolDepth(torch.autograd.Function):
         grad_depth = torch.empty((BN, D, fH, fW), dtype=torch.float32, device=g.device)
         grad_context = torch.empty((BN, C, fH, fW), dtype=torch.float32, device=g.device)
         P.backward_depth(idx, g, C, g.stride(0), g.stride(1), C * g.stride(1), depth_flat, rows,
-                         D, fH * fW, grad_depth.view(-1), grad_context.view(BN, C, fH * fW))
+                         D, fH, fW, grad_depth.view(-1), grad_context.view(BN, C, fH * fW))
         return grad_depth, grad_context, None, None, None, None, None, None
 
 

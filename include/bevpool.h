@@ -357,6 +357,22 @@ int bevpool_backward_depth(const float *grad, int64_t grad_stride_b, int64_t gra
                            void *stream);
 
 /*
+ * bevpool_backward_depth for a caller that states the image plane, HW = fH *
+ * fW with hw = h*fW + w: the points of a depth bin and an image column mostly
+ * share a cell, so pixels are taken column by column.  The same sums in the
+ * same order.
+ */
+int bevpool_backward_depth_image(const float *grad, int64_t grad_stride_b, int64_t grad_stride_c,
+                                 int64_t grad_stride_z, int32_t C, const int32_t *rank,
+                                 int64_t n_points, int32_t D, int32_t fH, int32_t fW,
+                                 const float *depth, const float *context_rows,
+                                 const int32_t *cell_start, const int32_t *cell_end,
+                                 int32_t n_batch, int32_t n_z, int64_t n_xy, float *grad_depth,
+                                 float *grad_context, int64_t gctx_stride_bn,
+                                 int64_t gctx_stride_c, void *scratch, size_t scratch_bytes,
+                                 void *stream);
+
+/*
  * One-call op level: ops/bev_pool/src/bev_pool_triton.py:219-227
  * (bev_pool(feats, coords, B, D, H, W)) as bevpool_coord_ranks ->
  * bevpool_sort -> bevpool_forward.  Two caller-owned buffers:
