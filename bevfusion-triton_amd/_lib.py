@@ -123,6 +123,9 @@ _SIGNATURES = {
          _i32, _i64, _vp, _vp, _i64, _i64, _vp, _sz, _vp],
         ctypes.c_int,
     ),
+    'bevpool_planar_kept_rows': (
+        [_vp, _i64, _i64, _i32, _i32, _i64, _vp, _vp, _vp], ctypes.c_int,
+    ),
     'bevpool_timing_enable': ([ctypes.c_int], ctypes.c_int),
     'bevpool_timing_reset': ([], ctypes.c_int),
     'bevpool_timing_read': (

@@ -289,21 +289,23 @@ def _backward_call(lib, idx, grad, dtype, C, stride_b, stride_c, stride_z, x_gra
 
 # ---- depth-weighted (fused depth x context) pooling -------------------------
 
-def planar_rows(src3d):
+def planar_rows(src3d, rank=None):
     """(BN, C, S) fp32 planar tensor (S contiguous, any batch/channel strides)
-    -> (BN*S, C) channel-last rows."""
+    -> (BN*S, C) channel-last rows.  With the points' ``rank``, the rows of
+    dropped points are left undefined (nothing reads them)."""
     BN, C, S = src3d.shape
     if src3d.stride(2) != 1:
         src3d = src3d.contiguous()
     rows = torch.empty((BN * S, C), dtype=torch.float32, device=src3d.device)
+    src = (L.ptr(src3d), src3d.stride(0), src3d.stride(1), BN, C, S)
+    lib = L.library()
     with torch.cuda.device(src3d.device):
-        L.check(
-            L.library().bevpool_planar_rows(
-                L.ptr(src3d), src3d.stride(0), src3d.stride(1), BN, C, S, L.ptr(rows),
-                L.stream_handle(src3d.device),
-            ),
-            'bevpool_planar_rows',
-        )
+        stream = L.stream_handle(src3d.device)
+        if rank is None:
+            L.check(lib.bevpool_planar_rows(*src, L.ptr(rows), stream), 'bevpool_planar_rows')
+        else:
+            L.check(lib.bevpool_planar_kept_rows(*src, L.ptr(rank), L.ptr(rows), stream),
+                    'bevpool_planar_kept_rows')
     return rows
 
 

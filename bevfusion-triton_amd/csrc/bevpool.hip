@@ -43,7 +43,7 @@
 //                               each point's cell row (zero rows for dropped
 //                               points)
 //   planar (channel-first) operands
-//     planar_rows_kernel        (BN, C, S) -> channel-last rows (context, or
+//     planar_tile_kernel        (BN, C, S) -> channel-last rows (context, or
 //                               channel-first camera features)
 //     gather_planar_kernel      backward straight into a (BN, C, S) gradient
 //   depth-weighted pooling (fused depth x context)
@@ -2351,7 +2351,8 @@ __global__ __launch_bounds__(kThreads) void accum_group_kernel(
 // channel with one 16-byte (fp32) or 8-byte (16-bit) access.  With kVecBev
 // (n_xy, the b/z/c strides and the base are multiples of 4 elements) 4 cells
 // starting at a multiple of 4 always share a (b, z) plane and the access is
-// aligned; otherwise it is an access at element alignment, and the few groups
+// aligned (and the output's stores non-temporal: it is not read again here);
+// otherwise it is an access at element alignment, and the few groups
 // of 4 cells that a plane's end cuts go cell by cell.  On the row side
 // kVecRow (rows of 16 bytes or more) moves 16-byte pieces of a row; where the
 // row is no multiple of 16 bytes the last piece ends at the row's end and
@@ -2470,7 +2471,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
           if constexpr (kVecBev)
             __builtin_nontemporal_store(V{}, reinterpret_cast<V *>(dst));
           else
-            __builtin_nontemporal_store(V{}, reinterpret_cast<VA *>(dst));
+            *reinterpret_cast<VA *>(dst) = V{};
         } else {
 #pragma unroll
           for (int u = 0; u < 4; ++u)
@@ -2573,7 +2574,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
           if constexpr (kVecBev)
             __builtin_nontemporal_store(w, reinterpret_cast<u32x4 *>(dst));
           else
-            __builtin_nontemporal_store(w, reinterpret_cast<u32x4_any *>(dst));
+            reinterpret_cast<Bytes16 *>(dst)->v = w;
         } else {
           u32x2 w;
           w.x = uint32_t(r[0]) | (uint32_t(r[1]) << 16);
@@ -2581,7 +2582,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
           if constexpr (kVecBev)
             __builtin_nontemporal_store(w, reinterpret_cast<u32x2 *>(dst));
           else
-            __builtin_nontemporal_store(w, reinterpret_cast<u32x2_any *>(dst));
+            reinterpret_cast<Bytes8 *>(dst)->v = w;
         }
       } else {
 #pragma unroll
@@ -3239,70 +3240,62 @@ __global__ __launch_bounds__(kThreads) void run_length_kernel(const int32_t *__r
 // features (S = D*fH*fW, the storage behind the reference's rearrange view,
 // depth_lss.py:94).  Point p = bn*S + s.
 
-// planar -> rows (BN*S, C), fp32.  Tiled form (C <= 128, C, S, sbn, sc
-// multiples of 4, 16-byte aligned bases): planar_tile_kernel.  Vector form
-// (wider rows): a block covers 256 consecutive s of one bn; thread
-// (wave w, lane l) owns points s0 + [0, 4) and walks the channels in 4x4
-// blocks c0 + [0, 4) (c0 = 4 (l >> 4) + 16 i): four 16-byte loads along s (16
-// lanes of a channel read 256 contiguous bytes), a register transpose, four
-// 16-byte row stores (4 lanes write 64 contiguous bytes of a row; the wave
-// completes its 64 rows within one pass over the channels).  Non-temporal
-// stores: the rows are read back by a random gather, not from cache.  No LDS,
-// no barrier.  Scalar form: one element per thread.
-#ifndef BEVPOOL_PLANAR_NT
-#define BEVPOOL_PLANAR_NT 1
-#endif
-
-__device__ __forceinline__ void store16(u32x4 *p, u32x4 v) {
-#if BEVPOOL_PLANAR_NT
-  __builtin_nontemporal_store(v, p);
-#else
-  *p = v;
-#endif
+__device__ __forceinline__ void store16(float *p, u32x4 v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any *>(p));
 }
 
-// Tiled planar -> rows: a block moves kPlanarTile consecutive s of one bn,
-// all C channels, through an LDS tile [s][C + 1] (<= 66 KB at C = 128).  Each
-// group of kPlanarTile / 4 lanes loads kPlanarTile * 4 contiguous bytes of one
-// channel (kPer 16-byte loads per thread, all issued before the tile is
-// written); after one barrier the block writes its rows as one contiguous run
-// of kPlanarTile * C floats, 16 bytes per thread, consecutive threads at
-// consecutive addresses (non-temporal).  Measured at det (1.28 GB): 64-point
-// tiles 248 us against 288 us for the register transpose, whose row stores
-// scatter 16-byte pieces over 16 rows; 128-point tiles (512-byte runs per
-// channel) a further -6 us on the channel-first forward.
-#ifndef BEVPOOL_PLANAR_TS
-#define BEVPOOL_PLANAR_TS 128
-#endif
-constexpr int kPlanarTile = BEVPOOL_PLANAR_TS;  // points per tile (64 or 128)
+// planar -> rows (BN*S, C), fp32, for C >= 4 and S >= 4 of any alignment: a
+// block moves kPlanarTile consecutive s of one bn and at most kPlanarChannels
+// channels through an LDS tile [s][channel] (<= 66 KB).  Each group of
+// kPlanarTile / 4 lanes loads kPlanarTile * 4 contiguous bytes of one channel
+// (kPer 16-byte loads per thread, all issued before the tile is written);
+// after one barrier the block writes its rows, 16 bytes per thread,
+// consecutive threads at consecutive addresses.  Ragged sizes keep to 16-byte
+// accesses by overlap: a camera's last tile is shifted back to end at S, a
+// row's last piece to end at its last channel; what is moved twice is the
+// same.  Non-temporal stores: the rows are read back by a random gather, and
+// left temporal, their dirty lines slowed the accumulation that follows from
+// 126 to 171 us.  With `rank`, rows of dropped points (rank -1), which nothing
+// reads, are not written.
+// HBM traffic bounds it (1.28 GB at 1 x 360 x 360: 235 us; 64-point tiles 6 us
+// more, a register transpose whose stores scatter 16-byte pieces 288 us).
+// Without the dropped points' rows, 14% of them at 1 x 256 x 256, it takes 219
+// us, and with four height bins, where 46% are dropped, 183 us.  Maps that 4
+// does not divide (2 x 6 x 45 x 29 x 51 points, C = 64): 80 us, 244 one element
+// per thread (and the planar gradient 42 us, 155).
+constexpr int kPlanarTile = 128, kPlanarChannels = 128;
 template <int kPer>
 __global__ __launch_bounds__(kThreads) void planar_tile_kernel(
-    const float *__restrict__ src, int C, int64_t S, int64_t tiles_s, int64_t sbn, int64_t sc,
-    float *__restrict__ rows) {
+    const float *__restrict__ src, int C, int cmax, int64_t S, int64_t tiles_s, int64_t sbn,
+    int64_t sc, const int32_t *__restrict__ rank, float *__restrict__ rows) {
   constexpr int kQ = kPlanarTile / 4;  // 16-byte pieces per channel of a tile
-  extern __shared__ float tile[];  // [kPlanarTile][C + 1]
-  const int pitch = C + 1, tid = threadIdx.x;
+  extern __shared__ float tile[];  // [kPlanarTile][cb + 1]
+  __shared__ int s_rank[kPlanarTile];
+  const int tid = threadIdx.x;
+  const int c0 = int(blockIdx.y) * cmax, cb = C - c0 < cmax ? C - c0 : cmax;
+  const int pitch = cb + 1;
   const int64_t bn = int64_t(blockIdx.x) / tiles_s;
-  const int64_t s0 = (int64_t(blockIdx.x) - bn * tiles_s) * kPlanarTile;
-  const int np = S - s0 < kPlanarTile ? int(S - s0) : kPlanarTile;  // a multiple of 4
-  const float *in = src + bn * sbn + s0;
-  const int npc = C * kQ;  // 16-byte pieces on the channel side
+  const int np = S < kPlanarTile ? int(S) : kPlanarTile;
+  int64_t s0 = (int64_t(blockIdx.x) - bn * tiles_s) * kPlanarTile;
+  s0 = s0 < S - np ? s0 : S - np;
+  const float *in = src + bn * sbn + int64_t(c0) * sc + s0;
   u32x4 v[kPer];
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
-    // piece e: channel e / 16, points 4 (e % 16) + [0, 4); pieces past the
-    // tile reload an in-bounds one and are not written
+    // piece e: channel e / kQ, points 4 (e % kQ) + [0, 4), or the last 4;
+    // pieces past the channels reload the last one and are not written
     const int e = tid + kThreads * i;
-    const int c = e / kQ, pq = e % kQ;
-    const int cc = c < C ? c : C - 1, pp = 4 * pq < np ? pq : 0;
-    v[i] = *reinterpret_cast<const u32x4 *>(in + int64_t(cc) * sc + 4 * pp);
+    const int c = e / kQ < cb ? e / kQ : cb - 1;
+    const int p = 4 * (e % kQ) < np - 4 ? 4 * (e % kQ) : np - 4;
+    v[i] = reinterpret_cast<const Bytes16 *>(in + int64_t(c) * sc + p)->v;
   }
+  if (rank && tid < np) s_rank[tid] = rank[bn * S + s0 + tid];
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int e = tid + kThreads * i;
-    const int c = e / kQ, pq = e % kQ;
-    if (e < npc && 4 * pq < np) {
-      float *t = tile + (4 * pq) * pitch + c;
+    const int c = e / kQ, p = 4 * (e % kQ) < np - 4 ? 4 * (e % kQ) : np - 4;
+    if (c < cb) {
+      float *t = tile + p * pitch + c;
       t[0] = __uint_as_float(v[i].x);
       t[pitch] = __uint_as_float(v[i].y);
       t[2 * pitch] = __uint_as_float(v[i].z);
@@ -3310,115 +3303,90 @@ __global__ __launch_bounds__(kThreads) void planar_tile_kernel(
     }
   }
   __syncthreads();
-  const int q = C >> 2, nrp = np * q;
-  u32x4 *out = reinterpret_cast<u32x4 *>(rows + (bn * S + s0) * C);
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int e = tid + kThreads * i;  // row e / q, 16-byte column e % q
-    if (e < nrp) {
-      const int p = e / q, j = e - p * q;
-      const float *t = tile + p * pitch + 4 * j;
-      store16(out + e, u32x4{__float_as_uint(t[0]), __float_as_uint(t[1]), __float_as_uint(t[2]),
-                             __float_as_uint(t[3])});
-    }
+  const int q = (cb + 3) >> 2, n = np * q;
+  float *out = rows + (bn * S + s0) * C + c0;
+  for (int e = tid; e < n; e += kThreads) {
+    const int p = e / q;  // row p, its piece e % q
+    const int c = 4 * (e - p * q) < cb - 4 ? 4 * (e - p * q) : cb - 4;
+    if (rank && s_rank[p] < 0) continue;
+    const float *t = tile + p * pitch + c;
+    store16(out + int64_t(p) * C + c, u32x4{__float_as_uint(t[0]), __float_as_uint(t[1]),
+                                            __float_as_uint(t[2]), __float_as_uint(t[3])});
   }
 }
 
-template <bool kVec, int kIt>
+// The same one element per thread, for fewer than 4 channels or points.
 __global__ __launch_bounds__(kThreads) void planar_rows_kernel(
-    const float *__restrict__ src, int C, int64_t S, int64_t tiles_s, int64_t n_rows,
-    int64_t sbn, int64_t sc, float *__restrict__ rows) {
-  if constexpr (kVec) {
-    const int64_t bn = int64_t(blockIdx.x) / tiles_s;
-    const int64_t ts = int64_t(blockIdx.x) - bn * tiles_s;
-    const int lane = lane_id(), w = threadIdx.x >> 6;
-    const int64_t s0 = ts * 256 + w * 64 + (lane & 15) * 4;
-    if (s0 >= S) return;
-    const float *in = src + bn * sbn + s0;
-    u32x4 *out = reinterpret_cast<u32x4 *>(rows + (bn * S + s0) * C);
-    const int q = C / 4;  // 16-byte pieces per row
-    // all channels of these rows, 16 at a time (kIt passes with every load
-    // issued before the first store), so each row is completed by this wave
-    // within a few instructions
-    for (int cb = (lane >> 4) * 4; cb < C; cb += 16 * kIt) {
-      u32x4 a[kIt][4];
-#pragma unroll
-      for (int i = 0; i < kIt; ++i) {
-        const int c0 = cb + 16 * i < C ? cb + 16 * i : cb;  // past C: reload (not stored)
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          a[i][k] = *reinterpret_cast<const u32x4 *>(in + int64_t(c0 + k) * sc);
-      }
-#pragma unroll
-      for (int i = 0; i < kIt; ++i) {
-        if (cb + 16 * i < C) {
-          u32x4 *o = out + (cb + 16 * i) / 4;
-          store16(o, u32x4{a[i][0].x, a[i][1].x, a[i][2].x, a[i][3].x});
-          store16(o + q, u32x4{a[i][0].y, a[i][1].y, a[i][2].y, a[i][3].y});
-          store16(o + 2 * q, u32x4{a[i][0].z, a[i][1].z, a[i][2].z, a[i][3].z});
-          store16(o + 3 * q, u32x4{a[i][0].w, a[i][1].w, a[i][2].w, a[i][3].w});
-        }
-      }
-    }
-  } else {
-    const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= n_rows * C) return;
-    const int64_t r = i / C;
-    const int c = int(i - r * C);
-    const int64_t bn = r / S, sp = r - bn * S;
-    rows[i] = src[bn * sbn + int64_t(c) * sc + sp];
-  }
+    const float *__restrict__ src, int C, int64_t S, int64_t n_rows, int64_t sbn, int64_t sc,
+    float *__restrict__ rows) {
+  const int64_t i = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+  if (i >= n_rows * C) return;
+  const int64_t r = i / C;
+  const int c = int(i - r * C);
+  const int64_t bn = r / S, sp = r - bn * S;
+  rows[i] = src[bn * sbn + int64_t(c) * sc + sp];
 }
 
 // Backward of the op-level pooling into a planar gradient:
 // x_grad[bn, c, s] = g[rank[bn*S + s], c] (0 for dropped points), g the
-// cell-major rows of bev_to_rows_kernel.  Vector form (C, S, sbn, sc multiples
-// of 4, 16-byte aligned x_grad): a thread takes 4 consecutive points and walks
-// the channels 4 at a time: four 16-byte row loads (cache-resident rows), a
-// register transpose, four 16-byte stores along s (a wave writes 1 KB
-// contiguous per channel, non-temporal).  Blocks map XCD-contiguously.
-template <bool kVec, int kIt>
+// cell-major rows of bev_to_rows_kernel.  Vector form (C >= 4, S >= 4, any
+// alignment; what does not divide by 4 overlaps as in planar_tile_kernel): a
+// thread takes 4 consecutive points of one bn and walks the channels 4 at a
+// time, kIt such groups in flight: four 16-byte row loads (cache-resident
+// rows), a register transpose, four 16-byte stores along s (a wave writes 1 KB
+// contiguous per channel).  Blocks map XCD-contiguously.  The write stream
+// bounds it: 638 MB at 1 x 360 x 360 in 130-140 us.  Aligned stores are
+// non-temporal (kStream; temporal ones took 148 us there and the next forward
+// 50 more, and gained nothing over whole steps on new inputs where the
+// memory-side cache holds the gradient); stores at other addresses are
+// temporal, so that the caches merge the lines that two of them share.
+template <bool kVec, bool kStream>
 __global__ __launch_bounds__(kThreads) void gather_planar_kernel(
     const float *__restrict__ g, int C, const int32_t *__restrict__ rank, int64_t n_points,
-    int64_t S, int64_t sbn, int64_t sc, float *__restrict__ x_grad) {
+    int64_t S, FastDiv groups, int64_t n_groups, int64_t sbn, int64_t sc,
+    float *__restrict__ x_grad) {
   if constexpr (kVec) {
-    const int64_t groups = n_points / 4;  // S % 4 == 0: a group never spans two bn
+    constexpr int kIt = 2;
     const int64_t gi = xcd_chunk(blockIdx.x, gridDim.x) * kThreads + threadIdx.x;
-    if (gi >= groups) return;
-    const int64_t p0 = gi * 4;
-    const u32x4 rk = *reinterpret_cast<const u32x4 *>(rank + p0);
+    if (gi >= n_groups) return;
+    // groups of 4 points per bn, the last one shifted back to end at S
+    const uint32_t bn = groups.div(uint32_t(gi));
+    int64_t sp = 4 * int64_t(uint32_t(gi) - bn * groups.d);
+    sp = sp < S - 4 ? sp : S - 4;
+    const u32x4 rk = reinterpret_cast<const Bytes16 *>(rank + bn * S + sp)->v;
     const int r0 = int(rk.x), r1 = int(rk.y), r2 = int(rk.z), r3 = int(rk.w);
-    const u32x4 *g0 = reinterpret_cast<const u32x4 *>(g + int64_t(r0 >= 0 ? r0 : 0) * C);
-    const u32x4 *g1 = reinterpret_cast<const u32x4 *>(g + int64_t(r1 >= 0 ? r1 : 0) * C);
-    const u32x4 *g2 = reinterpret_cast<const u32x4 *>(g + int64_t(r2 >= 0 ? r2 : 0) * C);
-    const u32x4 *g3 = reinterpret_cast<const u32x4 *>(g + int64_t(r3 >= 0 ? r3 : 0) * C);
+    const float *g0 = g + int64_t(r0 >= 0 ? r0 : 0) * C;
+    const float *g1 = g + int64_t(r1 >= 0 ? r1 : 0) * C;
+    const float *g2 = g + int64_t(r2 >= 0 ? r2 : 0) * C;
+    const float *g3 = g + int64_t(r3 >= 0 ? r3 : 0) * C;
     const uint32_t m0 = r0 >= 0 ? 0xFFFFFFFFu : 0u, m1 = r1 >= 0 ? 0xFFFFFFFFu : 0u;
     const uint32_t m2 = r2 >= 0 ? 0xFFFFFFFFu : 0u, m3 = r3 >= 0 ? 0xFFFFFFFFu : 0u;
-    const int64_t bn = p0 / S, sp = p0 - bn * S;
-    float *out = x_grad + bn * sbn + sp;
-    const int nq = C / 4;
-    for (int qb = 0; qb < nq; qb += kIt) {
+    float *out = x_grad + int64_t(bn) * sbn + sp;
+    auto put = [](float *p, u32x4 v) {
+      if constexpr (kStream)
+        store16(p, v);
+      else
+        reinterpret_cast<Bytes16 *>(p)->v = v;
+    };
+    auto piece = [](const float *p) { return reinterpret_cast<const Bytes16 *>(p)->v; };
+    for (int cb = 0; cb < C; cb += 4 * kIt) {
       u32x4 a[kIt][4];
 #pragma unroll
       for (int i = 0; i < kIt; ++i) {  // every row piece of kIt groups, then the stores
-        const int q = qb + i < nq ? qb + i : qb;
-        a[i][0] = g0[q] & m0;
-        a[i][1] = g1[q] & m1;
-        a[i][2] = g2[q] & m2;
-        a[i][3] = g3[q] & m3;
+        const int c = cb + 4 * i < C - 4 ? cb + 4 * i : C - 4;
+        a[i][0] = piece(g0 + c) & m0;
+        a[i][1] = piece(g1 + c) & m1;
+        a[i][2] = piece(g2 + c) & m2;
+        a[i][3] = piece(g3 + c) & m3;
       }
 #pragma unroll
       for (int i = 0; i < kIt; ++i) {
-        if (qb + i < nq) {
-          float *o = out + int64_t(4 * (qb + i)) * sc;
-          __builtin_nontemporal_store(u32x4{a[i][0].x, a[i][1].x, a[i][2].x, a[i][3].x},
-                                      reinterpret_cast<u32x4 *>(o));
-          __builtin_nontemporal_store(u32x4{a[i][0].y, a[i][1].y, a[i][2].y, a[i][3].y},
-                                      reinterpret_cast<u32x4 *>(o + sc));
-          __builtin_nontemporal_store(u32x4{a[i][0].z, a[i][1].z, a[i][2].z, a[i][3].z},
-                                      reinterpret_cast<u32x4 *>(o + 2 * sc));
-          __builtin_nontemporal_store(u32x4{a[i][0].w, a[i][1].w, a[i][2].w, a[i][3].w},
-                                      reinterpret_cast<u32x4 *>(o + 3 * sc));
+        if (cb + 4 * i < C) {
+          float *o = out + int64_t(cb + 4 * i < C - 4 ? cb + 4 * i : C - 4) * sc;
+          put(o, u32x4{a[i][0].x, a[i][1].x, a[i][2].x, a[i][3].x});
+          put(o + sc, u32x4{a[i][0].y, a[i][1].y, a[i][2].y, a[i][3].y});
+          put(o + 2 * sc, u32x4{a[i][0].z, a[i][1].z, a[i][2].z, a[i][3].z});
+          put(o + 3 * sc, u32x4{a[i][0].w, a[i][1].w, a[i][2].w, a[i][3].w});
         }
       }
     }
@@ -3468,7 +3436,7 @@ constexpr int kDgPix = 16;  // pixels per depth_grad block (4 per wave)
 // its context sums, bins d = 4 i + u in chain u; the chains are added in order
 // at the end.  The dot products replace the ranks in LDS and, like the context
 // sums, are written out from there.  g: cell-major fp32 rows of the occupied
-// cells; ctx: channel-last rows (planar_rows_kernel).  Blocks map
+// cells; ctx: channel-last rows (planar_tile_kernel).  Blocks map
 // XCD-contiguously, so the cells of neighbouring pixels' rays meet in one L2.
 // Gathered rows from L2 bound it: 4 x 360 x 360, C = 80 (2.26 GB): 216 us with
 // one bin per row of the wave and 4-byte loads, 184 with 16-byte loads, 162
@@ -4527,56 +4495,62 @@ int bevpool_forward(const void *feats, int32_t dtype, int64_t feats_row_stride, 
                       scratch, scratch_bytes, stream, MetaReport{});
 }
 
-int bevpool_planar_rows(const float *src, int64_t stride_bn, int64_t stride_c, int32_t BN,
-                        int32_t C, int64_t S, float *rows, void *stream) {
-  g_last_error.clear();
+// rank: null, or the points' ranks: rows of dropped points need not be written.
+static int planar_rows_impl(const float *src, int64_t stride_bn, int64_t stride_c, int32_t BN,
+                            int32_t C, int64_t S, const int32_t *rank, float *rows,
+                            void *stream) {
   if (BN < 0 || C < 1 || S < 0) return fail(BEVPOOL_EINVAL, "bad planar shape");
   const int64_t n_rows = int64_t(BN) * S;
   if (n_rows == 0) return BEVPOOL_OK;
   if (!src || !rows) return fail(BEVPOOL_EINVAL, "null argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool vec = C % 4 == 0 && S % 4 == 0 && stride_bn % 4 == 0 && stride_c % 4 == 0 &&
-                   reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(rows) % 16 == 0;
+  const bool vec = C >= 4 && S >= 4;
+  const int64_t tiles_s = ceil_div(S, kPlanarTile);
   LaunchTimer t("planar_rows", s);
-  int st = check_grid(vec ? BN * ceil_div(S, C <= 128 ? kPlanarTile : 256) : ceil_div(n_rows * C, kThreads),
-                      kThreads, "planar_rows");
+  // (sizes that do not divide by 4 keep the limit of one element per thread)
+  const bool even = C % 4 == 0 && S % 4 == 0 && stride_bn % 4 == 0 && stride_c % 4 == 0;
+  int st = check_grid(vec && even ? BN * tiles_s : ceil_div(n_rows * C, kThreads), kThreads,
+                      "planar_rows");
   if (st) return st;
-  if (vec && C <= 128) {
-    const int64_t tiles_s = ceil_div(S, kPlanarTile);
-    const size_t smem = size_t(kPlanarTile) * size_t(C + 1) * sizeof(float);
+  if (vec) {
+    // channel blocks of about equal width (each at least 4)
+    const int blocks = int(ceil_div(C, kPlanarChannels));
+    const int cmax = int(ceil_div(ceil_div(C, blocks), 4)) * 4;
+    const size_t smem = size_t(kPlanarTile) * size_t((C < cmax ? C : cmax) + 1) * sizeof(float);
+    const dim3 grid(unsigned(BN * tiles_s), unsigned(blocks));
 #define BEVPOOL_PT(K)                                                                          \
   case K:                                                                                      \
-    hipLaunchKernelGGL((planar_tile_kernel<K>), dim3(unsigned(int64_t(BN) * tiles_s)),          \
-                       dim3(kThreads), smem, s, src, C, S, tiles_s, stride_bn, stride_c, rows); \
+    hipLaunchKernelGGL((planar_tile_kernel<K>), grid, dim3(kThreads), smem, s, src, C, cmax, S, \
+                       tiles_s, stride_bn, stride_c, rank, rows);                              \
     break;
-    switch ((C * (kPlanarTile / 4) + kThreads - 1) / kThreads) {
+    switch (ceil_div(int64_t(cmax) * (kPlanarTile / 4), kThreads)) {
       BEVPOOL_PT(1) BEVPOOL_PT(2) BEVPOOL_PT(3) BEVPOOL_PT(4)
       BEVPOOL_PT(5) BEVPOOL_PT(6) BEVPOOL_PT(7) BEVPOOL_PT(8)
       BEVPOOL_PT(9) BEVPOOL_PT(10) BEVPOOL_PT(11) BEVPOOL_PT(12)
       BEVPOOL_PT(13) BEVPOOL_PT(14) BEVPOOL_PT(15) BEVPOOL_PT(16)
       default:
-        return fail(BEVPOOL_EINVAL, "internal: %d channels on the tiled path", C);
+        return fail(BEVPOOL_EINVAL, "internal: %d channels per planar tile", cmax);
     }
 #undef BEVPOOL_PT
-  } else if (vec) {
-    const int64_t tiles_s = ceil_div(S, 256);
-    const int passes = (C + 15) / 16;  // 16-channel passes per thread
-#define BEVPOOL_PR(IT)                                                                         \
-  hipLaunchKernelGGL((planar_rows_kernel<true, IT>), dim3(unsigned(int64_t(BN) * tiles_s)),     \
-                     dim3(kThreads), 0, s, src, C, S, tiles_s, n_rows, stride_bn, stride_c, rows)
-    if (passes <= 1) BEVPOOL_PR(1);
-    else if (passes <= 2) BEVPOOL_PR(2);
-    else if (passes <= 3) BEVPOOL_PR(3);
-    else if (passes <= 5) BEVPOOL_PR(5);
-    else BEVPOOL_PR(4);
-#undef BEVPOOL_PR
   } else {
-    hipLaunchKernelGGL((planar_rows_kernel<false, 1>),
-                       dim3(unsigned(ceil_div(n_rows * C, kThreads))), dim3(kThreads), 0, s, src,
-                       C, S, int64_t(0), n_rows, stride_bn, stride_c, rows);
+    hipLaunchKernelGGL(planar_rows_kernel, dim3(unsigned(ceil_div(n_rows * C, kThreads))),
+                       dim3(kThreads), 0, s, src, C, S, n_rows, stride_bn, stride_c, rows);
   }
   return check_launch("planar_rows");
+}
+
+int bevpool_planar_rows(const float *src, int64_t stride_bn, int64_t stride_c, int32_t BN,
+                        int32_t C, int64_t S, float *rows, void *stream) {
+  g_last_error.clear();
+  return planar_rows_impl(src, stride_bn, stride_c, BN, C, S, nullptr, rows, stream);
+}
+
+int bevpool_planar_kept_rows(const float *src, int64_t stride_bn, int64_t stride_c, int32_t BN,
+                             int32_t C, int64_t S, const int32_t *rank, float *rows,
+                             void *stream) {
+  g_last_error.clear();
+  if (BN > 0 && S > 0 && !rank) return fail(BEVPOOL_EINVAL, "null rank");
+  return planar_rows_impl(src, stride_bn, stride_c, BN, C, S, rank, rows, stream);
 }
 
 int bevpool_context_rows(const float *context, int64_t stride_bn, int64_t stride_c, int32_t BN,
@@ -4603,12 +4577,12 @@ int bevpool_backward_planar(const float *grad, int64_t grad_stride_b, int64_t gr
   if (!scratch || scratch_bytes < bevpool_backward_scratch_bytes(n_cells, C, BEVPOOL_F32))
     return fail(BEVPOOL_ESPACE, "backward scratch too small");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool vec = C % 4 == 0 && S % 4 == 0 && x_stride_bn % 4 == 0 && x_stride_c % 4 == 0 &&
-                   reinterpret_cast<uintptr_t>(x_grad) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(rank) % 16 == 0 &&
-                   reinterpret_cast<uintptr_t>(scratch) % 16 == 0;
+  const bool vec = C >= 4 && S >= 4;
+  const int64_t per_bn = ceil_div(S, 4), n_groups = n_points / S * per_bn;  // groups of 4 points
+  // (sizes that do not divide by 4 keep the limit of one element per thread)
+  const bool even = C % 4 == 0 && S % 4 == 0 && x_stride_bn % 4 == 0 && x_stride_c % 4 == 0;
   int st;
-  if ((st = check_grid(vec ? ceil_div(n_points / 4, kThreads) + kXcds
+  if ((st = check_grid(vec && even ? ceil_div(n_groups, kThreads) + kXcds
                            : ceil_div(n_points * C, kThreads),
                        kThreads, "gather_planar")))
     return st;
@@ -4617,18 +4591,16 @@ int bevpool_backward_planar(const float *grad, int64_t grad_stride_b, int64_t gr
     return st;
   const float *g = static_cast<const float *>(scratch);
   LaunchTimer t("gather_planar", s);
-  if (vec) {
-    const unsigned grid = xcd_grid(ceil_div(n_points / 4, kThreads));
-#ifndef BEVPOOL_GP_IT
-#define BEVPOOL_GP_IT 2
-#endif
-    hipLaunchKernelGGL((gather_planar_kernel<true, BEVPOOL_GP_IT>), dim3(grid), dim3(kThreads),
-                       0, s, g, C, rank, n_points, S, x_stride_bn, x_stride_c, x_grad);
-  } else {
-    hipLaunchKernelGGL((gather_planar_kernel<false, 1>),
-                       dim3(unsigned(ceil_div(n_points * C, kThreads))), dim3(kThreads), 0, s, g,
-                       C, rank, n_points, S, x_stride_bn, x_stride_c, x_grad);
-  }
+  const FastDiv groups = make_fast_div(uint32_t(per_bn));
+  const bool past_caches = even && reinterpret_cast<uintptr_t>(x_grad) % 16 == 0;
+#define BEVPOOL_GP(VEC, STREAM, BLOCKS)                                                        \
+  hipLaunchKernelGGL((gather_planar_kernel<VEC, STREAM>), dim3(BLOCKS), dim3(kThreads), 0, s, g, \
+                     C, rank, n_points, S, groups, n_groups, x_stride_bn, x_stride_c, x_grad)
+  const unsigned group_blocks = xcd_grid(ceil_div(n_groups, kThreads));
+  if (vec && past_caches) BEVPOOL_GP(true, true, group_blocks);
+  else if (vec) BEVPOOL_GP(true, false, group_blocks);
+  else BEVPOOL_GP(false, false, unsigned(ceil_div(n_points * C, kThreads)));
+#undef BEVPOOL_GP
   return check_launch("gather_planar");
 }
 
@@ -4803,7 +4775,10 @@ int bevpool_backward(const void *grad, int32_t dtype, int64_t grad_stride_b,
   const int64_t total = n_points * vpr;
   const int64_t gather_blocks = ceil_div(total, int64_t(kThreads));
   int st;
-  if ((st = check_grid(gather_blocks + kXcds, kThreads, "gather_rows"))) return st;
+  // (rows that are no run of aligned pieces keep the limit of one element per thread)
+  if ((st = check_grid((aligned ? gather_blocks : ceil_div(n_points * C, kThreads)) + kXcds,
+                       kThreads, "gather_rows")))
+    return st;
   const unsigned grid = xcd_grid(gather_blocks);
   const bool narrow = total < (int64_t(1) << 32);
   // cache warm-up (gather_warm_block): ranks per XCD + occupied rows

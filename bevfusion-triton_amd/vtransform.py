@@ -81,19 +81,20 @@ class _LSSBevPool(torch.autograd.Function):
         B, N, D, fH, fW, C = x.shape
         X, Y, Z = nx
         planar = planar_layout(x) if x.numel() else None
-        if planar is not None:
-            # channel-first storage: one transposing kernel instead of the
-            # reshape copy of base.py:136; the gradient goes back planar
-            sbn, sc, S = planar
-            x2 = P.planar_rows(x.as_strided((B * N, C, S), (sbn, sc, 1)))
-        else:
-            x2 = x.reshape(B * N * D * fH * fW, C)
-            if x2.stride(1) != 1 and x2.shape[0]:
-                x2 = x2.contiguous()
         if index is None:
             idx = P.index_from_geom(geom_feats.reshape(-1, 3), B, offset, dx, nx)
         else:
             idx = index
+        if planar is not None:
+            # channel-first storage: one transposing kernel for the kept points'
+            # rows instead of the reshape copy of base.py:136; the gradient
+            # goes back planar
+            sbn, sc, S = planar
+            x2 = P.planar_rows(x.as_strided((B * N, C, S), (sbn, sc, 1)), idx.rank)
+        else:
+            x2 = x.reshape(B * N * D * fH * fW, C)
+            if x2.stride(1) != 1 and x2.shape[0]:
+                x2 = x2.contiguous()
         out = torch.empty((B, Z * C, X, Y), dtype=torch.float32, device=x.device)
         # element (b, c, z, xy) of the (B, C, Dz, H, W) pool at channel z*C + c
         P.forward(idx, x2, out, Z * C * X * Y, X * Y, C * X * Y)

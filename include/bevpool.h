@@ -264,11 +264,19 @@ int bevpool_backward(const void *grad, int32_t dtype, int64_t grad_stride_b,
 
 /*
  * Planar (BN, C, S) fp32 -> rows [BN*S, C] fp32 (the copy of base.py:136,
- * as one transposing kernel).  Any strides; the fast form needs C, S and both
- * strides multiples of 4 and 16-byte aligned pointers.
+ * as one transposing kernel).  Any strides and alignment of the elements.
  */
 int bevpool_planar_rows(const float *src, int64_t stride_bn, int64_t stride_c, int32_t BN,
                         int32_t C, int64_t S, float *rows, void *stream);
+
+/*
+ * The same for rows that only kept points are read from (bevpool_forward on
+ * the ranks' index): with rank int32 [BN*S], rows of dropped points (rank -1)
+ * may be left unwritten.
+ */
+int bevpool_planar_kept_rows(const float *src, int64_t stride_bn, int64_t stride_c, int32_t BN,
+                             int32_t C, int64_t S, const int32_t *rank, float *rows,
+                             void *stream);
 
 /*
  * Backward of the pooling straight into a planar fp32 gradient:
