@@ -28,6 +28,10 @@ def require_gpu(*tensors) -> None:
             )
 
 
+def _align256(nbytes: int) -> int:
+    return (nbytes + 255) & ~255
+
+
 class PoolIndex:
     """Device-resident index of one pooling call.
 
@@ -36,28 +40,68 @@ class PoolIndex:
     cell_start  int32 (n_cells,)   sorted range [start, end) of each cell
     cell_end    int32 (n_cells,)
     meta        int32 (8,)         device counters (n_kept, n_intervals, ...)
+
+    The five lie in one buffer (one allocation per call); the attributes are
+    views made when asked for, the calls take the addresses of
+    :meth:`pointers`.
     """
 
-    __slots__ = ('rank', 'keys', 'cell_start', 'cell_end', 'meta', 'n_points', 'B', 'D', 'H',
-                 'W', 'device')
+    __slots__ = ('buf', 'offsets', 'n_points', 'B', 'D', 'H', 'W', 'device')
 
     def __init__(self, n_points, B, D, H, W, device):
         self.n_points, self.B, self.D, self.H, self.W = int(n_points), int(B), int(D), int(H), int(W)
         self.device = device
-        n_cells = self.n_cells
-        self.rank = torch.empty(self.n_points, dtype=torch.int32, device=device)
-        self.keys = torch.empty(self.n_points, dtype=torch.int64, device=device)
-        self.cell_start = torch.empty(n_cells, dtype=torch.int32, device=device)
-        self.cell_end = torch.empty(n_cells, dtype=torch.int32, device=device)
-        self.meta = torch.empty(L.META_LEN, dtype=torch.int32, device=device)
+        cells = self.n_cells
+        rank = _align256(4 * L.META_LEN)
+        keys = rank + _align256(4 * self.n_points)
+        start = keys + _align256(8 * self.n_points)
+        end = start + _align256(4 * cells)
+        self.offsets = (rank, keys, start, end, 0)
+        self.buf = torch.empty(end + _align256(4 * cells), dtype=torch.uint8, device=device)
 
     @property
     def n_cells(self) -> int:
         return self.B * self.D * self.H * self.W
 
+    def pointers(self):
+        """Addresses of (rank, keys, cell_start, cell_end, meta)."""
+        base = self.buf.data_ptr()
+        return tuple(base + o for o in self.offsets)
+
+    def _view(self, which: int, count: int, dtype):
+        o = self.offsets[which]
+        return self.buf[o:o + count * dtype.itemsize].view(dtype)
+
+    @property
+    def rank(self):
+        return self._view(0, self.n_points, torch.int32)
+
+    @property
+    def keys(self):
+        return self._view(1, self.n_points, torch.int64)
+
+    @property
+    def cell_start(self):
+        return self._view(2, self.n_cells, torch.int32)
+
+    @property
+    def cell_end(self):
+        return self._view(3, self.n_cells, torch.int32)
+
+    @property
+    def meta(self):
+        return self._view(4, L.META_LEN, torch.int32)
+
     def workspace(self):
         nbytes = L.library().bevpool_index_workspace_bytes(self.n_points, self.n_cells)
         return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=self.device)
+
+
+def _grid_args(offset, dx, nx):
+    """(offset, dx, nx) as the C arrays of the quantisation calls."""
+    off = np.ascontiguousarray(offset, dtype=np.float32)
+    d = np.ascontiguousarray(dx, dtype=np.float32)
+    return L._f3.from_buffer_copy(off), L._f3.from_buffer_copy(d), L._i3(*nx)
 
 
 def _check_sizes(n_points: int, n_cells: int) -> None:
@@ -68,12 +112,10 @@ def _check_sizes(n_points: int, n_cells: int) -> None:
 
 
 def _sort(idx: PoolIndex, ws, stream) -> None:
-    lib = L.library()
+    rank, keys, start, end, meta = idx.pointers()
     L.check(
-        lib.bevpool_sort(
-            L.ptr(idx.rank), idx.n_points, idx.n_cells, L.ptr(idx.keys), L.ptr(idx.cell_start),
-            L.ptr(idx.cell_end), L.ptr(idx.meta), L.ptr(ws), ws.numel(), stream,
-        ),
+        L.library().bevpool_sort(rank, idx.n_points, idx.n_cells, keys, start, end, meta,
+                                 L.ptr(ws), ws.numel(), stream),
         'bevpool_sort',
     )
 
@@ -101,11 +143,8 @@ def index_from_geom(geom2d, B: int, offset, dx, nx) -> PoolIndex:
     idx = PoolIndex(n_points, B, nx[2], nx[0], nx[1], geom2d.device)
     ws = idx.workspace()
     stream = L.stream_handle(geom2d.device)
-    lib = L.library()
-    off = np.asarray(offset, dtype=np.float32)
-    d = np.asarray(dx, dtype=np.float32)
     with torch.cuda.device(geom2d.device):
-        _quantize(lib, geom2d, n_points, B, off, d, nx, idx, ws, stream)
+        _quantize(L.library(), geom2d, n_points, B, offset, dx, nx, idx, ws, stream)
         _sort(idx, ws, stream)
     return idx
 
@@ -137,15 +176,12 @@ def index_from_cameras(frustum, mats, B: int, N: int, offset, dx, nx) -> PoolInd
     idx = PoolIndex(n_points, B, nx[2], nx[0], nx[1], frustum.device)
     ws = idx.workspace()
     stream = L.stream_handle(frustum.device)
-    lib = L.library()
-    off = np.asarray(offset, dtype=np.float32)
-    d = np.asarray(dx, dtype=np.float32)
+    rank, _, _, _, meta = idx.pointers()
     with torch.cuda.device(frustum.device):
         L.check(
-            lib.bevpool_quantize_cameras(
+            L.library().bevpool_quantize_cameras(
                 L.ptr(frustum), D, fH, fW, *[L.ptr(m) for m in flat], N, B,
-                L._f3(*[float(v) for v in off]), L._f3(*[float(v) for v in d]), L._i3(*nx),
-                L.ptr(idx.rank), L.ptr(idx.meta), L.ptr(ws), ws.numel(), stream,
+                *_grid_args(offset, dx, nx), rank, meta, L.ptr(ws), ws.numel(), stream,
             ),
             'bevpool_quantize_cameras',
         )
@@ -153,13 +189,13 @@ def index_from_cameras(frustum, mats, B: int, N: int, offset, dx, nx) -> PoolInd
     return idx
 
 
-def _quantize(lib, geom2d, n_points, B, off, d, nx, idx, ws, stream):
+def _quantize(lib, geom2d, n_points, B, offset, dx, nx, idx, ws, stream):
+    rank, _, _, _, meta = idx.pointers()
     L.check(
         lib.bevpool_quantize_geom(
             L.ptr(geom2d), n_points, geom2d.stride(0) if n_points else 3,
-            max(1, n_points // B), B,
-            L._f3(*[float(v) for v in off]), L._f3(*[float(v) for v in d]), L._i3(*nx),
-            L.ptr(idx.rank), L.ptr(idx.meta), L.ptr(ws), ws.numel(), stream,
+            max(1, n_points // B), B, *_grid_args(offset, dx, nx), rank, meta, L.ptr(ws),
+            ws.numel(), stream,
         ),
         'bevpool_quantize_geom',
     )
@@ -184,10 +220,11 @@ def index_from_coords(coords, B: int, D: int, H: int, W: int) -> PoolIndex:
 
 
 def _coord_ranks(coords, n_points, B, D, H, W, idx, ws, stream):
+    rank, _, _, _, meta = idx.pointers()
     L.check(
         L.library().bevpool_coord_ranks(
             L.ptr(coords), coords.element_size(), n_points, coords.stride(0) if n_points else 4,
-            B, D, H, W, L.ptr(idx.rank), L.ptr(idx.meta), L.ptr(ws), ws.numel(), stream,
+            B, D, H, W, rank, meta, L.ptr(ws), ws.numel(), stream,
         ),
         'bevpool_coord_ranks',
     )
@@ -229,10 +266,10 @@ def intervals(idx: PoolIndex):
 
 
 def _intervals(idx, n, starts, lengths, cells, ws):
+    _, keys, _, end, meta = idx.pointers()
     L.check(
         L.library().bevpool_intervals(
-            L.ptr(idx.keys), n, L.ptr(idx.cell_end), L.ptr(starts), L.ptr(lengths), L.ptr(cells),
-            L.ptr(idx.meta), L.ptr(ws), ws.numel(), L.stream_handle(idx.device),
+            keys, n, end, L.ptr(starts), L.ptr(lengths), L.ptr(cells), meta, L.ptr(ws), ws.numel(), L.stream_handle(idx.device),
         ),
         'bevpool_intervals',
     )
@@ -253,11 +290,11 @@ def forward(idx: PoolIndex, feats2d, out, stride_b: int, stride_c: int, stride_z
 
 
 def _forward_call(lib, idx, feats2d, dtype, C, out, stride_b, stride_c, stride_z, scratch):
+    _, keys, start, end, meta = idx.pointers()
     L.check(
         lib.bevpool_forward(
             L.ptr(feats2d), dtype, feats2d.stride(0) if idx.n_points else C, C, idx.n_points,
-            L.ptr(idx.keys), L.ptr(idx.cell_start), L.ptr(idx.cell_end), L.ptr(idx.meta), idx.B,
-            idx.D, idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out), L.ptr(scratch),
+            keys, start, end, meta, idx.B, idx.D, idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out), L.ptr(scratch),
             scratch.numel(), L.stream_handle(idx.device),
         ),
         'bevpool_forward',
@@ -276,11 +313,11 @@ def backward(idx: PoolIndex, grad, C: int, stride_b: int, stride_c: int, stride_
 
 
 def _backward_call(lib, idx, grad, dtype, C, stride_b, stride_c, stride_z, x_grad, scratch):
+    rank, _, start, end, _ = idx.pointers()
     L.check(
         lib.bevpool_backward(
-            L.ptr(grad), dtype, stride_b, stride_c, stride_z, C, L.ptr(idx.rank), idx.n_points,
-            L.ptr(idx.cell_start), L.ptr(idx.cell_end), idx.B, idx.D, idx.H * idx.W,
-            L.ptr(x_grad), x_grad.stride(0) if idx.n_points else C, 1, L.ptr(scratch),
+            L.ptr(grad), dtype, stride_b, stride_c, stride_z, C, rank, idx.n_points, start, end,
+            idx.B, idx.D, idx.H * idx.W, L.ptr(x_grad), x_grad.stride(0) if idx.n_points else C, 1, L.ptr(scratch),
             scratch.numel(), L.stream_handle(idx.device),
         ),
         'bevpool_backward',
@@ -289,9 +326,9 @@ def _backward_call(lib, idx, grad, dtype, C, stride_b, stride_c, stride_z, x_gra
 
 # ---- depth-weighted (fused depth x context) pooling -------------------------
 
-def planar_rows(src3d, rank=None):
+def planar_rows(src3d, idx=None):
     """(BN, C, S) fp32 planar tensor (S contiguous, any batch/channel strides)
-    -> (BN*S, C) channel-last rows.  With the points' ``rank``, the rows of
+    -> (BN*S, C) channel-last rows.  With the points' index, the rows of
     dropped points are left undefined (nothing reads them)."""
     BN, C, S = src3d.shape
     if src3d.stride(2) != 1:
@@ -301,10 +338,10 @@ def planar_rows(src3d, rank=None):
     lib = L.library()
     with torch.cuda.device(src3d.device):
         stream = L.stream_handle(src3d.device)
-        if rank is None:
+        if idx is None:
             L.check(lib.bevpool_planar_rows(*src, L.ptr(rows), stream), 'bevpool_planar_rows')
         else:
-            L.check(lib.bevpool_planar_kept_rows(*src, L.ptr(rank), L.ptr(rows), stream),
+            L.check(lib.bevpool_planar_kept_rows(*src, idx.pointers()[0], L.ptr(rows), stream),
                     'bevpool_planar_kept_rows')
     return rows
 
@@ -320,11 +357,12 @@ def backward_planar(idx: PoolIndex, grad, C: int, stride_b: int, stride_c: int, 
     lib = L.library()
     scratch_bytes = lib.bevpool_backward_scratch_bytes(idx.n_cells, C, L.F32)
     scratch = torch.empty(max(int(scratch_bytes), 256), dtype=torch.uint8, device=idx.device)
+    rank, _, start, end, _ = idx.pointers()
     with torch.cuda.device(idx.device):
         L.check(
             lib.bevpool_backward_planar(
-                L.ptr(grad), stride_b, stride_c, stride_z, C, L.ptr(idx.rank), idx.n_points,
-                L.ptr(idx.cell_start), L.ptr(idx.cell_end), idx.B, idx.D, idx.H * idx.W, S,
+                L.ptr(grad), stride_b, stride_c, stride_z, C, rank, idx.n_points, start, end,
+                idx.B, idx.D, idx.H * idx.W, S,
                 L.ptr(x_grad3d), x_grad3d.stride(0), x_grad3d.stride(1), L.ptr(scratch),
                 scratch.numel(), L.stream_handle(idx.device),
             ),
@@ -339,12 +377,12 @@ def forward_depth(idx: PoolIndex, depth_flat, rows, D: int, HW: int, out, stride
     lib = L.library()
     scratch_bytes = lib.bevpool_forward_scratch_bytes(idx.n_cells, C)
     scratch = torch.empty(max(int(scratch_bytes), 256), dtype=torch.uint8, device=idx.device)
+    _, keys, start, end, meta = idx.pointers()
     with torch.cuda.device(idx.device):
         L.check(
             lib.bevpool_forward_depth(
-                L.ptr(depth_flat), L.ptr(rows), C, idx.n_points, D, HW, L.ptr(idx.keys),
-                L.ptr(idx.cell_start), L.ptr(idx.cell_end), L.ptr(idx.meta), idx.B, idx.D,
-                idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out), L.ptr(scratch),
+                L.ptr(depth_flat), L.ptr(rows), C, idx.n_points, D, HW, keys, start, end, meta,
+                idx.B, idx.D, idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out), L.ptr(scratch),
                 scratch.numel(), L.stream_handle(idx.device),
             ),
             'bevpool_forward_depth',
@@ -357,12 +395,12 @@ def backward_depth(idx: PoolIndex, grad, C: int, stride_b: int, stride_c: int, s
     lib = L.library()
     scratch_bytes = lib.bevpool_backward_scratch_bytes(idx.n_cells, C, L.F32)
     scratch = torch.empty(max(int(scratch_bytes), 256), dtype=torch.uint8, device=idx.device)
+    rank, _, start, end, _ = idx.pointers()
     with torch.cuda.device(idx.device):
         L.check(
             lib.bevpool_backward_depth_image(
-                L.ptr(grad), stride_b, stride_c, stride_z, C, L.ptr(idx.rank), idx.n_points, D,
-                fH, fW, L.ptr(depth_flat), L.ptr(rows), L.ptr(idx.cell_start),
-                L.ptr(idx.cell_end), idx.B, idx.D, idx.H * idx.W, L.ptr(grad_depth),
+                L.ptr(grad), stride_b, stride_c, stride_z, C, rank, idx.n_points, D, fH, fW,
+                L.ptr(depth_flat), L.ptr(rows), start, end, idx.B, idx.D, idx.H * idx.W, L.ptr(grad_depth),
                 L.ptr(grad_context3d), grad_context3d.stride(0), grad_context3d.stride(1),
                 L.ptr(scratch), scratch.numel(), L.stream_handle(idx.device),
             ),

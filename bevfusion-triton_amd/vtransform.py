@@ -90,7 +90,7 @@ class _LSSBevPool(torch.autograd.Function):
             # rows instead of the reshape copy of base.py:136; the gradient
             # goes back planar
             sbn, sc, S = planar
-            x2 = P.planar_rows(x.as_strided((B * N, C, S), (sbn, sc, 1)), idx.rank)
+            x2 = P.planar_rows(x.as_strided((B * N, C, S), (sbn, sc, 1)), idx)
         else:
             x2 = x.reshape(B * N * D * fH * fW, C)
             if x2.stride(1) != 1 and x2.shape[0]:
