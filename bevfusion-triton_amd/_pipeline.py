@@ -49,7 +49,8 @@ class PoolIndex:
     __slots__ = ('buf', 'offsets', 'n_points', 'B', 'D', 'H', 'W', 'device')
 
     def __init__(self, n_points, B, D, H, W, device):
-        self.n_points, self.B, self.D, self.H, self.W = int(n_points), int(B), int(D), int(H), int(W)
+        self.n_points = int(n_points)
+        self.B, self.D, self.H, self.W = int(B), int(D), int(H), int(W)
         self.device = device
         cells = self.n_cells
         rank = _align256(4 * L.META_LEN)
@@ -269,7 +270,8 @@ def _intervals(idx, n, starts, lengths, cells, ws):
     _, keys, _, end, meta = idx.pointers()
     L.check(
         L.library().bevpool_intervals(
-            keys, n, end, L.ptr(starts), L.ptr(lengths), L.ptr(cells), meta, L.ptr(ws), ws.numel(), L.stream_handle(idx.device),
+            keys, n, end, L.ptr(starts), L.ptr(lengths), L.ptr(cells), meta, L.ptr(ws), ws.numel(),
+            L.stream_handle(idx.device),
         ),
         'bevpool_intervals',
     )
@@ -294,8 +296,8 @@ def _forward_call(lib, idx, feats2d, dtype, C, out, stride_b, stride_c, stride_z
     L.check(
         lib.bevpool_forward(
             L.ptr(feats2d), dtype, feats2d.stride(0) if idx.n_points else C, C, idx.n_points,
-            keys, start, end, meta, idx.B, idx.D, idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out), L.ptr(scratch),
-            scratch.numel(), L.stream_handle(idx.device),
+            keys, start, end, meta, idx.B, idx.D, idx.H * idx.W, stride_b, stride_c, stride_z,
+            L.ptr(out), L.ptr(scratch), scratch.numel(), L.stream_handle(idx.device),
         ),
         'bevpool_forward',
     )
@@ -317,8 +319,8 @@ def _backward_call(lib, idx, grad, dtype, C, stride_b, stride_c, stride_z, x_gra
     L.check(
         lib.bevpool_backward(
             L.ptr(grad), dtype, stride_b, stride_c, stride_z, C, rank, idx.n_points, start, end,
-            idx.B, idx.D, idx.H * idx.W, L.ptr(x_grad), x_grad.stride(0) if idx.n_points else C, 1, L.ptr(scratch),
-            scratch.numel(), L.stream_handle(idx.device),
+            idx.B, idx.D, idx.H * idx.W, L.ptr(x_grad), x_grad.stride(0) if idx.n_points else C, 1,
+            L.ptr(scratch), scratch.numel(), L.stream_handle(idx.device),
         ),
         'bevpool_backward',
     )
@@ -382,8 +384,8 @@ def forward_depth(idx: PoolIndex, depth_flat, rows, D: int, HW: int, out, stride
         L.check(
             lib.bevpool_forward_depth(
                 L.ptr(depth_flat), L.ptr(rows), C, idx.n_points, D, HW, keys, start, end, meta,
-                idx.B, idx.D, idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out), L.ptr(scratch),
-                scratch.numel(), L.stream_handle(idx.device),
+                idx.B, idx.D, idx.H * idx.W, stride_b, stride_c, stride_z, L.ptr(out),
+                L.ptr(scratch), scratch.numel(), L.stream_handle(idx.device),
             ),
             'bevpool_forward_depth',
         )
@@ -400,9 +402,10 @@ def backward_depth(idx: PoolIndex, grad, C: int, stride_b: int, stride_c: int, s
         L.check(
             lib.bevpool_backward_depth_image(
                 L.ptr(grad), stride_b, stride_c, stride_z, C, rank, idx.n_points, D, fH, fW,
-                L.ptr(depth_flat), L.ptr(rows), start, end, idx.B, idx.D, idx.H * idx.W, L.ptr(grad_depth),
-                L.ptr(grad_context3d), grad_context3d.stride(0), grad_context3d.stride(1),
-                L.ptr(scratch), scratch.numel(), L.stream_handle(idx.device),
+                L.ptr(depth_flat), L.ptr(rows), start, end, idx.B, idx.D, idx.H * idx.W,
+                L.ptr(grad_depth), L.ptr(grad_context3d), grad_context3d.stride(0),
+                grad_context3d.stride(1), L.ptr(scratch), scratch.numel(),
+                L.stream_handle(idx.device),
             ),
             'bevpool_backward_depth_image',
         )
