@@ -482,10 +482,10 @@ int bevpool_op_backward(const void *grad, int32_t dtype, int64_t grad_stride_b,
  * Differences from the reference: an interval whose rows or cell fall outside
  * the arrays is skipped and counted in meta[BEVPOOL_META_N_BAD] (meta may be
  * NULL) instead of reading/writing out of bounds.  The backward also uses
- * meta[4]: intervals that are in order and do not overlap let it write every
- * row once, without the zero fill; it fills first when they are not, when
- * meta is NULL or when meta[4] comes in as anything but zero.  The interval
- * count is
+ * meta[4]: intervals that are in order, do not overlap and leave no gap of
+ * more than 4096 rows let it write every row once, without the zero fill; it
+ * fills first when they are not, when meta is NULL or when meta[4] comes in
+ * as anything but zero.  The interval count is
  * n_intervals, or, when n_intervals_dev is not NULL, min(n_intervals,
  * *n_intervals_dev) read on the device (capacity + device count, so a caller
  * chaining bevpool_runs needs no host synchronisation).  The caller passes

@@ -228,3 +228,24 @@ def test_ext_module_interval_lengths(pkg, cuda, C, order):
     if bad:
         with pytest.raises(RuntimeError, match='bev_pool_backward: 1 intervals'):
             pkg.check_errors()
+
+
+@pytest.mark.parametrize('gap', [4095, 4096, 4097, 40000])
+@pytest.mark.parametrize('where', ['first', 'middle', 'last'])
+def test_ext_module_long_gaps(pkg, cuda, where, gap):
+    """Gaps around the longest that the backward writes with its intervals
+    (longer ones are left to the zero fill): every row of them is zero."""
+    g = torch.Generator().manual_seed(gap)
+    lengths = torch.tensor([3, 20, 1, 300], dtype=torch.int32)
+    gaps = torch.tensor([gap if where == 'first' else 2, 0, gap if where == 'middle' else 0, 1],
+                        dtype=torch.int32)
+    ends = (lengths + gaps).cumsum(0).int()
+    starts, n = ends - lengths, int(ends[-1]) + (gap if where == 'last' else 0)
+    coords = torch.zeros((n, 4), dtype=torch.int32)
+    coords[starts.long(), 1] = torch.arange(4, dtype=torch.int32)
+    up = torch.randn((1, 1, 1, 4, 20), generator=g)
+    torch.full((n, 20), float('nan'), device=cuda)  # what a freed block may hold
+    xg = pkg.legacy.ext_module.bev_pool_backward(up.to(cuda), coords.to(cuda), lengths.to(cuda),
+                                                 starts.to(cuda), 1, 1, 1, 4)
+    exp = ref.legacy_backward(up, coords, lengths, starts, 1, 1, 1, 4)[0]
+    assert_bit_equal(xg, exp, 'backward')
