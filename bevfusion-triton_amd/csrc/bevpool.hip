@@ -71,8 +71,13 @@
 #include <vector>
 
 #include "bevpool.h"
+#include "channel_blocks.h"
 
 namespace {
+
+using channel_blocks::kTileChannels;
+using channel_blocks::first_channel;
+using channel_blocks::tile_channels;
 
 // ---------------------------------------------------------------------------
 // constants
@@ -93,7 +98,6 @@ inline int sort_items(int64_t n_points) {
 constexpr int kMaxDigitBits = 10;
 constexpr int kMaxRadix = 1 << kMaxDigitBits;
 constexpr int kCellTile = 64;              // cells per transpose tile
-constexpr int kTileChannels = 128;         // max channels per transpose pass
 
 // 16- and 8-byte integer vectors.  HIP's uint4 struct blocks register
 // promotion.  Float vectors are avoided on purpose: with packed fp32 ops
@@ -2495,10 +2499,11 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
     __syncthreads();
   }
   const uint16_t *acch = reinterpret_cast<const uint16_t *>(acc);
-  for (int c0 = 0; c0 < C; c0 += CT) {
+  constexpr uint32_t kPer = kRaw16 ? 8 : 4;  // channels per 16-byte piece
+  for (int cn = 0; cn < C; cn += CT) {
+    const int c0 = first_channel(C, kVecRow ? int(kPer) : 1, cn);
     const int cb = C - c0 < CT ? C - c0 : CT;
     if (kVecRow) {
-      constexpr uint32_t kPer = kRaw16 ? 8 : 4;  // channels per 16-byte piece
       const uint32_t q = (uint32_t(cb) + kPer - 1) / kPer;  // 16-byte pieces per row
       const uint32_t last = uint32_t(cb) - kPer;            // first channel of the last one
       const uint32_t n_items = kCellTile * q;
@@ -2515,7 +2520,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
         v[it] = ((occm >> t) & 1) ? reinterpret_cast<const Bytes16 *>(src)->v
                                   : u32x4{0u, 0u, 0u, 0u};
       }
-      if (c0 == 0 && tid < kCellTile) {
+      if (cn == 0 && tid < kCellTile) {
         occ[tid] = occ_mine;
         off[tid] = off_mine;
       }
@@ -2646,7 +2651,8 @@ __global__ __launch_bounds__(kThreads) void bev_to_rows_kernel(
   // are they 4 consecutive elements of a channel?
   const bool run =
       kVecBev || (cell0 + j + 3 < n_cells && cell_offset(uint32_t(cell0 + j + 3)) == offj + 3);
-  for (int c0 = 0; c0 < C; c0 += CT) {
+  for (int cn = 0; cn < C; cn += CT) {
+    const int c0 = first_channel(C, kVecRow ? kPer : 1, cn);
     const int cb = C - c0 < CT ? C - c0 : CT;
     using V = typename std::conditional<sizeof(TR) == 4, u32x4, u32x2>::type;
     using VA = typename std::conditional<sizeof(TR) == 4, Bytes16, Bytes8>::type;
@@ -2685,7 +2691,7 @@ __global__ __launch_bounds__(kThreads) void bev_to_rows_kernel(
     }
     // the cells' occupancy, loaded after the gradient loads so that one
     // round trip brings both
-    if (!occ_first && c0 == 0 && tid < kCellTile)
+    if (!occ_first && cn == 0 && tid < kCellTile)
       occ[tid] = cell0 + tid < n_cells && cend[cell0 + tid] != 0 ? 1 : 0;
 #pragma unroll
     for (int it = 0; it < kTileSlots; ++it) {
@@ -3839,14 +3845,6 @@ int launch_accum_group(int32_t dtype, const GroupPlan &g, const char *x, int64_t
 #undef BEVPOOL_AG_K
 #undef BEVPOOL_AG
   return check_launch("accum_group");
-}
-
-// Channels per transpose pass: at most kTileChannels, the passes about equal
-// (so that the last one too holds a whole 16-byte piece) and multiples of 8.
-int tile_channels(int C) {
-  const int passes = (C + kTileChannels - 1) / kTileChannels;
-  const int per = ((C + passes - 1) / passes + 7) / 8 * 8;
-  return C < per ? C : per;
 }
 
 // cell-major fp32 rows -> channel-first output (zeros for empty cells).

@@ -98,3 +98,22 @@ def test_odd_planes(pkg, cuda, grid, C, dtype):
     assert_bit_equal(out, ref.bev_pool(feats.float(), coords, B, D, H, W).to(dtype), 'forward')
     x, y, z, b = coords.unbind(1)
     assert_bit_equal(grad, up[b, :, z, x, y], 'backward')
+
+
+@pytest.mark.parametrize('grid', [(2, 1, 13, 11), (2, 2, 8, 16)])
+@pytest.mark.parametrize('C,dtype', [(1921, F32), (1923, F32), (2049, F32), (1921, F16),
+                                     (1927, BF16), (2055, F16)])
+def test_wide_rows(pkg, cuda, grid, C, dtype):
+    """Rows whose last transpose pass would hold fewer channels than a 16-byte
+    piece, every cell occupied (what one cell's row spills into is another's)."""
+    B, D, H, W = grid
+    cells = B * D * H * W
+    g = torch.Generator().manual_seed(C)
+    rank = torch.cat((torch.arange(cells), torch.randint(cells, (300,), generator=g)))
+    rank = rank[torch.randperm(rank.numel(), generator=g)]
+    b, z, x, y = (t for t in torch.unravel_index(rank, grid))
+    coords = torch.stack((x, y, z, b), 1).to(torch.int32)
+    feats = torch.randn((rank.numel(), C), generator=g).to(dtype)
+    out, grad, up = run_op(pkg, feats, coords, grid, cuda)
+    assert_bit_equal(out, ref.bev_pool(feats.float(), coords, *grid).to(dtype), 'forward')
+    assert_bit_equal(grad, up.to(dtype)[b, :, z, x, y], 'backward')
