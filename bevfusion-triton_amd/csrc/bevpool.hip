@@ -77,6 +77,8 @@ namespace {
 
 using channel_blocks::kTileChannels;
 using channel_blocks::first_channel;
+using channel_blocks::planar_blocks;
+using channel_blocks::planar_channels;
 using channel_blocks::tile_channels;
 
 // ---------------------------------------------------------------------------
@@ -3259,8 +3261,8 @@ __device__ __forceinline__ void store16(float *p, u32x4 v) {
 }
 
 // planar -> rows (BN*S, C), fp32, for C >= 4 and S >= 4 of any alignment: a
-// block moves kPlanarTile consecutive s of one bn and at most kPlanarChannels
-// channels through an LDS tile [s][channel] (<= 66 KB).  Each group of
+// block moves kPlanarTile consecutive s of one bn and a block of channels
+// (planar_channels) through an LDS tile [s][channel] (<= 66 KB).  Each group of
 // kPlanarTile / 4 lanes loads kPlanarTile * 4 contiguous bytes of one channel
 // (kPer 16-byte loads per thread, all issued before the tile is written);
 // after one barrier the block writes its rows, 16 bytes per thread,
@@ -3277,7 +3279,7 @@ __device__ __forceinline__ void store16(float *p, u32x4 v) {
 // us, and with four height bins, where 46% are dropped, 183 us.  Maps that 4
 // does not divide (2 x 6 x 45 x 29 x 51 points, C = 64): 80 us, 244 one element
 // per thread (and the planar gradient 42 us, 155).
-constexpr int kPlanarTile = 128, kPlanarChannels = 128;
+constexpr int kPlanarTile = 128;
 template <int kPer>
 __global__ __launch_bounds__(kThreads) void planar_tile_kernel(
     const float *__restrict__ src, int C, int cmax, int64_t S, int64_t tiles_s, int64_t sbn,
@@ -3286,7 +3288,8 @@ __global__ __launch_bounds__(kThreads) void planar_tile_kernel(
   extern __shared__ float tile[];  // [kPlanarTile][cb + 1]
   __shared__ int s_rank[kPlanarTile];
   const int tid = threadIdx.x;
-  const int c0 = int(blockIdx.y) * cmax, cb = C - c0 < cmax ? C - c0 : cmax;
+  const int c0 = first_channel(C, 4, int(blockIdx.y) * cmax);
+  const int cb = C - c0 < cmax ? C - c0 : cmax;
   const int pitch = cb + 1;
   const int64_t bn = int64_t(blockIdx.x) / tiles_s;
   const int np = S < kPlanarTile ? int(S) : kPlanarTile;
@@ -4519,11 +4522,9 @@ static int planar_rows_impl(const float *src, int64_t stride_bn, int64_t stride_
                       "planar_rows");
   if (st) return st;
   if (vec) {
-    // channel blocks of about equal width (each at least 4)
-    const int blocks = int(ceil_div(C, kPlanarChannels));
-    const int cmax = int(ceil_div(ceil_div(C, blocks), 4)) * 4;
-    const size_t smem = size_t(kPlanarTile) * size_t((C < cmax ? C : cmax) + 1) * sizeof(float);
-    const dim3 grid(unsigned(BN * tiles_s), unsigned(blocks));
+    const int cmax = planar_channels(C);
+    const size_t smem = size_t(kPlanarTile) * size_t(cmax + 1) * sizeof(float);
+    const dim3 grid(unsigned(BN * tiles_s), unsigned(planar_blocks(C)));
 #define BEVPOOL_PT(K)                                                                          \
   case K:                                                                                      \
     hipLaunchKernelGGL((planar_tile_kernel<K>), grid, dim3(kThreads), smem, s, src, C, cmax, S, \

@@ -15,6 +15,18 @@ constexpr int tile_channels(int C) {
   return C < per ? C : per;
 }
 
+// Most channels that a block of the planar transpose stages in LDS, and the
+// channels per block of C: about equal and multiples of 4.  (The last one may
+// be left with any width from 1.)
+constexpr int kPlanarChannels = 128;
+
+constexpr int planar_blocks(int C) { return (C + kPlanarChannels - 1) / kPlanarChannels; }
+
+constexpr int planar_channels(int C) {
+  const int per = ((C + planar_blocks(C) - 1) / planar_blocks(C) + 3) / 4 * 4;
+  return C < per ? C : per;
+}
+
 // First channel of the block whose nominal first channel is c (< C).  A block
 // is moved as pieces of `piece` channels, the last of them ending at the
 // block's end, so no block may be narrower than a piece: the last one starts

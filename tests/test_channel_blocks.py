@@ -1,4 +1,5 @@
-"""The channel blocks of the transposes (``csrc/channel_blocks.h``), compiled
+"""The channel blocks of the transposes, to and from the cells' rows and of planar
+features (``csrc/channel_blocks.h``), compiled
 for the host: for every channel count the blocks lie inside the row, cover it,
 are no wider than the LDS tile and hold at least one whole piece, which the
 kernels' 16-byte accesses rely on."""
@@ -40,6 +41,11 @@ int main() {
     for (int piece : {1, 4, 8})
       if (C >= piece)
         bad += check("tile_channels", C, tile_channels(C), kTileChannels, piece);
+  for (int C = 4; C <= 20000; ++C) {
+    bad += check("planar_channels", C, planar_channels(C), kPlanarChannels, 4);
+    bad += planar_blocks(C) * planar_channels(C) < C ||
+           (planar_blocks(C) - 1) * planar_channels(C) >= C;
+  }
   return bad ? 1 : 0;
 }
 '''

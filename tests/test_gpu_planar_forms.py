@@ -63,3 +63,10 @@ def test_planar_forward(pkg, cuda, kind, B, N, D, fH, fW, C):
     xc = store.clone().requires_grad_(True)
     want, = torch.autograd.grad(ref.lss_bev_pool(geom, view(xc), dx, bx, nx), xc, up)
     assert_bit_equal(grad, want, 'backward')
+
+
+@pytest.mark.parametrize('C', [3969, 3971, 4097])
+def test_planar_wide_rows(pkg, cuda, C):
+    """Channel counts whose last block would hold fewer than 4 channels (and
+    whose last transpose pass fewer than a 16-byte piece)."""
+    test_planar_forward(pkg, cuda, 'any', 1, 2, 3, 5, 9, C)
