@@ -2377,6 +2377,13 @@ struct CellMap {
     const uint32_t plane = xy.div(cell), b = z.div(plane);
     return int64_t(b) * sb + int64_t(plane - b * z.d) * sz + int64_t(cell - plane * xy.d);
   }
+  // Are 4 cells, the first a multiple of 4, at offsets first .. last
+  // consecutive elements?  They lie in two planes at most, each a run of its
+  // own, so the ends tell; planes of one cell, of which there are 4, can lie in
+  // any order between them.
+  __device__ __forceinline__ bool run_of_4(int64_t first, int64_t last) const {
+    return xy.d > 1 && last == first + 3;
+  }
 };
 
 // acc rows (cell-major fp32, written for occupied cells only) -> out
@@ -2468,7 +2475,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         o[u] = cell0 + j + u < n_cells ? cell_offset(uint32_t(cell0 + j + u)) : -1;
-      const bool run = kVecBev || o[3] == o[0] + 3;
+      const bool run = kVecBev || cell_offset.run_of_4(o[0], o[3]);
       for (int c = tid >> 4; c < C; c += kThreads / 16) {
         if (run) {
           using V = typename std::conditional<sizeof(raw) == 4, u32x4, u32x2>::type;
@@ -2570,7 +2577,7 @@ __global__ __launch_bounds__(kThreads) void rows_to_bev_kernel(
           r[u] = T::to_raw(__builtin_bit_cast(float, b));
       }
       if (kVecBev && off[j] < 0) continue;
-      if (kVecBev || (off[j] >= 0 && off[j + 3] == off[j] + 3)) {
+      if (kVecBev || (off[j] >= 0 && cell_offset.run_of_4(off[j], off[j + 3]))) {
         raw *dst = out + off[j] + int64_t(c0 + c) * sc;
         if constexpr (sizeof(raw) == 4) {
           u32x4 w;
@@ -2652,7 +2659,8 @@ __global__ __launch_bounds__(kThreads) void bev_to_rows_kernel(
   const int64_t offj = cell_offset(uint32_t(live ? cell0 + j : cell0));
   // are they 4 consecutive elements of a channel?
   const bool run =
-      kVecBev || (cell0 + j + 3 < n_cells && cell_offset(uint32_t(cell0 + j + 3)) == offj + 3);
+      kVecBev || (cell0 + j + 3 < n_cells &&
+                  cell_offset.run_of_4(offj, cell_offset(uint32_t(cell0 + j + 3))));
   for (int cn = 0; cn < C; cn += CT) {
     const int c0 = first_channel(C, kVecRow ? kPer : 1, cn);
     const int cb = C - c0 < CT ? C - c0 : CT;
