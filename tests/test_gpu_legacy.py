@@ -249,3 +249,23 @@ def test_ext_module_long_gaps(pkg, cuda, where, gap):
                                                  starts.to(cuda), 1, 1, 1, 4)
     exp = ref.legacy_backward(up, coords, lengths, starts, 1, 1, 1, 4)[0]
     assert_bit_equal(xg, exp, 'backward')
+
+
+def test_ext_module_row_limit(pkg, cuda):
+    """A long interval at the end of 2^31 - 1 rows, the most that are accepted:
+    the loads ahead of its sum stay inside the arrays."""
+    n, length = 2**31 - 1, 300
+    x = torch.empty((n, 4), device=cuda)
+    coords = torch.empty((n, 4), dtype=torch.int32, device=cuda)
+    rows = torch.randn((length, 4), generator=torch.Generator().manual_seed(3))
+    x[n - length:] = rows.to(cuda)
+    coords[n - length:] = 0
+    span = torch.tensor([length], dtype=torch.int32, device=cuda)
+    out = pkg.legacy.ext_module.bev_pool_forward(x, coords, span, n - span, 1, 1, 1, 2)
+    del x, coords
+    torch.cuda.empty_cache()
+    pkg.check_errors()
+    zero = torch.zeros(1, dtype=torch.int32)
+    exp, _ = ref.legacy_forward(rows, torch.zeros((length, 4), dtype=torch.int32),
+                                zero + length, zero, 1, 1, 1, 2)
+    assert_bit_equal(out, exp, 'forward')
