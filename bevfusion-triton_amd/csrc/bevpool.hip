@@ -2034,6 +2034,11 @@ __global__ __launch_bounds__(kPipeThreads) void accum_pipe_kernel(
 // bytes of the row: 16 rows per load, 64 in flight and 64 more being added,
 // transposed through LDS so that lane c adds element c of the rows in order.
 // Every element is still one sequential chain from +0.0 in point order.
+// The slowest of these blocks sets the kernel's time where cells are long, so
+// a block takes kLongPieces pieces of its cells, one 64-byte slice per wave,
+// and rows of more are dealt to several blocks (with all slices of a cell in
+// one block, 5 or 8 of them on 4 waves: 1.43 M depth-weighted points on 2 x 127
+// x 127 cells, C = 92, 144 us; one per wave 73, accum_pipe_kernel 160).
 
 // Rows of the depth-weighted forward (fused depth x context pooling): the row
 // of point p = (bn*D + d)*HW + hw is context row pix = bn*HW + hw, weighted by
@@ -2224,16 +2229,17 @@ __device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64
   }
 }
 
-constexpr int kLongLanes = 16;  // long-cell candidates per block
+constexpr int kLongPieces = 4 * kWaves;  // row pieces per block of long cells
 
 // blockIdx.y: block of at most qmax (<= 64) row pieces.  The first
-// long_blocks blocks of x take the long cells, the others the ranges.
+// long_blocks blocks of x take the long cells (long_sets sets of long_lanes
+// candidates, each set once per kLongPieces pieces), the others the ranges.
 template <typename T, int kK, int kRows>
 __global__ __launch_bounds__(kThreads) void accum_group_kernel(
     const char *__restrict__ xb, int64_t ld_bytes, int C, int qmax,
     const uint64_t *__restrict__ keys, const int32_t *__restrict__ meta,
     const int32_t *__restrict__ cstart, const int32_t *__restrict__ cend, char *__restrict__ acc,
-    int P, int lcell, int long_blocks, DepthRows dr) {
+    int P, int lcell, int long_blocks, int long_sets, int long_lanes, DepthRows dr) {
   constexpr bool kMul = kRows == kRowsDepth;
   constexpr int kH = kK / 2;
   __shared__ u32x4 s_ent[kWaves][64];
@@ -2248,10 +2254,13 @@ __global__ __launch_bounds__(kThreads) void accum_group_kernel(
   const int q = qt - q0 < qmax ? qt - q0 : qmax;
 
   if (int(blockIdx.x) < long_blocks) {
-    const int64_t pos = (int64_t(lane) * long_blocks + blockIdx.x) * lcell;
+    const int part = int(blockIdx.x) / long_sets, set = int(blockIdx.x) - part * long_sets;
+    const int js = q0 + kLongPieces * part;
+    const int je = q0 + q < js + kLongPieces ? q0 + q : js + kLongPieces;
+    const int64_t pos = (int64_t(lane) * long_sets + set) * lcell;
     int cs = 0, ce = 0, r = 0;
     bool found = false;
-    if (lane < kLongLanes && pos < n) {
+    if (lane < long_lanes && pos < n) {
       r = key_rank(keys[pos]);
       cs = cstart[r];
       ce = cend[r];
@@ -2263,9 +2272,9 @@ __global__ __launch_bounds__(kThreads) void accum_group_kernel(
       const uint32_t b0 = uint32_t(__builtin_amdgcn_readlane(cs, src));
       const uint32_t b1 = uint32_t(__builtin_amdgcn_readlane(ce, src));
       const int cell = __builtin_amdgcn_readlane(r, src);
-      for (int j0 = q0; j0 < q0 + q; j0 += 4)
+      for (int j0 = js; j0 < je; j0 += 4)
         if ((task++ & (kWaves - 1)) == wave)
-          sum_long_cell<T, kRows>(xb, ld_bytes, row_bytes, j0, q0 + q, kw, b0, b1,
+          sum_long_cell<T, kRows>(xb, ld_bytes, row_bytes, j0, je, kw, b0, b1,
                                   acc + int64_t(cell) * row_bytes, ent, dr);
     }
     return;
@@ -3801,18 +3810,41 @@ struct GroupPlan {
   int qmax, nblk;   // 16-byte pieces per channel block, channel blocks
   int kk, ng;       // points per batch and groups per wave
   int P, lcell;     // nominal points per group, points of a long cell (P < lcell)
+  int long_parts, long_sets, long_lanes;  // blocks of the long cells
   int64_t waves64;  // waves at 64 points per group
+  bool small;       // faster than accum_pipe_kernel where that takes the rows
 };
 
-// Points per group: fewer where 64 would leave the chip without waves, since a
-// group's chain of loads is the whole kernel there.  Measured (MI355X, rows
-// of 64-512 bytes, 31 K to 4 M points; us at (P, lcell) = (16, 64), (64, 128),
-// (64, 256)): below 4 waves per CU at 64 points (31 K points, C = 80) 14.1,
-// 14.2, 20.1 and (140 K, C = 16) 14.9, 26, 34; below 16 per CU (498 K points,
-// C = 80, depth-weighted) 26.5, 21.2, 24.6; above (1.99 M) 106, 59, 54.
-constexpr int64_t kGroupFewWaves = 4 * 256, kGroupManyWaves = 16 * 256;
+// Points per group: 16 where 64 would leave the chip without waves, since a
+// group's chain of loads is the whole kernel there (MI355X: 31 K points, C = 80,
+// 11-13 us with 16 points a group, 14-15 with 64; 467 K, C = 20, 14 against 22).
+// Batches of fewer than 16 points make the chain longer, hence two lines.
+//
+// Points of a long cell: a group's chain of lcell / kk round trips must not
+// outlast the rest of the launch (lcell <= kk * waves64 / 96: 0.75 us per round
+// trip against the time that the rows of all waves take), but the groups move
+// rows faster than the long cells' waves do, so cells that are ordinary for the
+// grid, up to 6 times its mean at kk = 16, stay with them; cells of fewer than
+// 64 to 256 points always do.  Depth-weighted forwards of 6 cameras, C = 80, us
+// with 256 for every grid, with this rule and with accum_pipe_kernel: 64 x 176 x
+// 118 points on 360 x 360 cells 302, 270, 309; on 128 x 128 772, 358, 532; on
+// 90 x 90 861, 481, 647; 32 x 88 x 118 on 90 x 90 190, 114, 167.
+//
+// Blocks of the long cells: about kLongBlocks, so that the candidates are
+// spread over the chip (60 K points in cells of 100: 45 us with 16 candidates
+// a block, 20 so), up to kLongLanes candidates for each part where more blocks
+// would only wait for their keys to learn that they have nothing to do (7.1 M
+// points on 4 x 360 x 360: 192 us with 16, 189 with 32).
+//
+// Aligned rows of at most kPipeRowBytes: from 4 waves per CU on (C = 80: 197 K
+// points) the pipelined blocks are as fast or faster (25 against 25-31 us at 249
+// K points, 131 against 147 at 2 M), below them the groups' shorter chain is:
+// 23.5 -> 21-22.5 us at 188 K points, C = 80, 22 -> 18 at 121 K, 23 -> 10-12 at
+// 31 K and 18 -> 11 at C = 16.
+constexpr int64_t kGroupFewWaves = 2 * 256, kPipeWaves = 4 * 256, kGroupManyWaves = 16 * 256;
+constexpr int kLongBlocks = 384, kLongLanes = 16;
 
-GroupPlan group_plan(int32_t dtype, int C, int64_t n_points) {
+GroupPlan group_plan(int32_t dtype, int C, int64_t n_points, int64_t n_cells) {
   GroupPlan g;
   const int qt = int((size_t(C) * dtype_size(dtype) + 15) / 16);
   g.nblk = (qt + 63) / 64;
@@ -3821,8 +3853,19 @@ GroupPlan group_plan(int32_t dtype, int C, int64_t n_points) {
   g.kk = per <= 4 ? 16 : (per <= 8 ? 8 : 4);
   g.ng = per < 64 / g.kk ? per : 64 / g.kk;
   g.waves64 = ceil_div(ceil_div(n_points, int64_t(64)), int64_t(g.ng));
-  g.P = g.waves64 < kGroupFewWaves ? 16 : 64;
-  g.lcell = g.waves64 < kGroupFewWaves ? 64 : (g.waves64 < kGroupManyWaves ? 128 : 256);
+  const bool few = g.waves64 < (g.kk == 16 ? kGroupFewWaves : 2 * kGroupFewWaves);
+  g.small = g.waves64 < kPipeWaves;
+  g.P = few ? 16 : 64;
+  const int64_t least = few ? 64 : (g.waves64 < kGroupManyWaves ? 128 : 256);
+  const int64_t mean = 3 * g.kk * n_points / (8 * n_cells), chain = g.kk * g.waves64 / 96;
+  const int64_t lcell = mean < chain ? mean : chain;
+  g.lcell = int(lcell > least ? lcell : least);
+  g.long_parts = int(ceil_div(g.qmax, kLongPieces));
+  const int64_t candidates = ceil_div(n_points, int64_t(g.lcell));
+  const int64_t lanes = ceil_div(candidates * g.long_parts, int64_t(kLongBlocks));
+  const int64_t most = kLongLanes * g.long_parts;  // <= 64 lanes
+  g.long_lanes = int(lanes < most ? lanes : most);
+  g.long_sets = int(ceil_div(candidates, int64_t(g.long_lanes)));
   return g;
 }
 
@@ -3832,7 +3875,7 @@ int launch_accum_group(int32_t dtype, const GroupPlan &g, const char *x, int64_t
                        int64_t n_points, const uint64_t *keys, const int32_t *meta,
                        const int32_t *cstart, const int32_t *cend, void *acc, const DepthRows &dr,
                        bool stream_rows, hipStream_t s) {
-  const int long_blocks = int(ceil_div(ceil_div(n_points, int64_t(g.lcell)), kLongLanes));
+  const int long_blocks = g.long_sets * g.long_parts;
   const int64_t waves = ceil_div(ceil_div(n_points, int64_t(g.P)), int64_t(g.ng));
   const int64_t blocks = long_blocks + ceil_div(waves, kWaves);
   if (int st = check_grid(blocks, kThreads, "accum_group")) return st;
@@ -3840,7 +3883,7 @@ int launch_accum_group(int32_t dtype, const GroupPlan &g, const char *x, int64_t
 #define BEVPOOL_AG(T, K, M)                                                                    \
   hipLaunchKernelGGL((accum_group_kernel<T, K, M>), grid, dim3(kThreads), 0, s, x, ld_bytes, C, \
                      g.qmax, keys, meta, cstart, cend, static_cast<char *>(acc), g.P, g.lcell, \
-                     long_blocks, dr)
+                     long_blocks, g.long_sets, g.long_lanes, dr)
 #define BEVPOOL_AG_K(T, M)                                                                     \
   {                                                                                            \
     if (g.kk == 16) BEVPOOL_AG(T, 16, M);                                                     \
@@ -4469,13 +4512,9 @@ static int forward_impl(const void *feats, int32_t dtype, int64_t feats_row_stri
                        reinterpret_cast<uintptr_t>(feats) % 16 == 0;
     // rows of every point (an upper bound of the kept rows read)
     const bool stream_rows = n_points * int64_t(row_bytes) <= kStreamRowBytes;
-    const GroupPlan plan = group_plan(dtype, C, n_points);
+    const GroupPlan plan = group_plan(dtype, C, n_points, n_cells);
     LaunchTimer t("accum_rows", s);
-    if (vec16 && row_bytes <= size_t(kPipeRowBytes) && plan.waves64 >= kGroupFewWaves) {
-      // From 4 waves per CU on (C = 80: 197 K points) the pipelined blocks are
-      // as fast or faster: 43.9 against 42.4-46 us at 498 K points, 131 against
-      // 147 at 2 M.  Below, the groups' shorter chain is: 20.6 -> 12.5 us at
-      // 31 K points, C = 80, and 18.4 -> 13.4 at C = 16.
+    if (vec16 && row_bytes <= size_t(kPipeRowBytes) && !plan.small) {
       st = launch_accum_pipe(dtype, x, ld_bytes, C, n_points, keys, meta, cell_end, acc,
                              stream_rows, s);
     } else if (row_bytes >= 16) {
@@ -4650,7 +4689,7 @@ int bevpool_forward_depth(const float *depth, const float *context_rows, int32_t
   if (n_points > 0) {
     const DepthRows dr{depth, make_fast_div(uint32_t(HW)), make_fast_div(uint32_t(D))};
     LaunchTimer t("accum_rows", s);
-    st = launch_accum_group(BEVPOOL_F32, group_plan(BEVPOOL_F32, C, n_points),
+    st = launch_accum_group(BEVPOOL_F32, group_plan(BEVPOOL_F32, C, n_points, n_cells),
                             reinterpret_cast<const char *>(context_rows), int64_t(C) * 4, C,
                             n_points, keys, meta, cell_start, cell_end, acc, dr, false, s);
     if (st) return st;

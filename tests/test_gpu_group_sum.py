@@ -117,3 +117,25 @@ def test_wide_rows(pkg, cuda, grid, C, dtype):
     out, grad, up = run_op(pkg, feats, coords, grid, cuda)
     assert_bit_equal(out, ref.bev_pool(feats.float(), coords, *grid).to(dtype), 'forward')
     assert_bit_equal(grad, up.to(dtype)[b, :, z, x, y], 'backward')
+
+
+@pytest.mark.parametrize('C,dtype,N,grid', [
+    (68, F32, 30000, (7, 9)), (80, F32, 70000, (40, 50)), (80, F32, 130000, (6, 6)),
+    (132, F32, 200000, (20, 30)), (256, F32, 60000, (1, 2)), (260, F32, 90000, (30, 40)),
+    (39, F32, 30000, (5, 3)), (130, F16, 60000, (6, 8)), (520, BF16, 40000, (9, 5)),
+    (1032, BF16, 20000, (20, 20)), (17, F32, 300000, (30, 30))])
+def test_points_per_cell(pkg, cuda, C, dtype, N, grid):
+    """Grids from a few points a cell to all of them in two cells: the points
+    of a long cell from their floor to the chain's limit, rows of one to four
+    blocks of long-cell pieces (the last of one piece or more) and of two and
+    three channel blocks."""
+    g = torch.Generator().manual_seed(N + C)
+    H, W = grid
+    hot = torch.randint(max(1, H * W // 9), (N,), generator=g)
+    rank = torch.where(torch.rand(N, generator=g) < 0.3, hot, torch.randint(H * W, (N,), generator=g))
+    coords = torch.stack((rank // W, rank % W, rank * 0, rank * 0), 1).to(torch.int32)
+    feats = torch.randn((N, C), generator=g).to(dtype)
+    out, grad, up = run_op(pkg, feats, coords, (1, 1, H, W), cuda)
+    assert_bit_equal(out, ref.bev_pool(feats.float(), coords, 1, 1, H, W).to(dtype), 'forward')
+    want = up.to(dtype).permute(0, 2, 3, 4, 1).reshape(H * W, C)[rank]
+    assert_bit_equal(grad, want, 'backward')
