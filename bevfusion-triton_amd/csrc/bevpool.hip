@@ -3820,6 +3820,12 @@ struct GroupPlan {
 // 11-13 us with 16 points a group, 14-15 with 64; 467 K, C = 20, 14 against 22).
 // Batches of fewer than 16 points make the chain longer, hence two lines.
 //
+// Points per batch: as many as the groups' LDS entries hold.  Context rows of 4
+// to 7 pieces would leave 9 to 16 groups 4 rows each; with enough waves fewer
+// groups of 8 are faster (2 M points, C = 16, 51 -> 36 us, accum_pipe_kernel 48;
+// C = 24 48 -> 41, 51), of 16 on grids with few points a cell (2.35 M on 7 x
+// 330 x 330, C = 24, 74, 66 and 54 us with 4, 8 and 16, accum_pipe_kernel 60).
+//
 // Points of a long cell: a group's chain of lcell / kk round trips must not
 // outlast the rest of the launch (lcell <= kk * waves64 / 96: 0.75 us per round
 // trip against the time that the rows of all waves take), but the groups move
@@ -3844,7 +3850,7 @@ struct GroupPlan {
 constexpr int64_t kGroupFewWaves = 2 * 256, kPipeWaves = 4 * 256, kGroupManyWaves = 16 * 256;
 constexpr int kLongBlocks = 384, kLongLanes = 16;
 
-GroupPlan group_plan(int32_t dtype, int C, int64_t n_points, int64_t n_cells) {
+GroupPlan group_plan(int32_t dtype, int C, int64_t n_points, int64_t n_cells, bool depth_rows) {
   GroupPlan g;
   const int qt = int((size_t(C) * dtype_size(dtype) + 15) / 16);
   g.nblk = (qt + 63) / 64;
@@ -3854,6 +3860,11 @@ GroupPlan group_plan(int32_t dtype, int C, int64_t n_points, int64_t n_cells) {
   g.ng = per < 64 / g.kk ? per : 64 / g.kk;
   g.waves64 = ceil_div(ceil_div(n_points, int64_t(64)), int64_t(g.ng));
   const bool few = g.waves64 < (g.kk == 16 ? kGroupFewWaves : 2 * kGroupFewWaves);
+  if (depth_rows && g.kk == 4 && g.qmax >= 4 && !few) {
+    g.kk = n_points < 8 * n_cells ? 16 : 8;
+    g.ng = 64 / g.kk;
+    g.waves64 = ceil_div(ceil_div(n_points, int64_t(64)), int64_t(g.ng));
+  }
   g.small = g.waves64 < kPipeWaves;
   g.P = few ? 16 : 64;
   const int64_t least = few ? 64 : (g.waves64 < kGroupManyWaves ? 128 : 256);
@@ -4512,7 +4523,7 @@ static int forward_impl(const void *feats, int32_t dtype, int64_t feats_row_stri
                        reinterpret_cast<uintptr_t>(feats) % 16 == 0;
     // rows of every point (an upper bound of the kept rows read)
     const bool stream_rows = n_points * int64_t(row_bytes) <= kStreamRowBytes;
-    const GroupPlan plan = group_plan(dtype, C, n_points, n_cells);
+    const GroupPlan plan = group_plan(dtype, C, n_points, n_cells, false);
     LaunchTimer t("accum_rows", s);
     if (vec16 && row_bytes <= size_t(kPipeRowBytes) && !plan.small) {
       st = launch_accum_pipe(dtype, x, ld_bytes, C, n_points, keys, meta, cell_end, acc,
@@ -4689,7 +4700,7 @@ int bevpool_forward_depth(const float *depth, const float *context_rows, int32_t
   if (n_points > 0) {
     const DepthRows dr{depth, make_fast_div(uint32_t(HW)), make_fast_div(uint32_t(D))};
     LaunchTimer t("accum_rows", s);
-    st = launch_accum_group(BEVPOOL_F32, group_plan(BEVPOOL_F32, C, n_points, n_cells),
+    st = launch_accum_group(BEVPOOL_F32, group_plan(BEVPOOL_F32, C, n_points, n_cells, true),
                             reinterpret_cast<const char *>(context_rows), int64_t(C) * 4, C,
                             n_points, keys, meta, cell_start, cell_end, acc, dr, false, s);
     if (st) return st;

@@ -139,3 +139,21 @@ def test_points_per_cell(pkg, cuda, C, dtype, N, grid):
     assert_bit_equal(out, ref.bev_pool(feats.float(), coords, 1, 1, H, W).to(dtype), 'forward')
     want = up.to(dtype).permute(0, 2, 3, 4, 1).reshape(H * W, C)[rank]
     assert_bit_equal(grad, want, 'backward')
+
+
+@pytest.mark.parametrize('C', [16, 20, 28, 32, 92])
+@pytest.mark.parametrize('D,fH,fW,half', [(59, 32, 90, 8), (59, 32, 90, 200), (20, 64, 176, 400)])
+def test_depth_batches(pkg, cuda, C, D, fH, fW, half):
+    """Context rows with enough waves for batches of 8 and 16 points, on dense
+    and on sparse grids."""
+    g = torch.Generator().manual_seed(C + half)
+    shape = (1, 6, D, fH, fW)
+    geom = torch.stack([(torch.rand(shape, generator=g) - 0.5) * 2.1 * half * s for s in (1, 1)]
+                       + [torch.zeros(shape)], -1)
+    depth = torch.randn(6, D, fH, fW, generator=g).softmax(1)
+    context = torch.randn(6, C, fH, fW, generator=g)
+    bounds = ((-half, half, 1.0), (-half, half, 1.0), (-1.0, 1.0, 2.0))
+    module = pkg.BevPoolTransform(*bounds).to(cuda)
+    out = module.bev_pool_depth(geom.to(cuda), depth.to(cuda), context.to(cuda))
+    want = ref.lss_bev_pool_depth(geom, depth, context, *ref.gen_dx_bx(*bounds))
+    assert_bit_equal(out, want, 'forward')
