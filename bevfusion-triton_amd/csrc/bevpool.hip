@@ -3462,8 +3462,7 @@ constexpr int kDgPix = 16;  // pixels per depth_grad block (4 per wave)
 //   grad_ctx[bn, c, hw]  = sum_d g[rank[p_d], c] * depth[p_d]
 // with p_d = (bn*D + d)*HW + hw.
 // A block takes a patch of kDgPix pixels: 4 rows of 4 columns of the image
-// (pw = 4), or 16 in a row (pw = 16, fH = 1) where the image's width is not
-// known.  Their ranks and depths are staged in LDS ([d][pixel]); each wave
+// (pw = 4), or 16 in a row (pw = 16, fH = 1) where patches do not fit.  Their ranks and depths are staged in LDS ([d][pixel]); each wave
 // then takes 4 pixels, one per 16-lane row of the wave: of a 4 x 4 patch a
 // column of 4, which lie above each other and so, bin by bin, mostly hit one
 // cell: the wave's four row loads are then one row's lines.  Lane j of a row
@@ -4739,11 +4738,20 @@ static int backward_depth_impl(const float *grad, int64_t grad_stride_b, int64_t
                 (long long)(2 * int64_t(D) + C));
   if (HW > INT32_MAX) return fail(BEVPOOL_EINVAL, "bad depth layout");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int fW = int(HW / fH);
-  // 4 x 4 pixels per block, or 16 in a row without an image plane (or with one
-  // of fewer than 4 rows or columns, which would leave most of a patch empty)
-  const int pw = fH >= 4 && fW >= 4 ? 4 : kDgPix;
-  const int h_tiles = int(ceil_div(fH, kDgPix / pw)), w_tiles = int(ceil_div(fW, pw));
+  int fW = int(HW / fH);
+  int pw = 4, h_tiles = int(ceil_div(fH, 4)), w_tiles = int(ceil_div(fW, 4));
+  // 4 x 4 pixels per block, or 16 in a row of all HW where the image plane is
+  // not known or cuts into more than 1.1 times as many patches, some of them
+  // partial: a patch is at most that much faster than 16 pixels in a row.  Both
+  // in us, C = 80: 24 maps of 32 x 88 (1408 blocks each) 162 and 184, 24 of 25 x
+  // 41 (1848 and 1560) 82 and 68, 6 of 704 x 2 (1056 and 528) 73 and 21, 3000 of
+  // 5 x 5 (12,000 and 6000) 190 and 117.
+  if (int64_t(h_tiles) * w_tiles * 10 > ceil_div(HW, kDgPix) * 11) {
+    pw = kDgPix;
+    fH = h_tiles = 1;
+    fW = int(HW);
+    w_tiles = int(ceil_div(HW, kDgPix));
+  }
   const int64_t n_tiles = n_pix / HW * h_tiles * w_tiles;
   int st;
   if ((st = check_grid(n_tiles + kXcds, kThreads, "depth_grad"))) return st;

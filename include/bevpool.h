@@ -367,8 +367,8 @@ int bevpool_backward_depth(const float *grad, int64_t grad_stride_b, int64_t gra
 /*
  * bevpool_backward_depth for a caller that states the image plane, HW = fH *
  * fW with hw = h*fW + w: the points of a depth bin and an image column mostly
- * share a cell, so pixels are taken column by column.  The same sums in the
- * same order.
+ * share a cell, so pixels are taken column by column where the plane cuts into
+ * few partial 4 x 4 patches.  The same sums in the same order.
  */
 int bevpool_backward_depth_image(const float *grad, int64_t grad_stride_b, int64_t grad_stride_c,
                                  int64_t grad_stride_z, int32_t C, const int32_t *rank,

@@ -75,3 +75,14 @@ def test_not_finite(pkg, cuda, kind):
         assert torch.equal(got.isnan(), want.isnan())
         assert torch.equal(got[got.isinf()], want[want.isinf()])
         assert ((got - want).abs()[fin] <= (n + 2) * U * mag[fin]).all()
+
+
+@pytest.mark.parametrize('kind', ['column', 'points'])
+@pytest.mark.parametrize('D,fH,fW,C', [
+    (5, 70, 1, 8), (9, 70, 2, 80), (6, 41, 3, 64), (7, 5, 6, 80), (4, 5, 9, 36), (5, 8, 22, 80),
+    (3, 33, 89, 4), (4, 29, 51, 16), (5, 7, 7, 128),
+    (4, 2, 9, 20), (3, 3, 3, 64), (3, 1, 47, 32)])
+def test_narrow_maps(pkg, cuda, kind, D, fH, fW, C):
+    """Maps that 4 x 4 patches would leave half empty (taken 16 pixels in a
+    row of the whole map) and those around what is worth patches."""
+    test_sizes(pkg, cuda, kind, D, fH, fW, C)
