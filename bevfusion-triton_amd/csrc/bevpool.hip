@@ -3352,7 +3352,7 @@ __global__ __launch_bounds__(kThreads) void planar_tile_kernel(
   }
 }
 
-// The same one element per thread, for fewer than 4 channels or points.
+// The same one element per thread, for fewer than 4 channels or few points.
 __global__ __launch_bounds__(kThreads) void planar_rows_kernel(
     const float *__restrict__ src, int C, int64_t S, int64_t n_rows, int64_t sbn, int64_t sc,
     float *__restrict__ rows) {
@@ -4573,18 +4573,23 @@ static int planar_rows_impl(const float *src, int64_t stride_bn, int64_t stride_
   if (n_rows == 0) return BEVPOOL_OK;
   if (!src || !rows) return fail(BEVPOOL_EINVAL, "null argument");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool vec = C >= 4 && S >= 4;
   const int64_t tiles_s = ceil_div(S, kPlanarTile);
-  LaunchTimer t("planar_rows", s);
-  // (sizes that do not divide by 4 keep the limit of one element per thread)
+  const int64_t tiles = BN * tiles_s, elements = ceil_div(n_rows * C, kThreads);  // blocks
+  // the launch limit is the tiles' where 4 divides every size, else that of one
+  // element per thread (within which the tiles' grid always fits)
   const bool even = C % 4 == 0 && S % 4 == 0 && stride_bn % 4 == 0 && stride_c % 4 == 0;
-  int st = check_grid(vec && even ? BN * tiles_s : ceil_div(n_rows * C, kThreads), kThreads,
-                      "planar_rows");
-  if (st) return st;
+  if (int st = check_grid(even ? tiles : elements, kThreads, "planar_rows")) return st;
+  // A tile of a few points costs what a larger one does: with fewer than 12
+  // points or 400 elements one element per thread is faster (tiles against
+  // elements, us, 1 M rows: C = 80, S = 5 647 and 254, S = 15 271 and 321; C =
+  // 16, S = 15 55 and 39, S = 31 33 and 41).
+  const bool small = S < 12 || S * C < 400;
+  const bool vec = C >= 4 && S >= 4 && !(small && elements * kThreads <= int64_t(UINT32_MAX));
+  LaunchTimer t("planar_rows", s);
   if (vec) {
     const int cmax = planar_channels(C);
     const size_t smem = size_t(kPlanarTile) * size_t(cmax + 1) * sizeof(float);
-    const dim3 grid(unsigned(BN * tiles_s), unsigned(planar_blocks(C)));
+    const dim3 grid(unsigned(tiles), unsigned(planar_blocks(C)));
 #define BEVPOOL_PT(K)                                                                          \
   case K:                                                                                      \
     hipLaunchKernelGGL((planar_tile_kernel<K>), grid, dim3(kThreads), smem, s, src, C, cmax, S, \
@@ -4600,8 +4605,8 @@ static int planar_rows_impl(const float *src, int64_t stride_bn, int64_t stride_
     }
 #undef BEVPOOL_PT
   } else {
-    hipLaunchKernelGGL(planar_rows_kernel, dim3(unsigned(ceil_div(n_rows * C, kThreads))),
-                       dim3(kThreads), 0, s, src, C, S, n_rows, stride_bn, stride_c, rows);
+    hipLaunchKernelGGL(planar_rows_kernel, dim3(unsigned(elements)), dim3(kThreads), 0, s, src, C,
+                       S, n_rows, stride_bn, stride_c, rows);
   }
   return check_launch("planar_rows");
 }

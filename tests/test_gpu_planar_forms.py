@@ -70,3 +70,25 @@ def test_planar_wide_rows(pkg, cuda, C):
     """Channel counts whose last block would hold fewer than 4 channels (and
     whose last transpose pass fewer than a 16-byte piece)."""
     test_planar_forward(pkg, cuda, 'any', 1, 2, 3, 5, 9, C)
+
+
+@pytest.mark.parametrize('S', [4, 5, 8, 11, 12, 13, 24, 25, 100])
+@pytest.mark.parametrize('C', [4, 16, 33, 36, 80])
+def test_planar_small_planes(pkg, cuda, S, C):
+    """Many planes of a few points, by elements and by tiles."""
+    from bevfusion_triton_amd import _pipeline as P
+
+    src = torch.randn(300, C, S, generator=torch.Generator().manual_seed(S + C))
+    rows = P.planar_rows(src.to(cuda))
+    assert_bit_equal(rows, src.transpose(1, 2).reshape(-1, C), 'rows')
+
+
+def test_planar_most_planes(pkg, cuda):
+    """More planes of 5 points than a launch has blocks (2^24 of 256 threads)."""
+    from bevfusion_triton_amd import _pipeline as P
+
+    src = torch.arange(((1 << 24) + 9) * 25, dtype=torch.int32, device=cuda).view(torch.float32)
+    src = src.view(-1, 5, 5)
+    rows = P.planar_rows(src)
+    want = src.transpose(1, 2).reshape(-1, 5)
+    assert torch.equal(rows.view(torch.int32), want.view(torch.int32))
