@@ -1667,7 +1667,12 @@ static_assert(kStageRows == 32, "only 32-row accumulation stages are supported")
 //                step.  With 2.6-5.1 GB of rows (4 x 360 x 360, 2 x 720 x 720)
 //                the accumulation itself got 4-6% slower and nothing else
 //                faster, so inputs of more than kStreamRowBytes of rows keep
-//                ordinary loads.
+//                ordinary loads.  accum_group_kernel takes the same rule:
+//                level for rows of whole lines (128 fp32 channels, 1.6 M points:
+//                accumulation 176 us, 173 with ordinary loads, the step 385 and
+//                391), slower for rows that share lines with their neighbours
+//                (90 fp16 channels, 1.06 M points: 80 and 65, the step 179 and
+//                172; 50 bf16 channels, 4.8 M: 254 and 177, 504 and 434).
 //   kRowsDepth   depth-weighted context rows (DepthRows), ordinary loads:
 //                a context row is read for every depth bin
 //                (accum_group_kernel only).
@@ -2014,17 +2019,19 @@ __global__ __launch_bounds__(kPipeThreads) void accum_pipe_kernel(
 //     next one are in flight meanwhile.
 //   * Rows are in flight kK at a time in two register halves: one is added
 //     while the other loads.
-// What bounds it: L2 -> CU traffic of the gathered rows when those are
-// context rows (1 x 360 x 360, C = 80: 568 MB in 55 us, 10.3 TB/s; the
-// pipelined kernel, bound by its instructions per row, took 88; 4 x 360 x 360
-// 204 against 339 us), HBM for feature rows.  There 16-byte aligned rows of
-// one channel block stay with accum_pipe_kernel, whose blocks keep more rows
-// of few cells in flight (131 against 147 us at 1 x 360 x 360).  Rows of 128
-// fp32 channels, two channel blocks to that kernel, take 189 against 215 us;
-// 180-byte fp16 rows at 1.06 M points 81 against 457 us for
-// accum_rows_kernel's element-wise loads.  Walking the ranges in
-// XCD-contiguous eighths cost 5-10%, rings of 4 + 4 rows 3-10%, and a
-// register limit for 4 waves per SIMD spilled.
+// What bounds it with context rows (counters at C = 80, 7.1 M points on 4 x 360 x
+// 360, 190 us, and 1.8 M on 1 x 360 x 360, 55 us): no unit by itself.  L2 takes
+// 157 and 123 G requests/s, about half of one per channel and clock, 77 and 80%
+// of them hits; an L1 miss returns after 274 and 252 clocks; the L1s make 0.7 and
+// 0.6 accesses per clock; the vector units issue 45 and 38% of the time, with 2.5
+// and 2.2 waves per SIMD resident.  (accum_pipe_kernel took 339 and 88 us.)
+// Feature rows come from HBM.  There 16-byte aligned rows of one channel block
+// stay with accum_pipe_kernel, whose blocks keep more rows of few cells in
+// flight (131 against 147 us at 1 x 360 x 360).  Rows of 128 fp32 channels, two
+// channel blocks to that kernel, take 189 against 215 us; 180-byte fp16 rows at
+// 1.06 M points 80 against 457 us for accum_rows_kernel's element-wise loads.
+// Walking the ranges in XCD-contiguous eighths cost 5-10%, rings of 4 + 4 rows
+// 3-10%, and a register limit for 4 waves per SIMD spilled.
 //
 // Long cells.  One group would walk a cell of L points as a chain of L / kK
 // round trips, so cells of at least lcell points go to the launch's first
@@ -2962,8 +2969,9 @@ __device__ __forceinline__ int64_t legacy_count(int64_t cap, const int32_t *__re
 // the row (sum_long_cell), so that no chain of loads outlasts the rest.
 // Neighbouring intervals go to different blocks: the long ones, the cells
 // near the cameras, are neighbours.  The rows are read once, so HBM bounds it:
-// 1.54 M rows of 80 channels (494 MB) in 39 K intervals 118 us, against 230 with
-// one wave per interval and 4 bytes per lane.
+// 1.54 M rows of 80 channels (494 MB, 514 fetched) in 39 K intervals 118 us, 4.5
+// TB/s with the sums written (a copy makes 5.2), against 230 with one wave per
+// interval and 4 bytes per lane.
 constexpr int kLegacyLong = 256;
 // Blocks of a legacy launch; more intervals loop (2048 and 16384 blocks: forward
 // 129 and 133 us, backward 110 and 108).
@@ -3128,10 +3136,10 @@ __global__ __launch_bounds__(kThreads) void legacy_order_kernel(
 // unordered: null or *unordered != 0: x_grad is zero already and invalid
 // intervals are skipped; else the wave also writes its interval's gap up to
 // the next one (and up to the first one) as zeros, and an invalid cell's rows.
-// The write stream bounds it: 1.54 M rows of 80 channels (494 MB) in 104 us
-// (and 6 + 3 for the order check and the skipped fill), against 78 us of zero
-// fill and 154 us with 4 bytes per lane.  Temporal stores took 94 us and the
-// forward that follows 36 us more.
+// The write stream bounds it: 1.54 M rows of 80 channels (494 MB, 500 written) in
+// 104 us, 4.8 TB/s where a fill makes 6.9 (and 6 + 3 us for the order check and
+// the skipped fill), against 78 us of zero fill and 154 us with 4 bytes per lane.
+// Temporal stores took 94 us and the forward that follows 36 us more.
 template <bool kWide>
 __global__ __launch_bounds__(kThreads) void legacy_spread_kernel(
     const char *__restrict__ g, int64_t n, int C, int qmax, const int32_t *__restrict__ geom,
@@ -3289,10 +3297,12 @@ __device__ __forceinline__ void store16(float *p, u32x4 v) {
 // consecutive threads at consecutive addresses.  Ragged sizes keep to 16-byte
 // accesses by overlap: a camera's last tile is shifted back to end at S, a
 // row's last piece to end at its last channel; what is moved twice is the
-// same.  Non-temporal stores: the rows are read back by a random gather, and
-// left temporal, their dirty lines slowed the accumulation that follows from
-// 126 to 171 us.  With `rank`, rows of dropped points (rank -1), which nothing
-// reads, are not written.
+// same.  Non-temporal stores, which are level with ordinary ones: the transpose
+// is slower, the accumulation that gathers the rows faster (us, 550 MB of rows at
+// 1 x 256 x 256 219 + 128 against 207 + 136, whole passes 538 and 533; 359 MB
+// 122 + 81 and 114 + 87, 346 and 341; 159 MB 57 + 43 and 52 + 44, 186 and 181;
+// 200 MB of 64 channels 72 + 49 and 70 + 54, 231 and 236).  With `rank`, rows of
+// dropped points (rank -1), which nothing reads, are not written.
 // HBM traffic bounds it (1.28 GB at 1 x 360 x 360: 235 us; 64-point tiles 6 us
 // more, a register transpose whose stores scatter 16-byte pieces 288 us).
 // Without the dropped points' rows, 14% of them at 1 x 256 x 256, it takes 219
@@ -3474,9 +3484,10 @@ constexpr int kDgPix = 16;  // pixels per depth_grad block (4 per wave)
 // sums, are written out from there.  g: cell-major fp32 rows of the occupied
 // cells; ctx: channel-last rows (planar_tile_kernel).  Blocks map
 // XCD-contiguously, so the cells of neighbouring pixels' rays meet in one L2.
-// Gathered rows from L2 bound it: 4 x 360 x 360, C = 80 (2.26 GB): 216 us with
-// one bin per row of the wave and 4-byte loads, 184 with 16-byte loads, 162
-// with the columns.
+// Vector instructions bound it: at 4 x 360 x 360, C = 80, 162 us, a SIMD issues
+// 98 K of them (50 per bin and wave), 4 clocks each, with 5.9 waves resident; L2
+// takes 80 G requests/s, 73% hits.  One bin per row of the wave and 4-byte loads
+// took 216 us, 16-byte loads 184, the columns 162.
 template <int kX, int kR>
 __global__ __launch_bounds__(kThreads) void depth_grad_kernel(
     const float *__restrict__ g, int C, const int32_t *__restrict__ rank,

@@ -157,3 +157,14 @@ def test_depth_batches(pkg, cuda, C, D, fH, fW, half):
     out = module.bev_pool_depth(geom.to(cuda), depth.to(cuda), context.to(cuda))
     want = ref.lss_bev_pool_depth(geom, depth, context, *ref.gen_dx_bx(*bounds))
     assert_bit_equal(out, want, 'forward')
+
+
+def test_more_rows_than_are_streamed(pkg, cuda):
+    """Feature rows of more than 1 GiB take ordinary loads."""
+    C, N, H, W = 257, 1_050_000, 60, 70
+    g = torch.Generator().manual_seed(5)
+    rank = torch.randint(H * W, (N,), generator=g)
+    coords = torch.stack((rank // W, rank % W, rank * 0, rank * 0), 1).to(torch.int32)
+    feats = torch.randn((N, C), generator=g)
+    out = pkg.bev_pool(feats.to(cuda), coords.to(cuda), 1, 1, H, W)
+    assert_bit_equal(out, ref.bev_pool(feats, coords, 1, 1, H, W), 'forward')
