@@ -2154,14 +2154,14 @@ __device__ __forceinline__ void group_add(const GroupRing<kH> &R, PieceSum<T> &s
 // One wave's share of a long cell: elements of pieces [j0, j0 + 4) of the row
 // (pieces from jend on repeat the last one and are not stored) summed over
 // sorted positions [b0, b1).  The loads run up to 192 positions ahead of the
-// sum, and b1 may be 2^31 - 1: positions are unsigned.  tile: the wave's 64
-// 16-byte LDS entries.
+// sum, and b1 may be 2^31 - 1: positions are counted from the cell's last.
+// tile: the wave's 64 16-byte LDS entries.
 template <typename T, int kRows>
 __device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64_t ld_bytes,
                                               int row_bytes, int j0, int jend,
-                                              const uint32_t *__restrict__ kw, uint32_t b0,
-                                              uint32_t b1, char *__restrict__ out_row,
-                                              u32x4 *tile, const DepthRows &dr) {
+                                              const uint32_t *__restrict__ kw, int b0, int b1,
+                                              char *__restrict__ out_row, u32x4 *tile,
+                                              const DepthRows &dr) {
   using raw = typename T::raw;
   constexpr bool kMul = kRows == kRowsDepth;
   constexpr int kPe = 16 / int(sizeof(raw));  // elements per piece
@@ -2173,12 +2173,12 @@ __device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64
   float a = 0.0f, w[kT];
   u32x4 v[kT];
   uint32_t idx[kT];
-  auto indices = [&](uint32_t base) {  // past the cell: its last point
+  auto indices = [&](int rest) {  // from `rest` before the last point; past that: itself
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
-      const uint32_t p = base + uint32_t(16 * t + slot);
-      const uint32_t pc = p < b1 ? p : b1 - 1;
-      idx[t] = kRows == kRowsRun ? pc : kw[2 * int64_t(pc)];
+      const int back = rest - (16 * t + slot);
+      const int p = b1 - 1 - (back > 0 ? back : 0);
+      idx[t] = kRows == kRowsRun ? uint32_t(p) : kw[2 * int64_t(p)];
     }
   };
   auto rows = [&]() {
@@ -2189,10 +2189,10 @@ __device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64
       v[t] = load_piece<kRows>(xp + int64_t(row) * ld_bytes);
     }
   };
-  indices(b0);
+  indices(b1 - 1 - b0);
   rows();
-  indices(b0 + 16 * kT);
-  for (uint32_t base = b0; base < b1; base += 16 * kT) {
+  indices(b1 - 1 - b0 - 16 * kT);
+  for (int rest = b1 - 1 - b0; rest >= 0; rest -= 16 * kT) {
     u32x4 c[kT];
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
@@ -2207,10 +2207,10 @@ __device__ __forceinline__ void sum_long_cell(const char *__restrict__ xb, int64
       }
     }
     rows();  // of the next 64 positions, whose indices have arrived
-    indices(base + 32 * kT);
+    indices(rest - 32 * kT);
 #pragma unroll
     for (int t = 0; t < kT; ++t) {
-      const int left = int(b1 - base) - 16 * t;
+      const int left = rest + 1 - 16 * t;
       if (left <= 0) break;
       wave_lds_order();
       tile[lane] = c[t];
@@ -2276,8 +2276,7 @@ __global__ __launch_bounds__(kThreads) void accum_group_kernel(
     int task = 0;  // the block's waves take its (cell, four pieces) tasks in turn
     for (uint64_t m = __ballot(found); m; m &= m - 1) {
       const int src = __builtin_ctzll(m);
-      const uint32_t b0 = uint32_t(__builtin_amdgcn_readlane(cs, src));
-      const uint32_t b1 = uint32_t(__builtin_amdgcn_readlane(ce, src));
+      const int b0 = __builtin_amdgcn_readlane(cs, src), b1 = __builtin_amdgcn_readlane(ce, src);
       const int cell = __builtin_amdgcn_readlane(r, src);
       for (int j0 = js; j0 < je; j0 += 4)
         if ((task++ & (kWaves - 1)) == wave)
@@ -3059,8 +3058,8 @@ __global__ __launch_bounds__(kThreads) void legacy_sum_kernel(
       const int64_t sl = starts[jl];
       const int ll = lengths[jl];
       const int64_t cl = legacy_cell(geom, n, sl, ll, nb, nd, nh, nw);
-      const uint32_t b0 = uint32_t(__builtin_amdgcn_readfirstlane(int(sl)));
-      const uint32_t b1 = b0 + uint32_t(__builtin_amdgcn_readfirstlane(ll));
+      const int b0 = __builtin_amdgcn_readfirstlane(int(sl));
+      const int b1 = b0 + __builtin_amdgcn_readfirstlane(ll);
       sum_long_cell<F32, kRowsRun>(x, row_bytes, row_bytes, q0 + 4 * (t % slices), q0 + q, nullptr,
                                    b0, b1, out + cl * row_bytes, s_tile[wave], DepthRows{});
     }
