@@ -2241,8 +2241,11 @@ constexpr int kLongPieces = 4 * kWaves;  // row pieces per block of long cells
 // blockIdx.y: block of at most qmax (<= 64) row pieces.  The first
 // long_blocks blocks of x take the long cells (long_sets sets of long_lanes
 // candidates, each set once per kLongPieces pieces), the others the ranges.
+// Feature rows in batches of 4 keep to 80 VGPRs, 6 waves per SIMD (82: 5, and 90
+// -> 113 us at 1.6 M rows of 27 fp32 channels); with context rows that spills.
 template <typename T, int kK, int kRows>
-__global__ __launch_bounds__(kThreads) void accum_group_kernel(
+__global__ __launch_bounds__(kThreads, kK == 4 && kRows != kRowsDepth ? 6 : 1) void
+accum_group_kernel(
     const char *__restrict__ xb, int64_t ld_bytes, int C, int qmax,
     const uint64_t *__restrict__ keys, const int32_t *__restrict__ meta,
     const int32_t *__restrict__ cstart, const int32_t *__restrict__ cend, char *__restrict__ acc,
@@ -3827,7 +3830,10 @@ struct GroupPlan {
 // Points per group: 16 where 64 would leave the chip without waves, since a
 // group's chain of loads is the whole kernel there (MI355X: 31 K points, C = 80,
 // 11-13 us with 16 points a group, 14-15 with 64; 467 K, C = 20, 14 against 22).
-// Batches of fewer than 16 points make the chain longer, hence two lines.
+// Batches of fewer than 16 points make the chain longer, and on sparse grids few
+// cells are long at 16 points a group, hence three lines (170 K points, C = 52: on
+// 393 x 393 cells 12-13 us with 16, 15-16 with 64, on 128 x 128 17 and 16; C = 80,
+// 885 waves of 64: on 128 x 128 20-21 and 16-17, on 360 x 360 16-17 and 14-15).
 //
 // Points per batch: as many as the groups' LDS entries hold.  Context rows of 4
 // to 7 pieces would leave 9 to 16 groups 4 rows each; with enough waves fewer
@@ -3839,7 +3845,8 @@ struct GroupPlan {
 // outlast the rest of the launch (lcell <= kk * waves64 / 96: 0.75 us per round
 // trip against the time that the rows of all waves take), but the groups move
 // rows faster than the long cells' waves do, so cells that are ordinary for the
-// grid, up to 6 times its mean at kk = 16, stay with them; cells of fewer than
+// grid, up to 6 times its mean (kk / 4 times at kk = 4 and 8: 25.5 M points, C =
+// 28, 268 a cell, 457 us, 485 with 3 times), stay with them; cells of fewer than
 // 64 to 256 points always do.  Depth-weighted forwards of 6 cameras, C = 80, us
 // with 256 for every grid, with this rule and with accum_pipe_kernel: 64 x 176 x
 // 118 points on 360 x 360 cells 302, 270, 309; on 128 x 128 772, 358, 532; on
@@ -3868,7 +3875,9 @@ GroupPlan group_plan(int32_t dtype, int C, int64_t n_points, int64_t n_cells, bo
   g.kk = per <= 4 ? 16 : (per <= 8 ? 8 : 4);
   g.ng = per < 64 / g.kk ? per : 64 / g.kk;
   g.waves64 = ceil_div(ceil_div(n_points, int64_t(64)), int64_t(g.ng));
-  const bool few = g.waves64 < (g.kk == 16 ? kGroupFewWaves : 2 * kGroupFewWaves);
+  const bool sparse = n_points < n_cells + n_cells / 4;
+  const int few_halves = g.kk == 16 ? (sparse ? 3 : 2) : 4;
+  const bool few = g.waves64 < few_halves * (kGroupFewWaves / 2);
   if (depth_rows && g.kk == 4 && g.qmax >= 4 && !few) {
     g.kk = n_points < 8 * n_cells ? 16 : 8;
     g.ng = 64 / g.kk;
@@ -3877,7 +3886,8 @@ GroupPlan group_plan(int32_t dtype, int C, int64_t n_points, int64_t n_cells, bo
   g.small = g.waves64 < kPipeWaves;
   g.P = few ? 16 : 64;
   const int64_t least = few ? 64 : (g.waves64 < kGroupManyWaves ? 128 : 256);
-  const int64_t mean = 3 * g.kk * n_points / (8 * n_cells), chain = g.kk * g.waves64 / 96;
+  const int64_t mean = (g.kk == 16 ? 6 : g.kk / 4) * n_points / n_cells;
+  const int64_t chain = g.kk * g.waves64 / 96;
   const int64_t lcell = mean < chain ? mean : chain;
   g.lcell = int(lcell > least ? lcell : least);
   g.long_parts = int(ceil_div(g.qmax, kLongPieces));

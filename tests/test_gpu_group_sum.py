@@ -123,12 +123,14 @@ def test_wide_rows(pkg, cuda, grid, C, dtype):
     (68, F32, 30000, (7, 9)), (80, F32, 70000, (40, 50)), (80, F32, 130000, (6, 6)),
     (132, F32, 200000, (20, 30)), (256, F32, 60000, (1, 2)), (260, F32, 90000, (30, 40)),
     (39, F32, 30000, (5, 3)), (130, F16, 60000, (6, 8)), (520, BF16, 40000, (9, 5)),
-    (1032, BF16, 20000, (20, 20)), (17, F32, 300000, (30, 30))])
+    (1032, BF16, 20000, (20, 20)), (17, F32, 300000, (30, 30)),
+    (80, F32, 147000, (350, 360)), (80, F32, 148000, (350, 360)), (27, F32, 1600000, (360, 360))])
 def test_points_per_cell(pkg, cuda, C, dtype, N, grid):
     """Grids from a few points a cell to all of them in two cells: the points
     of a long cell from their floor to the chain's limit, rows of one to four
     blocks of long-cell pieces (the last of one piece or more) and of two and
-    three channel blocks."""
+    three channel blocks; sparse grids on both sides of the line to 64 points a
+    group."""
     g = torch.Generator().manual_seed(N + C)
     H, W = grid
     hot = torch.randint(max(1, H * W // 9), (N,), generator=g)
