@@ -3849,8 +3849,8 @@ struct GroupPlan {
 // 28, 268 a cell, 457 us, 485 with 3 times), stay with them; cells of fewer than
 // 64 to 256 points always do.  Depth-weighted forwards of 6 cameras, C = 80, us
 // with 256 for every grid, with this rule and with accum_pipe_kernel: 64 x 176 x
-// 118 points on 360 x 360 cells 302, 270, 309; on 128 x 128 772, 358, 532; on
-// 90 x 90 861, 481, 647; 32 x 88 x 118 on 90 x 90 190, 114, 167.
+// 118 points on 360 x 360 cells 302, 273, 309; on 128 x 128 772, 355, 532; on
+// 90 x 90 861, 487, 647; 32 x 88 x 118 on 90 x 90 190, 117, 167.
 //
 // Blocks of the long cells: about kLongBlocks, so that the candidates are
 // spread over the chip (60 K points in cells of 100: 45 us with 16 candidates
